@@ -133,9 +133,11 @@ int zant_hip_conv2d_out_shape(const int64_t xdim[4], const int64_t wdim[4], cons
  * workspace it grows with hipMalloc) lives in a static device array that every device the library runs on holds
  * until the process ends.  The call performs no hipMalloc / hipFree.  A convolution whose weights (K rounded up to
  * 32 and C to 8, x KH x KW x 4 bytes, + 256) exceed ZANT_HIP_STATIC_SCRATCH_BYTES returns ZANT_ArenaOverflow and
- * launches nothing; zant_hip_last_error() gives both sizes.  Every call on a device shares that device's array: calls on one stream may follow each
- * other freely (each re-packs the weights in stream order), calls that overlap on one
- * device (several contexts or streams) race. */
+ * launches nothing; zant_hip_last_error() gives both sizes.  Layers of fewer than 64 output positions, and layers that no
+ * tile of whole output rows suits (rows or filters too large for it, or half of it empty), need no array: beyond its size
+ * they run on a kernel without scratch.  Every call on a device shares that device's array: calls on one stream may follow
+ * each other freely (each re-packs the weights in stream order), calls that overlap on one device (several contexts or
+ * streams) race. */
 #define ZANT_HIP_STATIC_SCRATCH_BYTES (8u << 20)
 int zant_hip_conv2d_f32_static(zant_ctx *ctx, const float *x, const int64_t xdim[4], const float *w,
                                const int64_t wdim[4], const float *bias, float *y, const int64_t ydim[4],

@@ -116,3 +116,18 @@ def test_static_entry_point_rejects_weights_beyond_the_scratch_array():
     tm.conv_lean(X, W, y2, None, [1, 1], [1, 1, 1, 1], [1, 1], 1, "NOTSET")
     ref = zo.Conv(x, wt, None, [1, 1], [1, 1, 1, 1], [1, 1], 1, "NOTSET")
     np.testing.assert_allclose(host(y2), ref, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("n,c,h,w,k,ks", [
+    (1, 512, 7, 7, 512, 3),    # 49 output positions, 9.4 MB of weights
+    (1, 400, 10, 9, 112, 7),   # 7x7 filters: no two staging buffers of a tile of whole rows fit half of LDS; 8.8 MB
+    (1, 512, 4, 1100, 512, 3),  # rows of 1100 positions: longer than any such tile
+])
+def test_static_entry_point_takes_layers_that_need_no_scratch(n, c, h, w, k, ks):
+    g = np.random.default_rng(c)
+    x = g.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = (g.standard_normal((k, c, ks, ks)) * np.sqrt(2.0 / (ks * ks * c))).astype(np.float32)
+    p = [ks // 2] * 4
+    y = torch.full((n, k, h, w), float("nan"), dtype=torch.float32, device="cuda:0")
+    tm.conv_lean_static(dev(x), dev(wt), y, None, [1, 1], p, [1, 1], 1, "NOTSET")
+    np.testing.assert_allclose(host(y), zo.Conv(x, wt, None, [1, 1], p, [1, 1], 1, "NOTSET"), rtol=RTOL, atol=ATOL)

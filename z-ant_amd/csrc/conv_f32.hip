@@ -10,6 +10,7 @@
 
 #include "common.h"
 #include "conv_split_f32.h"
+#include "conv_tile.h"
 
 namespace {
 
@@ -411,10 +412,11 @@ extern "C" int zant_hip_conv2d_f32(zant_ctx *ctx, const float *x, const int64_t 
 // ---- zant_hip_conv2d_f32_static: the same convolution for callers that cannot allocate ---------------------------
 //
 // The matrix-core kernel's scratch (the packed weights) lives in a static device array instead of the context workspace;
-// three bf16 terms a weight and the kernel's own padding take at most four times the limit that is stated in f32 weights.  `scratch` below is only the host-side handle of that array: every device holds its own
-// copy at its own address, which hipGetSymbolAddress returns and which is what kernels, copies and fills must be
-// given.  The array is shared by every call on a device and keeps the previous call's contents; each call re-packs
-// the weights before its convolution kernel, in stream order, so calls on ONE stream are safe back to back, while calls that overlap on one device (two contexts, two streams) race.
+// three bf16 terms a weight and the kernel's own padding take at most four times the limit that is stated in f32 weights.
+// `scratch` below is only the host-side handle of that array: every device holds its own copy at its own address, which
+// hipGetSymbolAddress returns and which is what kernels, copies and fills must be given.  The array is shared by every call
+// on a device and keeps the previous call's contents; each call re-packs the weights before its convolution kernel, in stream
+// order, so calls on ONE stream are safe back to back, while calls that overlap on one device (two contexts, two streams) race.
 static __device__ __align__(256) unsigned char scratch[4 * ZANT_HIP_STATIC_SCRATCH_BYTES];
 
 namespace {
@@ -459,6 +461,24 @@ extern "C" int zant_hip_conv2d_f32_static(zant_ctx *ctx, const float *x, const i
                                 auto_pad, fuse_act, &slot);
 }
 
+namespace {
+// Layers that zant_hip_conv2d_f32_static takes whatever the size of their weights, on the direct kernel: fewer than 64 output
+// positions, or no tile of whole output rows (32 to 256 positions x 32 or 64 channels, 8 input channels a step, two staging
+// buffers in half of LDS) of which they fill half.  Callers rely on that line; it does not follow what the matrix-core kernel
+// can tile, which is more.
+bool needs_no_scratch(const ConvGeom &g) {
+    if (int64_t(g.N) * g.OH * g.OW < 64 || int64_t(g.N) * g.C * g.H * g.W >= (int64_t(1) << 40)) return true;
+    const size_t cap = 80 * 1024 - (size_t((g.K + 63) / 64) * 64 * sizeof(float) + 8);
+    auto tile = [&](int WM, int WN, TilePlan *p) {
+        return zant_plan_conv_tiles(g, WM, WN, 8, 8, sizeof(float), cap, p, false, 0, 32, 0, 2, 4, 256, 4096);
+    };
+    TilePlan narrow, wide;
+    const bool ok_n = tile(4, 1, &narrow), ok_w = g.K > 32 && tile(2, 2, &wide);
+    if (ok_w && !(ok_n && narrow.eff > wide.eff + 0.25)) return wide.eff < 0.5;
+    return !ok_n || narrow.eff < 0.5;
+}
+}  // namespace
+
 int zant_conv2d_f32_slot(zant_ctx *ctx, const float *x, const int64_t xdim[4], const float *w, const int64_t wdim[4],
                          const float *bias, float *y, const int64_t ydim[4], const int64_t *stride, int n_stride,
                          const int64_t *pads, int n_pads, const int64_t *dil, int n_dil, int64_t group, const char *auto_pad,
@@ -490,7 +510,8 @@ int zant_conv2d_f32_slot(zant_ctx *ctx, const float *x, const int64_t xdim[4], c
     zant_log("OnnxConvLean2");
 
     SplitPlan plan;
-    if (zant_conv_split_plan(g, false, ctx->num_cus, &plan)) {
+    const bool no_room = slot && slot->fixed && zant_conv_split_fixed_bytes(g) > ZANT_HIP_STATIC_SCRATCH_BYTES;
+    if (zant_conv_split_plan(g, false, ctx->num_cus, &plan) && !(no_room && needs_no_scratch(g))) {
         rc = zant_conv_split_run(ctx, x, w, bias, y, g, plan, relu, false, slot, x_c4);
         if (rc == ZANT_OK) zant_log("OnnxConvLean4");
         return rc;

@@ -31,6 +31,9 @@ struct SplitPlan {
 
 // Whether the kernel takes this convolution (with the fused 2x2/2 max pool or without), and the tiling it would run with.
 bool zant_conv_split_plan(const ConvGeom &g, bool pool, int num_cus, SplitPlan *plan);
+// What a layer counts against ZANT_HIP_STATIC_SCRATCH_BYTES.  The limit is stated in f32 weights; the static array itself has
+// room for their three terms and padding.
+size_t zant_conv_split_fixed_bytes(const ConvGeom &g);
 // Packs the weights (unless `slot` holds them) and launches.
 int zant_conv_split_run(zant_ctx *ctx, const float *x, const float *w, const float *bias, float *y, const ConvGeom &g,
                         const SplitPlan &plan, int relu, bool pool, zant_pack_slot *slot, int x_c4);
