@@ -153,3 +153,42 @@ def test_conv_split_pooled_non_finite_values(G, case, relu):
     others = [c for c in range(K) if c != 3]
     np.testing.assert_array_equal(z[:, others], y[:, others])
     assert (z[:, 3] == 0).all() if relu else np.isnan(z[:, 3]).all()
+
+
+# ---- Gemm: sums of few terms --------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("M,N", [(70, 66), (1, 17), (200, 33), (64, 128)])
+@pytest.mark.parametrize("K", [1, 2, 3, 7, 8, 9, 15, 16, 17])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_gemm_of_few_terms(G, M, N, K, ta, tb):
+    """One product is rounded once.  More: never further from 64 bits (2-norm) than the chain of f32 multiply-adds."""
+    g = np.random.default_rng(M + N + K)
+    a, b = g.standard_normal((M, K)).astype(np.float32), g.standard_normal((K, N)).astype(np.float32)
+    a[:, 0] = np.float32(1.0038986)  # 1 + 2^-8 - 2^-17: terms as large as they get, the same sign in every product
+    b[0, ::2] = np.float32(1.0038986)
+    y = G.dev(np.full((1, 1, M, N), np.nan, np.float32))
+    G.tm.gemm_lean(G.dev((a.T if ta else a)[None, None].copy()), G.dev((b.T if tb else b)[None, None].copy()), None, 1.0, 1.0, ta, tb, y)
+    assert G.tm.context().kernel_name().startswith("gemm_f32_split_kernel<1,1,%d," % (0 if K <= 16 else 4))
+    y = G.host(y)[0, 0]
+    if K == 1:
+        np.testing.assert_array_equal(y, a * b)
+        return
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    chain = np.zeros((M, N), np.float32)
+    for k in range(K):  # (a product of two f32 is exact in 64 bits; the sum's rounding there is far below f32's)
+        chain = (chain.astype(np.float64) + a[:, k:k + 1].astype(np.float64) * b[k].astype(np.float64)).astype(np.float32)
+    err, ref = np.linalg.norm(y - exact), np.linalg.norm(chain - exact)
+    assert err <= 1.02 * ref, (err / ref)
+
+
+def test_gemm_of_few_terms_non_finite_and_unaligned(G):
+    import torch
+    g = np.random.default_rng(5)
+    a, b = g.standard_normal((1, 1, 37, 16), dtype=np.float32), np.abs(g.standard_normal((1, 1, 16, 70), dtype=np.float32))
+    a[0, 0, 3, 2], a[0, 0, 20, 15], a[0, 0, 36, 0] = np.inf, np.nan, np.float32(3e38)
+    flat = torch.zeros(a.size + 4, device="cuda:0")
+    A = flat[1:1 + a.size].view(a.shape)
+    A.copy_(torch.from_numpy(a))
+    y = G.dev(np.full((1, 1, 37, 70), 7.0, np.float32))
+    G.tm.gemm_lean(A, G.dev(b), None, 1.0, 1.0, False, False, y)
+    with np.errstate(all="ignore"):
+        np.testing.assert_allclose(G.host(y), zo.gemm(a, b, None, 1.0, 1.0, False, False), rtol=G.RTOL, atol=G.ATOL)
