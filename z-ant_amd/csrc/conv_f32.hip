@@ -511,7 +511,7 @@ int zant_conv2d_f32_slot(zant_ctx *ctx, const float *x, const int64_t xdim[4], c
 
     SplitPlan plan;
     const bool no_room = slot && slot->fixed && zant_conv_split_fixed_bytes(g) > ZANT_HIP_STATIC_SCRATCH_BYTES;
-    if (zant_conv_split_plan(g, false, ctx->num_cus, &plan) && !(no_room && needs_no_scratch(g))) {
+    if (zant_conv_split_plan(g, false, ctx->num_cus, &plan, slot) && !(no_room && needs_no_scratch(g))) {
         rc = zant_conv_split_run(ctx, x, w, bias, y, g, plan, relu, false, slot, x_c4);
         if (rc == ZANT_OK) zant_log("OnnxConvLean4");
         return rc;
@@ -565,7 +565,7 @@ int zant_conv2d_f32_fused_pool(zant_ctx *ctx, const float *x, const int64_t xdim
     if (!k133 && !k155 && !k333) {
         // many-channel layers: the implicit-GEMM kernel with the pool folded into its epilogue
         SplitPlan plan;
-        if (!zant_conv_split_plan(g, true, ctx ? ctx->num_cus : 256, &plan)) return 1;
+        if (!zant_conv_split_plan(g, true, ctx ? ctx->num_cus : 256, &plan, slot)) return 1;
         if (query_only) return ZANT_OK;
         if (y_c4) return ZANT_InvalidInput;  // (zant_conv2d_f32_c4_caps says which kernel writes that layout)
         return zant_conv_split_run(ctx, x, w, bias, y, g, plan, relu, true, slot, x_c4);

@@ -29,8 +29,9 @@ struct SplitPlan {
     size_t wp_bytes;        // packed weights
 };
 
-// Whether the kernel takes this convolution (with the fused 2x2/2 max pool or without), and the tiling it would run with.
-bool zant_conv_split_plan(const ConvGeom &g, bool pool, int num_cus, SplitPlan *plan);
+// Whether the kernel takes this convolution (with the fused 2x2/2 max pool or without), and the tiling it would run with.  `slot`
+// keeps the tiling for the next call with the same geometry.
+bool zant_conv_split_plan(const ConvGeom &g, bool pool, int num_cus, SplitPlan *plan, zant_pack_slot *slot = nullptr);
 // What a layer counts against ZANT_HIP_STATIC_SCRATCH_BYTES.  The limit is stated in f32 weights; the static array itself has
 // room for their three terms and padding.
 size_t zant_conv_split_fixed_bytes(const ConvGeom &g);
