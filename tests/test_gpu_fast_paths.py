@@ -169,3 +169,21 @@ def test_dense_int8_layers_of_few_positions(G, case, act):
     y = G.tm.qlinearconv(G.dev(x), 0.02, 117, G.dev(w), G.dev(ws), None, 0.05, 120, G.dev(b), [s, s], [p] * 4, [1, 1], 1, **kw)
     assert G.tm.context().kernel_name().startswith("qconv_mfma_kernel<"), G.tm.context().kernel_name()
     np.testing.assert_array_equal(G.host(y), ref)
+
+
+@pytest.mark.parametrize("N,C,H,W,K,k,mfma", [
+    (2, 13, 5, 5, 215, 1, False), (4, 9, 2, 3, 81, 1, False), (1, 39, 3, 7, 20, 1, False), (1, 7, 5, 4, 6, 2, False),  # up to 39 terms
+    (1, 40, 3, 7, 20, 1, True), (1, 6, 5, 5, 20, 3, True),  # 40 and 54
+    (1, 13, 8, 8, 20, 1, True),  # 64 positions
+])
+def test_int8_layers_of_few_positions_and_few_terms(G, N, C, H, W, K, k, mfma):
+    """Less than a tile and less than 40 terms a sum: the direct kernel, whose whole call is the shorter one."""
+    g = np.random.default_rng(C + K)
+    x = g.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+    w = g.integers(-127, 128, (K, C, k, k), dtype=np.int8)
+    ws = (g.uniform(0.5, 1.5, K) * 0.08 / np.sqrt(C * k * k)).astype(np.float32)
+    b = g.integers(-500, 501, K, dtype=np.int32)
+    ref = zo.qlinearconv(x, 0.02, 117, w, ws, None, 0.05, 120, b, [1, 1], [0] * 4, [1, 1], 1)
+    y = G.tm.qlinearconv(G.dev(x), 0.02, 117, G.dev(w), G.dev(ws), None, 0.05, 120, G.dev(b), [1, 1], [0] * 4, [1, 1], 1)
+    assert G.tm.context().kernel_name().startswith("qconv_mfma_kernel<") == mfma, G.tm.context().kernel_name()
+    np.testing.assert_array_equal(G.host(y), ref)

@@ -697,6 +697,11 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
                    const ConvGeom &g0, const QConvArgs &q, bool x_blocked, bool y_blocked, zant_pack_slot *slot, bool pool = false,
                    bool plan_only = false) {
     if (g0.groups != 1 || g0.C < 5) return 1;
+    // Fewer than 64 positions are no whole tile, and sums of few terms are over before this kernel has packed its weights and copied
+    // its input: there the direct kernel's whole call is the shorter one.  Measured at 2 to 60 positions and 10 to 441 filters: 5 to
+    // 35 terms 4.8 - 7.9 us against 7.4 - 9.5, 43 to 46 terms 6.6 - 9.5 against 8.3 - 10.0, 62 to 105 terms 7.9 - 16.0 against
+    // 7.0 - 10.9, 3681 terms 216 against 13.
+    if (int64_t(g0.N) * g0.OH * g0.OW < 64 && int64_t(g0.C) * g0.KH * g0.KW < 40) return 1;
     // What the planning below decides depends on the geometry only: a node or plan that calls again with the same one
     // reuses it (the searches for a tile shape cost the host as much time as a small layer takes on the GPU).
     struct PlanKey { ConvGeom g; int x_blocked, y_blocked, pool, cus, act_ok, kind; } pkey;
@@ -753,7 +758,7 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
             plan = wide; WN = 2; have = true;
         }
     }
-    if (!have) return 1;  // (however few of a tile's position slots a small layer fills: the direct kernel is a hundred times slower)
+    if (!have) return 1;
     const int T = g.KH * g.KW, K_BLK = WN * 32;
     plan.t.n_chunks = (g.C + QCC - 1) / QCC;
     // Ring of staging buffers: as many stages as fit beside the tables in the LDS share of a workgroup -- half a CU's
