@@ -172,12 +172,12 @@ def test_dense_int8_layers_of_few_positions(G, case, act):
 
 
 @pytest.mark.parametrize("N,C,H,W,K,k,mfma", [
-    (2, 13, 5, 5, 215, 1, False), (4, 9, 2, 3, 81, 1, False), (1, 39, 3, 7, 20, 1, False), (1, 7, 5, 4, 6, 2, False),  # up to 39 terms
-    (1, 40, 3, 7, 20, 1, True), (1, 6, 5, 5, 20, 3, True),  # 40 and 54
+    (2, 13, 5, 5, 215, 1, False), (4, 9, 2, 3, 81, 1, False), (1, 39, 3, 7, 20, 1, False), (2, 5, 6, 9, 28, 3, False), (1, 6, 5, 5, 20, 3, False),  # up to 39 and 54 terms
+    (1, 40, 3, 7, 20, 1, True), (1, 7, 5, 5, 20, 3, True),  # 40 and 63
     (1, 13, 8, 8, 20, 1, True),  # 64 positions
 ])
 def test_int8_layers_of_few_positions_and_few_terms(G, N, C, H, W, K, k, mfma):
-    """Less than a tile and less than 40 terms a sum: the direct kernel, whose whole call is the shorter one."""
+    """Less than a tile and few terms a sum (below 40, of 3x3 filters below 56): the direct kernel, whose whole call is the shorter one."""
     g = np.random.default_rng(C + K)
     x = g.integers(0, 256, (N, C, H, W), dtype=np.uint8)
     w = g.integers(-127, 128, (K, C, k, k), dtype=np.int8)

@@ -698,10 +698,12 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
                    bool plan_only = false) {
     if (g0.groups != 1 || g0.C < 5) return 1;
     // Fewer than 64 positions are no whole tile, and sums of few terms are over before this kernel has packed its weights and copied
-    // its input: there the direct kernel's whole call is the shorter one.  Measured at 2 to 60 positions and 10 to 441 filters: 5 to
-    // 35 terms 4.8 - 7.9 us against 7.4 - 9.5, 43 to 46 terms 6.6 - 9.5 against 8.3 - 10.0, 62 to 105 terms 7.9 - 16.0 against
-    // 7.0 - 10.9, 3681 terms 216 against 13.
-    if (int64_t(g0.N) * g0.OH * g0.OW < 64 && int64_t(g0.C) * g0.KH * g0.KW < 40) return 1;
+    // its input: there the direct kernel's whole call is the shorter one.  Measured at 1 to 60 positions and 10 to 441 filters, all
+    // kernels of a call: 1x1 filters of 5 to 36 terms 3.5 - 12.5 us against 9.6 - 15.0, of 40 to 46 terms 11.5 - 14.7 against 10.9 -
+    // 15.4, of 62 to 105 terms 16 - 30 against 9.5 - 18; 3x3 filters of 45 and 54 terms 8.4 - 9.9 against 10.0 - 11.7, of 63 terms
+    // 10.8 - 11.4 against 12.0, of 81 to 99 terms 13.5 - 17.0 against 9.2 - 14.4.
+    const int64_t few_terms = g0.KH * g0.KW == 1 ? 40 : 56;
+    if (int64_t(g0.N) * g0.OH * g0.OW < 64 && int64_t(g0.C) * g0.KH * g0.KW < few_terms) return 1;
     // What the planning below decides depends on the geometry only: a node or plan that calls again with the same one
     // reuses it (the searches for a tile shape cost the host as much time as a small layer takes on the GPU).
     struct PlanKey { ConvGeom g; int x_blocked, y_blocked, pool, cus, act_ok, kind; } pkey;
