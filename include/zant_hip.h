@@ -153,8 +153,8 @@ int zant_hip_conv2d_f32_static(zant_ctx *ctx, const float *x, const int64_t xdim
  * fuse_pool != 0: the plan is Conv (-> ReLU with fuse_act) -> onnx_maxpool_lean with a 2 x 2 kernel, stride 2, no padding,
  * floor mode (op_pooling.zig:570-659) in ONE kernel -- what a code generator that peephole-fuses the chain emits
  * (hardcoded_mnist8.zig:186-268 is such a chain); ydim is then the pooled shape.  Taken for stride 1, dilation 1 and
- * the shapes whose convolution kernel has the pooled epilogue (8 or more input channels, or a 1- / 3-channel 3x3 or a
- * 1-channel 5x5 first layer); other shapes return ZANT_InvalidInput and the caller issues the two operators. */
+ * the shapes whose convolution kernel has the pooled epilogue (4 or more input channels and 32 or more terms a sum, or a 1- /
+ * 3-channel 3x3 or a 1-channel 5x5 first layer); other shapes return ZANT_InvalidInput and the caller issues the two operators. */
 typedef struct zant_conv_plan zant_conv_plan;
 int zant_hip_conv2d_f32_prepack(zant_ctx *ctx, const int64_t xdim[4], const float *w, const int64_t wdim[4],
                                 const float *bias, const int64_t ydim[4], const int64_t *stride, int n_stride,

@@ -192,3 +192,39 @@ def test_gemm_of_few_terms_non_finite_and_unaligned(G):
     G.tm.gemm_lean(A, G.dev(b), None, 1.0, 1.0, False, False, y)
     with np.errstate(all="ignore"):
         np.testing.assert_allclose(G.host(y), zo.gemm(a, b, None, 1.0, 1.0, False, False), rtol=G.RTOL, atol=G.ATOL)
+
+
+# ---- operands whose left-out term products are as large as they get ------------------------------------------------------------
+def test_split_error_bound_of_equal_operands(G):
+    """1.0038986 splits into 1 + 2^-8 - 2^-17: 2^-24 of every product is left out, always with the same sign.  The result may be
+    that far off, plus f32 roundings of n products of one sign: one per 16, each at most half a unit of the sum so far."""
+    v = np.float32(1.0038986)
+    for C, k in [(20, 3), (12, 3), (64, 1)]:
+        n = C * k * k
+        x, w = np.full((2, C, 9, 9), v, np.float32), np.full((33, C, k, k), v, np.float32)
+        y = G.host(G.tm.Conv(G.dev(x), G.dev(w), None, [1, 1], [0, 0, 0, 0], [1, 1], 1, "NOTSET"))
+        assert G.tm.context().kernel_name().startswith("conv_f32_split_kernel<")
+        exact = n * np.float64(v) ** 2
+        assert np.abs(y - exact).max() <= exact * 2.0 ** -24 * (1.05 + 6 * -(-n // 16) / 2)
+    a, b = np.full((1, 1, 70, 1600), v, np.float32), np.full((1, 1, 1600, 66), v, np.float32)
+    y = G.dev(np.zeros((1, 1, 70, 66), np.float32))
+    G.tm.gemm_lean(G.dev(a), G.dev(b), None, 1.0, 1.0, False, False, y)
+    exact = 1600 * np.float64(v) ** 2
+    assert np.abs(G.host(y) - exact).max() <= exact * 2.0 ** -24 * (1.05 + 6 * 100 / 2)
+
+
+# ---- rows of 2^22 elements and more: the kernel with 64-bit addresses, in every storage order -----------------------------------
+@pytest.mark.parametrize("M,K,N,ta,tb", [(3, 5, (1 << 22) + 3, False, False), ((1 << 22) + 5, 3, 17, True, False),
+                                         ((1 << 22) + 1, 3, 18, True, True), (5, (1 << 22) + 2, 19, False, True)])
+def test_gemm_long_rows_in_every_storage_order(G, M, K, N, ta, tb):
+    import torch
+    t = torch.Generator(device="cuda:0").manual_seed(M + N)
+    a = torch.randn((K, M) if ta else (M, K), generator=t, device="cuda:0")
+    b = torch.randn((N, K) if tb else (K, N), generator=t, device="cuda:0")
+    y = torch.full((1, 1, M, N), float("nan"), device="cuda:0")
+    G.tm.gemm_lean(a[None, None], b[None, None], None, 1.0, 1.0, ta, tb, y)
+    flags = "%s,%s>" % ("false" if ta else "true", "true" if tb else "false")
+    assert G.tm.context().kernel_name().startswith("gemm_f32_mfma_kernel<") and G.tm.context().kernel_name().endswith(flags)
+    ref = (a.T if ta else a).double().cpu().numpy() @ (b.T if tb else b).double().cpu().numpy()
+    rms = np.sqrt(np.mean(ref ** 2))
+    assert np.sqrt(np.mean((G.host(y)[0, 0] - ref) ** 2)) < np.sqrt(K) * 2.0 ** -24 * rms

@@ -2,6 +2,19 @@
 #pragma once
 #include "common.h"
 
+// max without the NaN-quieting pass the compiler puts in front of fmaxf (an MFMA result is never a signalling NaN); a NaN
+// operand yields the other one, like fmaxf
+__device__ __forceinline__ float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 // A convolution seen as one flat sequence of output slots (output positions, or 2x2 pooling windows with a fused pool) over
 // "strips": a strip is a run of whole output columns of one image (the whole image unless it is too wide for LDS).  The
 // input rows of a strip with their padding follow one another strip after strip, so the rows a run of slots needs are one

@@ -1,4 +1,4 @@
-// Tiling of the implicit-GEMM int8 convolution kernel.
+// Tiling of the implicit-GEMM int8 convolution kernel (and what zant_hip_conv2d_f32_static takes without scratch, conv_f32.hip).
 //
 // A tile is NB whole images x TH whole output rows x all OW columns, for one block of output
 // channels.  Per chunk of input channels a tile stages a patch of P1 = NB*PH*PW input positions.
