@@ -218,6 +218,25 @@ def test_resize_ragged_rows_match_oracle(G, shape, sizes, dtype, coord):
     np.testing.assert_array_equal(y, zo.resize(x, "nearest", None, sizes, coord))
 
 
+@pytest.mark.parametrize("shape,sizes,dtype,planes", [
+    ((3, 20, 60, 76), [3, 20, 15, 149], np.uint8, False),   # few workgroups, long input runs
+    ((3, 20, 60, 200), [3, 20, 24, 401], np.float32, False),
+    ((3, 20, 60, 76), [3, 20, 30, 149], np.float32, True),  # 18 rounds of copying
+    ((3, 1, 23, 157), [3, 1, 46, 314], np.uint8, True),
+    ((90, 80, 40, 25), [90, 80, 20, 49], np.uint8, False),  # one input an output, too few workgroups
+    ((150, 80, 40, 25), [150, 80, 20, 49], np.uint8, True),  # enough
+    ((100, 80, 60, 19), [100, 80, 12, 37], np.float32, False),  # 2.6 inputs an output
+])
+def test_resize_takes_the_planes_kernel_where_it_is_the_faster(G, shape, sizes, dtype, planes):
+    if dtype == np.uint8 and shape[0] in (90, 150):
+        cus = torch.cuda.get_device_properties(0).multi_processor_count
+        assert (-(-int(np.prod(sizes)) // (256 * 4 * 16)) >= 2 * cus) == planes
+    x = (np.random.default_rng(13).standard_normal(shape) * 90).astype(dtype)
+    y = G.tm.resize(dev(x), "nearest", None, sizes, "asymmetric").cpu().numpy()
+    assert G.tm.context().kernel_name().startswith("resize_planes_kernel<") == planes, G.tm.context().kernel_name()
+    np.testing.assert_array_equal(y, zo.resize(x, "nearest", None, sizes, "asymmetric"))
+
+
 @pytest.mark.parametrize("shape", [(512, 128, 6, 6), (256, 64, 28, 32)])
 def test_resize_at_full_size_repeats_elements(G, shape):
     x = torch.randint(0, 255, shape, dtype=torch.uint8, device="cuda")

@@ -381,6 +381,12 @@ bool launch_resize_planes(zant_ctx *ctx, const void *x, void *y, const ResizeGeo
     const int64_t span_bytes = (span * int64_t(sizeof(U)) + 15) & ~int64_t(15);
     const int64_t lds_bytes = span_bytes + (rows + OW) * int64_t(sizeof(int));
     if (lds_bytes > kLds) return false;
+    // Every input row of the run is copied, needed or not, an element a thread at a time.  Down to 22 rounds of that a workgroup's
+    // latency is no longer than the table launch it saves (60x200 -> 30x401 f32, 60 planes, 8.4 against 8.3 us of kernels; u8 12 to 29
+    // against 6 to 8 from 40 rounds on); longer runs need two workgroups per CU to hide it (u8 800 planes of 60x200 -> 30x401, 587
+    // workgroups, 27 against 36 us; -> 24x401, 470 workgroups, 34 against 30) and at most 1.6 inputs an output (f32 8000 planes of
+    // 60x76 -> 20x149 85 against 100 us, -> 15x149 93 against 78).
+    if (span > 22 * kThreads && (ceil_div64(g.total, CHUNK) < 2 * ctx->num_cus || 5 * H * W > 8 * OH * OW)) return false;
     ResizePlanes p;
     p.H = int(H); p.W = int(W); p.OH = int(OH); p.OW = int(OW);
     p.total = unsigned(g.total);
