@@ -1008,7 +1008,7 @@ int zant_qconv_ps(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float 
     const bool x_direct = !x_blocked && !y_blocked && g.C % 16 == 0 && g.W % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 4 == 0 &&
                           int64_t(g.N) * g.C * g.H * g.W < (int64_t(1) << 31);
     const size_t xb_bytes = x_blocked || x_direct ? 0 : size_t(g.N) * p.CB * g.H * g.W * 16;
-    // [tile counters (unused) | padding vector | multipliers, corrections (one contiguous table) | packed weights]
+    // [unused | padding vector | multipliers, corrections (one contiguous table) | packed weights]
     const size_t o_pad = 256, o_mult = 512, o_corr = o_mult + size_t(p.kpad) * 4,
                  o_wp = o_mult + ps_align256(size_t(p.kpad) * 8), static_bytes = o_wp + ps_align256(wp_bytes);
     void *ws = nullptr, *dyn = nullptr;
