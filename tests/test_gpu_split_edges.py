@@ -228,3 +228,18 @@ def test_gemm_long_rows_in_every_storage_order(G, M, K, N, ta, tb):
     ref = (a.T if ta else a).double().cpu().numpy() @ (b.T if tb else b).double().cpu().numpy()
     rms = np.sqrt(np.mean(ref ** 2))
     assert np.sqrt(np.mean((G.host(y)[0, 0] - ref) ** 2)) < np.sqrt(K) * 2.0 ** -24 * rms
+
+
+@pytest.mark.parametrize("M,K,N,tile", [(4001, 1601, 509, "<2,1,"), (6001, 997, 515, "<2,2,")])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_gemm_large_tiles_non_finite_values(G, M, K, N, tile, ta, tb):
+    """Blocks computed again at ragged edges of the larger tiles: the values 64 bits give, non-finite ones among them."""
+    g = np.random.default_rng(M)
+    a, b = g.standard_normal((M, K), dtype=np.float32), (np.abs(g.standard_normal((K, N))) * 0.01).astype(np.float32)
+    a[M - 1, 3], a[17, 5], a[M - 2, 0], b[7, N - 1] = np.inf, np.nan, np.float32(3e38), -np.inf
+    y = G.dev(np.full((1, 1, M, N), 7.0, np.float32))
+    G.tm.gemm_lean(G.dev((a.T if ta else a)[None, None].copy()), G.dev((b.T if tb else b)[None, None].copy()), None, 1.0, 1.0, ta, tb, y)
+    assert tile in G.tm.context().kernel_name()
+    with np.errstate(all="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+    np.testing.assert_allclose(G.host(y)[0, 0], ref, rtol=G.RTOL, atol=G.ATOL)
