@@ -2,9 +2,8 @@
 // of layers with few input channels.
 //
 // The reference materialises a zero-padded copy, an im2col matrix, a transposed weight matrix and a matmul result.  Here a
-// convolution is one implicit-GEMM kernel (conv_split_f32.hip) from four input channels and 32 terms a sum on; layers below
-// that are bound by writing their output and have kernels of their own, one of them on the f32 matrix cores with the channel's
-// nine taps as the reduction axis.  A direct kernel (one thread per output element) covers what is left.
+// convolution is one implicit-GEMM kernel (conv_split_f32.hip); layers of short sums are bound by writing their output and run on
+// conv_short_f32.hip, with a fused pool on the kernels here.  A direct kernel (one thread per output element) covers what is left.
 #include <algorithm>
 #include <mutex>
 
@@ -45,44 +44,6 @@ __global__ void __launch_bounds__(256) conv_f32_direct_kernel(const float *__res
         float r = acc + (bias ? bias[k] : 0.0f);
         if (relu) r = r > 0.0f ? r : 0.0f;
         y[i] = r;
-    }
-}
-
-// Few-input-channel convolution (C*KH*KW = CKK small: first layers with 1 or 3 channels).  The
-// implicit-GEMM K is then far below one MFMA tile and the layer is bound by writing its output, so
-// each thread keeps the CKK input taps of one output position in registers and streams all K output
-// channels (weights are wave-uniform: scalar loads); a wave writes 256 contiguous bytes per channel.
-template <int CKK>
-__global__ void __launch_bounds__(256) conv_f32_smallc_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                             const float *__restrict__ bias, float *__restrict__ y,
-                                                             ConvGeom g, int relu) {
-    const int64_t plane = int64_t(g.OH) * g.OW;
-    const int64_t total = int64_t(g.N) * plane;
-    const int64_t step = int64_t(gridDim.x) * blockDim.x;
-    const int taps = g.KH * g.KW;
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += step) {
-        const int n = int(i / plane);
-        const int pos = int(i - int64_t(n) * plane);
-        const int oh = pos / g.OW, ow = pos - oh * g.OW;
-        float xin[CKK];
-#pragma unroll
-        for (int e = 0; e < CKK; ++e) {
-            const int c = e / taps, t = e - c * taps;
-            const int kh = t / g.KW, kw = t - kh * g.KW;
-            const int ih = oh * g.sh - g.pt + kh * g.dh, iw = ow * g.sw - g.pl + kw * g.dw;
-            const bool ok = ih >= 0 && ih < g.H && iw >= 0 && iw < g.W;
-            xin[e] = ok ? x[((int64_t(n) * g.C + c) * g.H + ih) * g.W + iw] : 0.0f;
-        }
-        float *yp = y + int64_t(n) * g.K * plane + pos;
-        for (int k = 0; k < g.K; ++k) {
-            const float *wk = w + int64_t(k) * CKK;
-            float acc = 0.0f;
-#pragma unroll
-            for (int e = 0; e < CKK; ++e) acc = __builtin_fmaf(xin[e], wk[e], acc);
-            float r = acc + (bias ? bias[k] : 0.0f);
-            if (relu) r = r > 0.0f ? r : 0.0f;
-            yp[int64_t(k) * plane] = r;
-        }
     }
 }
 
@@ -498,26 +459,22 @@ int zant_conv2d_f32_slot(zant_ctx *ctx, const float *x, const int64_t xdim[4], c
 
     SplitPlan plan;
     const bool no_room = slot && slot->fixed && zant_conv_split_fixed_bytes(g) > ZANT_HIP_STATIC_SCRATCH_BYTES;
-    if (zant_conv_split_plan(g, false, ctx->num_cus, &plan, slot) && !(no_room && needs_no_scratch(g))) {
+    const bool short_ok = !x_c4 && zant_conv_short_ok(g);
+    const bool split_first = x_c4 || no_room || !short_ok || !zant_conv_short_better(g, slot && !slot->fixed);
+    if (split_first && zant_conv_split_plan(g, false, ctx->num_cus, &plan, slot) && !(no_room && needs_no_scratch(g))) {
         rc = zant_conv_split_run(ctx, x, w, bias, y, g, plan, relu, false, slot, x_c4);
         if (rc == ZANT_OK) zant_log("OnnxConvLean4");
         return rc;
     }
     if (x_c4) return ZANT_InvalidInput;  // only the matrix-core kernel reads the quad-blocked layout (see zant_conv2d_f32_c4_caps)
-    const int ckk = g.C * g.KH * g.KW;
-    if (ckk == 9 || ckk == 25 || ckk == 27) {
-        const int64_t positions = int64_t(g.N) * g.OH * g.OW;
-        const unsigned pb = unsigned(std::min<int64_t>(ceil_div64(positions, 256), int64_t(ctx->num_cus) * 16));
-        KernelTimer kt(ctx);
-        ZANT_KERNEL_NAME(ctx, "conv_f32_smallc_kernel<%d>", ckk);
-        if (ckk == 9) hipLaunchKernelGGL(conv_f32_smallc_kernel<9>, dim3(pb), dim3(256), 0, ctx->stream, x, w, bias, y, g, relu);
-        else if (ckk == 25) hipLaunchKernelGGL(conv_f32_smallc_kernel<25>, dim3(pb), dim3(256), 0, ctx->stream, x, w, bias, y, g, relu);
-        else hipLaunchKernelGGL(conv_f32_smallc_kernel<27>, dim3(pb), dim3(256), 0, ctx->stream, x, w, bias, y, g, relu);
-        ZANT_LAUNCH_CHECK(ctx);
-        zant_log("OnnxConvLean4");
-        return ZANT_OK;
-    }
     const int64_t total = int64_t(g.N) * g.K * g.OH * g.OW;
+    // (sums of one or two terms for few outputs: a thread an output is done before the other kernel has its weights in LDS,
+    // 7514 positions, 36 filters 4.5 against 4.8 us, 24192 positions, 19 filters 5.2 against 4.6)
+    if (short_ok && (int64_t(g.C) * g.KH * g.KW > 2 || total > 400 * 1000)) {
+        rc = zant_conv_short_run(ctx, x, w, bias, y, g, relu);
+        if (rc == ZANT_OK) zant_log("OnnxConvLean4");
+        return rc;
+    }
     int64_t blocks = ceil_div64(total, 256);
     if (blocks > int64_t(ctx->num_cus) * 32) blocks = int64_t(ctx->num_cus) * 32;
     KernelTimer kt(ctx);

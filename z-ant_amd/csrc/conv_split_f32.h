@@ -51,3 +51,9 @@ size_t zant_conv_split_fixed_bytes(const ConvGeom &g);
 // Packs the weights (unless `slot` holds them) and launches.
 int zant_conv_split_run(zant_ctx *ctx, const float *x, const float *w, const float *bias, float *y, const ConvGeom &g,
                         const SplitPlan &plan, int relu, bool pool, zant_pack_slot *slot, int x_c4);
+
+// Convolutions of short sums (conv_short_f32.hip): whether the kernel can take this one, whether it is then the better one of the two
+// (packed_once: the split kernel's weights are packed once for many calls), and its launch (no scratch).
+bool zant_conv_short_ok(const ConvGeom &g);
+bool zant_conv_short_better(const ConvGeom &g, bool packed_once);
+int zant_conv_short_run(zant_ctx *ctx, const float *x, const float *w, const float *bias, float *y, const ConvGeom &g, int relu);
