@@ -21,6 +21,9 @@ struct zant_ctx {
     // scratch for per-call packed weights / multiplier tables (grown on demand, never shrunk)
     void *workspace = nullptr;
     size_t workspace_bytes = 0;
+    // f32 Gemms whose K is cut among workgroups (gemm_split_f32.hip): partial sums, then a counter per block of them, zero between
+    // launches.  Allocated with the context, so that no call has to; null where that failed, and then no K is cut.
+    void *gemm_parts = nullptr;
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     hipEvent_t ev_k0 = nullptr, ev_k1 = nullptr;  // bracket the last main kernel when kernel_timing is on
     bool kernel_timing = false;
@@ -66,6 +69,10 @@ struct KernelTimer {
         if (ctx->kernel_timing) (void)hipEventRecord(ctx->ev_k1, ctx->stream);
     }
 };
+
+// What zant_ctx::gemm_parts holds.
+constexpr int ZANT_GEMM_PART_BLOCKS = 2048;  // partial 32 x 32 blocks
+constexpr size_t ZANT_GEMM_PART_BYTES = size_t(ZANT_GEMM_PART_BLOCKS) * (4096 + 4);
 
 // Grows the context's workspace to at least `bytes` (stream-ordered use only).
 int zant_workspace(zant_ctx *ctx, size_t bytes, void **out);

@@ -106,6 +106,23 @@ int zant_pack_region(zant_ctx *ctx, zant_pack_slot *slot, size_t static_bytes, s
     return ZANT_OK;
 }
 
+// The scratch of Gemms with a cut K, its counters zero.  On a stream of its own and with relaxed capture rules: somebody may be
+// capturing a graph on another stream.  Null on failure (the Gemms then run whole).
+static void *alloc_gemm_parts() {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+    void *p = nullptr;
+    hipStream_t s = nullptr;
+    bool ok = hipMalloc(&p, ZANT_GEMM_PART_BYTES) == hipSuccess && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess;
+    ok = ok && hipMemsetAsync(static_cast<char *>(p) + size_t(ZANT_GEMM_PART_BLOCKS) * 4096, 0, size_t(ZANT_GEMM_PART_BLOCKS) * 4, s) == hipSuccess;
+    ok = s && hipStreamSynchronize(s) == hipSuccess && ok;
+    if (s) (void)hipStreamDestroy(s);
+    if (!ok && p) { (void)hipFree(p); p = nullptr; }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ok) (void)hipGetLastError();
+    return p;
+}
+
 extern "C" int zant_hip_ctx_create(zant_ctx **out, int device, void *stream) {
     if (!out) return ZANT_NullPointer;
     *out = nullptr;
@@ -132,6 +149,7 @@ extern "C" int zant_hip_ctx_create(zant_ctx **out, int device, void *stream) {
             return create_failed(e, "hipEventCreate");
         }
     }
+    ctx->gemm_parts = alloc_gemm_parts();
     *out = ctx;
     return ZANT_OK;
 }
@@ -142,6 +160,7 @@ extern "C" void zant_hip_ctx_destroy(zant_ctx *ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->arena) (void)hipFree(ctx->arena);
     if (ctx->workspace) (void)hipFree(ctx->workspace);
+    if (ctx->gemm_parts) (void)hipFree(ctx->gemm_parts);
     if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
     if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
     if (ctx->ev_k0) (void)hipEventDestroy(ctx->ev_k0);
