@@ -33,7 +33,7 @@ HOST_TEST = os.path.join(HERE, "host", "test_host_mirror")
 
 
 # sources whose kernels hide LDS reads from the compiler (checked for spills at build time, see build())
-NO_SPILL_SOURCES = {"qconv_ps_i8.hip", "qblock_i8.hip", "qconv_i8.hip", "conv_f32.hip", "gemm_f32.hip"}
+NO_SPILL_SOURCES = {"qconv_ps_i8.hip", "qblock_i8.hip", "qblock_image_i8.hip", "qconv_i8.hip", "conv_f32.hip", "gemm_f32.hip"}
 
 # kernels whose hand-written stores take their bases from scalar registers: a scalar spill reloaded (v_readlane) right
 # in front of such a store would need wait states the compiler cannot count through inline asm

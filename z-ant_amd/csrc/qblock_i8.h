@@ -1,0 +1,43 @@
+// What the inverted residual block kernels share: a block's kernel arguments and their preparation (qblock_i8.hip).
+#pragma once
+#include "quant_common.h"
+#include "quant_layout.h"
+
+struct QBlockArgs {
+    int N, H, W, OH, OW, stride;
+    int CBin, Cin32, Ce32, CBo;        // input channel blocks (16) / chunks (32); expanded chunks; output blocks
+    int Co;                            // output channels (the rest of the last block is padding)
+    int NB, TH, PH, PW, P, Ppad, Q;    // tile: images, output rows, patch rows / columns / positions, output positions
+    int n_row_tiles, n_tiles;
+    int o_xl, o_e, o_w1, o_w2, o_wdw, o_tab, o_ptab;  // LDS byte offsets
+    int packed_units;                  // 16-byte units of weights and tables: the LDS bytes from o_w1 to o_ptab
+    int split;                         // stage D deals (position tile, channel chunk) units to the waves (few position tiles)
+    float zp1f, zp2f, zp3f;            // zero points of the three convolutions' own outputs
+    QAct act1, act2;
+    int has_act1, has_act2;
+    uint32_t pad_e4;                   // the depthwise input zero point ^ 0x80 in every byte
+    int half_last;                     // the last chunk of expanded channels holds at most 16 real ones
+    int has_res, fast_div;             // fast_div: the scales allow the unscaled division sequence
+    float ry_rcp;                      // refined reciprocal of ry_scale
+    float ra_scale, rb_scale, ry_scale;  // residual add: a = projection output, b = block input, y = sum
+    int ra_zp, rb_zp, ry_zp;
+};
+
+// What a launch needs of one block: its kernel arguments, LDS bytes, instantiation and packed weights.
+struct QBlockPrep {
+    QBlockArgs a;
+    size_t lds_bytes;
+    int CO32, MQv;
+    const uint4 *packed;  // weights, requantisation tables, then (see o_lut) what qblock_image_i8.hip wants beside them
+    int o_lut;            // bytes from `packed` to the two activation tables and the table of a whole image's patch positions
+};
+
+// Plans a block's tile, (re)packs its weights and tables into `slot` (or the context workspace) and fills the kernel
+// arguments.  force_nb > 0: tiles of exactly that many whole images, or 1.  plan_only: no packing, no pointers needed.
+int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *expand, const zant_qconv_desc *dw, int64_t dw_stride,
+                        const zant_qconv_desc *project, int residual, float add_scale, int add_zp, const int64_t ydim[4], bool plan_only,
+                        zant_pack_slot *slot, int force_nb, QBlockPrep *out);
+
+// zant_qblock_chain on one image a workgroup, activations in LDS from block to block (qblock_image_i8.hip); 1 when the blocks do not
+// fit that or tiles of several images are the better choice.
+int zant_qblock_image_chain(zant_ctx *ctx, int n, const zant_qblock_call *calls, bool query_only);

@@ -22,33 +22,12 @@
 #include <initializer_list>
 #include <type_traits>
 
-#include "quant_common.h"
-#include "quant_layout.h"
+#include "qblock_i8.h"
 
 namespace {
 
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-struct QBlockArgs {
-    int N, H, W, OH, OW, stride;
-    int CBin, Cin32, Ce32, CBo;        // input channel blocks (16) / chunks (32); expanded chunks; output blocks
-    int Co;                            // output channels (the rest of the last block is padding)
-    int NB, TH, PH, PW, P, Ppad, Q;    // tile: images, output rows, patch rows / columns / positions, output positions
-    int n_row_tiles, n_tiles;
-    int o_xl, o_e, o_w1, o_w2, o_wdw, o_tab, o_ptab;  // LDS byte offsets
-    int packed_units;                  // 16-byte units of weights and tables: the LDS bytes from o_w1 to o_ptab
-    int split;                         // stage D deals (position tile, channel chunk) units to the waves (few position tiles)
-    float zp1f, zp2f, zp3f;            // zero points of the three convolutions' own outputs
-    QAct act1, act2;
-    int has_act1, has_act2;
-    uint32_t pad_e4;                   // the depthwise input zero point ^ 0x80 in every byte
-    int half_last;                     // the last chunk of expanded channels holds at most 16 real ones
-    int has_res, fast_div;             // fast_div: the scales allow the unscaled division sequence
-    float ry_rcp;                      // refined reciprocal of ry_scale
-    float ra_scale, rb_scale, ry_scale;  // residual add: a = projection output, b = block input, y = sum
-    int ra_zp, rb_zp, ry_zp;
-};
 
 __device__ __forceinline__ i32x4 as_i32x4(const uint4 &v) {
     i32x4 r;
@@ -515,22 +494,28 @@ qblock_chain_kernel(QBlockChain c) {
     }
 }
 
+// A block's two activation tables and the table of patch positions of a whole image (row; bit 31: a halo column or past the patch),
+// for qblock_image_i8.hip.
+__global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, int P, uint8_t *out) {
+    const int tid = threadIdx.x;
+    const uint8_t b = uint8_t(tid);
+    out[tid] = uint8_t((a.has_act1 ? qact_apply(b, a.act1) : b) ^ 0x80);
+    out[256 + tid] = uint8_t((a.has_act2 ? qact_apply(b, a.act2) : b) ^ 0x80);
+    int *ptab = reinterpret_cast<int *>(out + 512);
+    for (int p = tid; p < ((P + 31) & ~31); p += 256) {
+        const int pp = min(p, P - 1), ph = pp / a.PW, pw = pp - ph * a.PW;
+        ptab[p] = ph | ((p >= P || pw == 0 || pw == a.PW - 1) ? int(0x80000000u) : 0);
+    }
+}
+
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 size_t align16(size_t v) { return (v + 15) & ~size_t(15); }
 
 bool conv1x1(const zant_qconv_desc *d) { return d && d->K > 0 && d->C > 0 && (d->n_wscale == 1 || d->n_wscale == d->K); }
 
-// What a launch needs of one block: its kernel arguments, LDS bytes, instantiation and packed weights.
-struct QBlockPrep {
-    QBlockArgs a;
-    size_t lds_bytes;
-    int CO32, MQv;
-    const uint4 *packed;
-};
+}  // namespace
 
-// Plans a block's tile, (re)packs its weights and tables into `slot` (or the context workspace) and fills the kernel
-// arguments.  force_nb > 0: tiles of exactly that many whole images, or 1.  plan_only: no packing, no pointers needed.
-int qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *expand, const zant_qconv_desc *dw, int64_t dw_stride,
+int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *expand, const zant_qconv_desc *dw, int64_t dw_stride,
                    const zant_qconv_desc *project, int residual, float add_scale, int add_zp, const int64_t ydim[4], bool plan_only,
                    zant_pack_slot *slot, int force_nb, QBlockPrep *out) {
     if (!ctx || !xdim || !ydim || !expand || !dw || !project) return ZANT_NullPointer;
@@ -658,6 +643,7 @@ int qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *
         out->CO32 = CO32;
         out->lds_bytes = cap_used;
     }
+    out->o_lut = int(align256(w1_bytes + w2_bytes + wdw_bytes + tab_bytes));
     if (plan_only) {
         out->a = a;
         out->packed = nullptr;
@@ -672,7 +658,7 @@ int qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *
     // the depthwise convolution, then the tables m1 c1 m2 c2 (CeP entries each) m3 c3 (kp3 entries each)
     const size_t o_w1p = 256, o_w2p = o_w1p + w1_bytes, o_wm = o_w2p + w2_bytes, o_m1 = o_wm + wdw_bytes, o_c1 = o_m1 + kp1 * 4,
                  o_m2 = o_c1 + kp1 * 4, o_c2 = o_m2 + kp1 * 4, o_m3 = o_c2 + kp1 * 4, o_c3 = o_m3 + kp3 * 4,
-                 static_bytes = align256(o_c3 + kp3 * 4);
+                 o_tables = o_w1p + size_t(out->o_lut), static_bytes = align256(o_tables + 512 + size_t((p_img + 31) & ~int64_t(31)) * 4);
     if (o_c3 + kp3 * 4 - o_w1p != w1_bytes + w2_bytes + wdw_bytes + tab_bytes || size_t(a.o_ptab - a.o_w1) != o_c3 + kp3 * 4 - o_w1p)
         return ZANT_InvalidInput;  // the two layouts must stay in step
     void *ws = nullptr, *dyn = nullptr;
@@ -686,19 +672,6 @@ int qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *
     int32_t *c1 = reinterpret_cast<int32_t *>(base + o_c1), *c2 = reinterpret_cast<int32_t *>(base + o_c2),
             *c3 = reinterpret_cast<int32_t *>(base + o_c3);
     uint32_t *wmk = reinterpret_cast<uint32_t *>(base + o_wm);
-    if (need_pack) {
-        int8_t *padvec = reinterpret_cast<int8_t *>(base + 16);
-        rc = zant_qpack_dense(ctx, expand->w, expand->w_scale, expand->n_wscale, expand->bias, int(Ce), int(Cin), 1, 32,
-                              expand->x_scale, expand->x_zp, expand->y_scale, w1p, m1, c1, padvec);
-        if (rc) return rc;
-        rc = zant_qpack_depthwise(ctx, dw->w, dw->w_scale, dw->n_wscale, dw->bias, int(Ce), CeP, dw->x_scale, dw->x_zp,
-                                  dw->y_scale, wmk, m2, c2);
-        if (rc) return rc;
-        rc = zant_qpack_dense(ctx, project->w, project->w_scale, project->n_wscale, project->bias, int(Co), int(Ce), 1, 32,
-                              project->x_scale, project->x_zp, project->y_scale, w2p, m3, c3, padvec + 16);
-        if (rc) return rc;
-    }
-
     a.zp1f = float(expand->y_zp); a.zp2f = float(dw->y_zp); a.zp3f = float(project->y_zp);
     a.has_act1 = expand->act != ZANT_ACT_NONE;
     a.act1.act = expand->act; a.act1.alpha = expand->act_alpha; a.act1.in_scale = expand->y_scale; a.act1.in_zp = expand->y_zp;
@@ -715,20 +688,33 @@ int qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *
     a.fast_div = residual && zant_fast_div_ok(a.ra_scale, a.rb_scale, add_scale);
     a.ry_rcp = a.fast_div ? zant_refined_rcp(add_scale) : 0.0f;
 
+    if (need_pack) {
+        int8_t *padvec = reinterpret_cast<int8_t *>(base + 16);
+        rc = zant_qpack_dense(ctx, expand->w, expand->w_scale, expand->n_wscale, expand->bias, int(Ce), int(Cin), 1, 32,
+                              expand->x_scale, expand->x_zp, expand->y_scale, w1p, m1, c1, padvec);
+        if (rc) return rc;
+        rc = zant_qpack_depthwise(ctx, dw->w, dw->w_scale, dw->n_wscale, dw->bias, int(Ce), CeP, dw->x_scale, dw->x_zp,
+                                  dw->y_scale, wmk, m2, c2);
+        if (rc) return rc;
+        rc = zant_qpack_dense(ctx, project->w, project->w_scale, project->n_wscale, project->bias, int(Co), int(Ce), 1, 32,
+                              project->x_scale, project->x_zp, project->y_scale, w2p, m3, c3, padvec + 16);
+        if (rc) return rc;
+        hipLaunchKernelGGL(qblock_tables_kernel, dim3(1), dim3(256), 0, ctx->stream, a, int(p_img), reinterpret_cast<uint8_t *>(base + o_tables));
+        ZANT_LAUNCH_CHECK(ctx);
+    }
+
     a.packed_units = int((a.o_ptab - a.o_w1) / 16);
     out->a = a;
     out->packed = reinterpret_cast<const uint4 *>(base + o_w1p);
     return ZANT_OK;
 }
 
-}  // namespace
-
 int zant_qblock_blocked(zant_ctx *ctx, const uint8_t *x, const int64_t xdim[4], const zant_qconv_desc *expand,
                         const zant_qconv_desc *dw, int64_t dw_stride, const zant_qconv_desc *project, int residual,
                         float add_scale, int add_zp, uint8_t *y, const int64_t ydim[4], bool query_only, zant_pack_slot *slot) {
     QBlockPrep prep;
     if (!query_only && (!x || !y)) return ZANT_NullPointer;
-    const int rc = qblock_prepare(ctx, xdim, expand, dw, dw_stride, project, residual, add_scale, add_zp, ydim, query_only, slot, 0, &prep);
+    const int rc = zant_qblock_prepare(ctx, xdim, expand, dw, dw_stride, project, residual, add_scale, add_zp, ydim, query_only, slot, 0, &prep);
     if (rc || query_only) return rc;
     const QBlockArgs &a = prep.a;
     const size_t cap_used = prep.lds_bytes;
@@ -770,6 +756,8 @@ int zant_qblock_blocked(zant_ctx *ctx, const uint8_t *x, const int64_t xdim[4], 
 // the block before's output.
 int zant_qblock_chain(zant_ctx *ctx, int n, const zant_qblock_call *calls, bool query_only) {
     if (!ctx || !calls) return ZANT_NullPointer;
+    const int rc = zant_qblock_image_chain(ctx, n, calls, query_only);  // few images: one a workgroup, nothing stored in between
+    if (rc != 1) return rc;
     if (n < 2 || n > QB_CHAIN_MAX) return 1;
     QBlockChain chain;
     chain.n = n;
@@ -779,7 +767,7 @@ int zant_qblock_chain(zant_ctx *ctx, int n, const zant_qblock_call *calls, bool 
         const zant_qblock_call &c = calls[b];
         if (!query_only && (!c.x || !c.y || (b > 0 && c.x != calls[b - 1].y))) return b > 0 && c.x && c.y ? 1 : ZANT_NullPointer;
         QBlockPrep prep;
-        const int rc = qblock_prepare(ctx, c.xdim, c.expand, c.dw, c.dw_stride, c.project, c.residual, c.add_scale, c.add_zp, c.ydim,
+        const int rc = zant_qblock_prepare(ctx, c.xdim, c.expand, c.dw, c.dw_stride, c.project, c.residual, c.add_scale, c.add_zp, c.ydim,
                                       query_only, c.slot, NB, &prep);
         if (rc) return rc;
         if (prep.a.n_row_tiles != 1) return 1;
