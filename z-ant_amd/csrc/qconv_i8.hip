@@ -17,6 +17,7 @@
 #include "conv_tile.h"
 #include "quant_common.h"
 #include "quant_layout.h"
+#include "to_blocked.h"
 
 namespace {
 
@@ -79,7 +80,7 @@ __device__ __forceinline__ i32x4 as_i32x4_q(const uint4 &v) {
     return r;
 }
 
-// NCHW u8 -> [N][CB][H][W][16] signed (value - 128); channels beyond C are 0 (their weights are 0 too).
+// NCHW u8 -> [N][CB][H][W][16] signed (value - 128), tensors too large for blocked_tile (to_blocked.h).
 // Each thread turns 4 consecutive positions x 16 channels: sixteen 4-byte loads (one per channel
 // row), a 4x4 byte transpose per group of 4 channels, four 16-byte stores.
 __global__ void __launch_bounds__(256) to_blocked_s8_kernel(const uint8_t *__restrict__ x, uint4 *__restrict__ xb, int N,
@@ -123,61 +124,31 @@ __global__ void __launch_bounds__(256) to_blocked_s8_kernel(const uint8_t *__res
     }
 }
 
-// The same for planes of whole dwords (HW a multiple of 4, an aligned base) and fewer than 2^31 units.  A workgroup
-// turns 64 quads of positions (counted through the whole tensor: rows of (image, channel block) follow each other in
-// the output) x 16 channels.  Wavefront g loads the dwords of channels 4g .. 4g+3, a quad per lane (256 contiguous bytes
-// per load), transposes its 4 x 4 bytes with byte permutes (dword b: position b, channels 4g .. 4g+3) and writes the
-// four dwords to LDS row g; then thread u gathers unit u's four dwords (one per row, consecutive lanes on consecutive
-// banks) and stores its 16 bytes: a workgroup's stores are one run of 4 KB.
-// (One tile per workgroup: with two, all eight loads of a thread in flight together, the kernel was slower.)
-__global__ void __launch_bounds__(256) to_blocked_s8_quads_kernel(const uint8_t *__restrict__ x, uint4 *__restrict__ xb,
-                                                                 unsigned n_quads, int C, unsigned CB, unsigned HW4) {
-    __shared__ __attribute__((aligned(16))) uint32_t stage[4][256];
-    const unsigned g = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const unsigned qi = blockIdx.x * 64u + lane;
-    uint32_t r[4] = {0u, 0u, 0u, 0u};  // r[j] = 4 consecutive positions of channel c0 + j
-    if (qi < n_quads) {
-        const unsigned row = qi / HW4, q = qi - row * HW4;  // row = image * CB + channel block
-        const unsigned n = row / CB, cb = row - n * CB;
-        const int c0 = int(cb) * 16 + int(g) * 4;
-        const uint32_t *src = reinterpret_cast<const uint32_t *>(x) + (int64_t(n) * C * HW4 + q);
-        // The four loads leave together: a channel past C reads channel C - 1 instead of branching around its load
-        // (with a branch per load the compiler waited for each one before the next), and is zeroed afterwards.
-        uint32_t v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = __builtin_nontemporal_load(src + int64_t(min(c0 + j, C - 1)) * HW4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = c0 + j < C ? v[j] ^ 0x80808080u : 0u;
-    }
-    const uint32_t lo01 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);  // r0.0 r1.0 r0.1 r1.1
-    const uint32_t hi01 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);  // r0.2 r1.2 r0.3 r1.3
-    const uint32_t lo23 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
-    const uint32_t hi23 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
-    uint4 o;  // dword b: position b, channels c0 .. c0+3
-    o.x = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-    o.y = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-    o.z = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-    o.w = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
-    *reinterpret_cast<uint4 *>(&stage[g][lane * 4]) = o;
-    __syncthreads();
-    const unsigned u = threadIdx.x;
-    if (blockIdx.x * 64u + (u >> 2) < n_quads)
-        xb[int64_t(blockIdx.x) * 256 + u] = make_uint4(stage[0][u], stage[1][u], stage[2][u], stage[3][u]);
-}
+__global__ void __launch_bounds__(256) to_blocked_kernel(BlockedJob j) { blocked_tile(j, blockIdx.x); }
 
 // Packs OIHW int8 weights into [chunk][kblock][tap][half][K_BLK][16] (zero padded; fc_g > 0: the weights of a 1x1
 // layer with c_orig channels, read as a 1 x fc_g filter over C = 16 * ceil(c_orig / 16) / fc_g channels), and writes the
 // per-channel requantisation multiplier, the integer correction (bias + (128 - x_zp) * sum w), the
 // 16-byte padding vector (x_zp - 128 in every lane).
-__global__ void __launch_bounds__(256)
-qpack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, const int32_t *__restrict__ bias,
-             int8_t *__restrict__ wp, float *__restrict__ mult, int32_t *__restrict__ corr, int8_t *__restrict__ padvec,
-             int K, int C, int T, int n_chunks, int n_kblocks, int k_blk,
-             float x_scale, float y_scale, int x_zp, int n_wscale, int fc_g, int c_orig) {
-    const int64_t total = int64_t(n_chunks) * n_kblocks * T * QCC * k_blk;
-    const int64_t step = int64_t(gridDim.x) * blockDim.x;
-    const int64_t gid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (gid < 16) padvec[gid] = int8_t(x_zp - 128);
+struct QPackJob {
+    const int8_t *w;
+    const float *w_scale;
+    const int32_t *bias;
+    int8_t *wp;
+    float *mult;
+    int32_t *corr;
+    int8_t *padvec;
+    int K, C, T, n_chunks, n_kblocks, k_blk;
+    float x_scale, y_scale;
+    int x_zp, n_wscale, fc_g, c_orig;
+};
+// by workgroup `block` of `blocks`
+__device__ __forceinline__ void qpack(const QPackJob &p, unsigned block, unsigned blocks) {
+    const int K = p.K, C = p.C, T = p.T, n_kblocks = p.n_kblocks, k_blk = p.k_blk, fc_g = p.fc_g, c_orig = p.c_orig;
+    const int64_t total = int64_t(p.n_chunks) * n_kblocks * T * QCC * k_blk;
+    const int64_t step = int64_t(blocks) * 256;
+    const int64_t gid = int64_t(block) * 256 + threadIdx.x;
+    if (gid < 16) p.padvec[gid] = int8_t(p.x_zp - 128);
     for (int64_t i = gid; i < total; i += step) {
         int64_t r = i;
         const int j = int(r & 15); r >>= 4;
@@ -190,9 +161,9 @@ qpack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, co
         if (fc_g) {
             // regrouped 1x1 layer: "tap" t of 16-channel block b is channel block b * fc_g + t of the c_orig real channels
             const int oc = ((c >> 4) * fc_g + tap) * 16 + j;
-            wp[i] = (k < K && oc < c_orig) ? w[int64_t(k) * c_orig + oc] : int8_t(0);
+            p.wp[i] = (k < K && oc < c_orig) ? p.w[int64_t(k) * c_orig + oc] : int8_t(0);
         } else {
-            wp[i] = (k < K && c < C) ? w[(int64_t(k) * C + c) * T + tap] : int8_t(0);
+            p.wp[i] = (k < K && c < C) ? p.w[(int64_t(k) * C + c) * T + tap] : int8_t(0);
         }
     }
     // per output channel: one wavefront sums the channel's weights
@@ -203,20 +174,26 @@ qpack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, co
         int sum = 0;
         if (k < K) {
             const int row = fc_g ? c_orig : C * T;
-            const int8_t *wk = w + k * int64_t(row);
+            const int8_t *wk = p.w + k * int64_t(row);
             for (int e = lane; e < row; e += 64) sum += int(wk[e]);
         }
         for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
         if (lane == 0) {
             if (k < K) {
-                corr[k] = (bias ? bias[k] : 0) + (128 - x_zp) * sum;
-                mult[k] = (x_scale * w_scale[n_wscale == 1 ? 0 : k]) / y_scale;
+                p.corr[k] = (p.bias ? p.bias[k] : 0) + (128 - p.x_zp) * sum;
+                p.mult[k] = (p.x_scale * p.w_scale[p.n_wscale == 1 ? 0 : k]) / p.y_scale;
             } else {
-                corr[k] = 0;
-                mult[k] = 0.0f;
+                p.corr[k] = 0;
+                p.mult[k] = 0.0f;
             }
         }
     }
+}
+__global__ void __launch_bounds__(256) qpack_kernel(QPackJob p) { qpack(p, blockIdx.x, gridDim.x); }
+// Packing and an input's change of layout, which do not depend on each other, as one launch: workgroups [0, pack_blocks) pack.
+__global__ void __launch_bounds__(256) qpack_blocked_kernel(QPackJob p, BlockedJob j, unsigned pack_blocks) {
+    if (blockIdx.x < pack_blocks) qpack(p, blockIdx.x, pack_blocks);
+    else blocked_tile(j, blockIdx.x - pack_blocks);
 }
 
 // Bytes of the weight region of a staging buffer: the slab rounded up to one 16-byte unit per thread and round.
@@ -826,13 +803,18 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
     const int8_t *xb = x_blocked ? reinterpret_cast<const int8_t *>(x) : static_cast<const int8_t *>(dyn);
     const int grid = int(std::min<int64_t>(plan.t.n_tiles, int64_t(ctx->num_cus) * 2));
     const unsigned pb = unsigned(std::min<int64_t>(std::max<int64_t>(ceil_div64(int64_t(wp_bytes), 256), ceil_div64(int64_t(kpad), 4)), 1024));
-    if (need_pack) {
-        hipLaunchKernelGGL(qpack_kernel, dim3(pb), dim3(256), 0, ctx->stream, w, w_scale, bias, wp, mult, corr, padvec,
-                           g.K, g.C, T, plan.t.n_chunks, plan.t.n_kblocks, K_BLK, q.x_scale, q.y_scale, q.x_zp,
-                           q.n_wscale, fc_g, g0.C);
+    const QPackJob job = {w, w_scale, bias, wp, mult, corr, padvec, g.K, g.C, T, plan.t.n_chunks, plan.t.n_kblocks, K_BLK,
+                          q.x_scale, q.y_scale, q.x_zp, q.n_wscale, fc_g, g0.C};
+    BlockedJob layout;
+    const bool one_launch = need_pack && !x_blocked && zant_blocked_job(x, g0.N, g0.C, int64_t(g0.H) * g0.W, dyn, &layout);
+    if (one_launch) {
+        hipLaunchKernelGGL(qpack_blocked_kernel, dim3(pb + layout.blocks()), dim3(256), 0, ctx->stream, job, layout, pb);
+        ZANT_LAUNCH_CHECK(ctx);
+    } else if (need_pack) {
+        hipLaunchKernelGGL(qpack_kernel, dim3(pb), dim3(256), 0, ctx->stream, job);
         ZANT_LAUNCH_CHECK(ctx);
     }
-    if (!x_blocked) {
+    if (!x_blocked && !one_launch) {
         const int rc2 = zant_to_blocked(ctx, x, g0.N, g0.C, int64_t(g0.H) * g0.W, static_cast<uint8_t *>(dyn));
         if (rc2) return rc2;
     }
@@ -1340,21 +1322,34 @@ int run_qconv_smallc(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const flo
 // pre-expanded to one dword per (tap, channel) with the weight in that channel's byte lane and zeros elsewhere, and
 // acc[ch] += v_dot4_i32_i8(x_dword, w_dword) picks the channel's byte without any unpacking.
 // ------------------------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-qdw_pack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, const int32_t *__restrict__ bias,
-                uint32_t *__restrict__ wm, float *__restrict__ mult, int32_t *__restrict__ corr, int K, int kpad, float x_scale,
-                float y_scale, int x_zp, int n_wscale) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= kpad) return;
+struct QdwPackJob {
+    const int8_t *w;
+    const float *w_scale;
+    const int32_t *bias;
+    uint32_t *wm;
+    float *mult;
+    int32_t *corr;
+    int K, kpad;
+    float x_scale, y_scale;
+    int x_zp, n_wscale;
+};
+__device__ __forceinline__ void qdw_pack(const QdwPackJob &p, unsigned block) {
+    const int k = int(block * 256 + threadIdx.x);
+    if (k >= p.kpad) return;
     int sum = 0;
     const int cb = k >> 4, qd = (k >> 2) & 3, j = k & 3;
     for (int t = 0; t < 9; ++t) {
-        const int wv = k < K ? int(w[int64_t(k) * 9 + t]) : 0;
+        const int wv = k < p.K ? int(p.w[int64_t(k) * 9 + t]) : 0;
         sum += wv;
-        wm[((cb * 4 + qd) * 9 + t) * 4 + j] = uint32_t(uint8_t(wv)) << (8 * j);
+        p.wm[((cb * 4 + qd) * 9 + t) * 4 + j] = uint32_t(uint8_t(wv)) << (8 * j);
     }
-    corr[k] = k < K ? (bias ? bias[k] : 0) + (128 - x_zp) * sum : 0;
-    mult[k] = k < K ? (x_scale * w_scale[n_wscale == 1 ? 0 : k]) / y_scale : 0.0f;
+    p.corr[k] = k < p.K ? (p.bias ? p.bias[k] : 0) + (128 - p.x_zp) * sum : 0;
+    p.mult[k] = k < p.K ? (p.x_scale * p.w_scale[p.n_wscale == 1 ? 0 : k]) / p.y_scale : 0.0f;
+}
+__global__ void __launch_bounds__(256) qdw_pack_kernel(QdwPackJob p) { qdw_pack(p, blockIdx.x); }
+__global__ void __launch_bounds__(256) qdw_pack_blocked_kernel(QdwPackJob p, BlockedJob j, unsigned pack_blocks) {
+    if (blockIdx.x < pack_blocks) qdw_pack(p, blockIdx.x);
+    else blocked_tile(j, blockIdx.x - pack_blocks);
 }
 
 __global__ void __launch_bounds__(256)
@@ -1591,8 +1586,9 @@ size_t qdw_table_bytes(int C) {
     return 2 * align256(size_t(CB) * 64) + size_t(CB) * 144 * 4;
 }
 
-// x, y blocked; `tables` holds qdw_table_bytes(C) bytes that are (re)filled when need_pack is set.
-int run_qdw_blocked(zant_ctx *ctx, const uint8_t *xb, const int8_t *w, const float *w_scale, const int32_t *bias, uint8_t *yb,
+// x, y blocked; `tables` holds qdw_table_bytes(C) bytes that are (re)filled when need_pack is set.  x_nchw: the input as it came, still to
+// be written to xb (null: xb holds it).
+int run_qdw_blocked(zant_ctx *ctx, const uint8_t *x_nchw, uint8_t *xb, const int8_t *w, const float *w_scale, const int32_t *bias, uint8_t *yb,
                     const ConvGeom &g, const QConvArgs &q, void *tables, bool need_pack) {
     const int CB = (g.C + 15) / 16, n_pairs = (CB + 1) / 2, kpad = n_pairs * 32;
     const size_t o_corr = align256(size_t(kpad) * 4), o_w = 2 * o_corr;
@@ -1600,10 +1596,20 @@ int run_qdw_blocked(zant_ctx *ctx, const uint8_t *xb, const int8_t *w, const flo
     float *mult = reinterpret_cast<float *>(base);
     int32_t *corr = reinterpret_cast<int32_t *>(base + o_corr);
     uint32_t *wm = reinterpret_cast<uint32_t *>(base + o_w);
-    if (need_pack) {
-        hipLaunchKernelGGL(qdw_pack_kernel, dim3((kpad + 255) / 256), dim3(256), 0, ctx->stream, w, w_scale, bias, wm, mult,
-                           corr, g.K, kpad, q.x_scale, q.y_scale, q.x_zp, q.n_wscale);
+    const QdwPackJob job = {w, w_scale, bias, wm, mult, corr, g.K, kpad, q.x_scale, q.y_scale, q.x_zp, q.n_wscale};
+    const unsigned pb = unsigned(kpad + 255) / 256;
+    BlockedJob layout;
+    const bool one_launch = need_pack && x_nchw && zant_blocked_job(x_nchw, g.N, g.C, int64_t(g.H) * g.W, xb, &layout);
+    if (one_launch) {
+        hipLaunchKernelGGL(qdw_pack_blocked_kernel, dim3(pb + layout.blocks()), dim3(256), 0, ctx->stream, job, layout, pb);
         ZANT_LAUNCH_CHECK(ctx);
+    } else if (need_pack) {
+        hipLaunchKernelGGL(qdw_pack_kernel, dim3(pb), dim3(256), 0, ctx->stream, job);
+        ZANT_LAUNCH_CHECK(ctx);
+    }
+    if (x_nchw && !one_launch) {
+        const int rc = zant_to_blocked(ctx, x_nchw, g.N, g.C, int64_t(g.H) * g.W, xb);
+        if (rc) return rc;
     }
     const int64_t per_cb = int64_t(g.N) * g.OH * g.OW;
     KernelTimer kt(ctx);
@@ -1648,18 +1654,30 @@ int zant_qpack_dense(zant_ctx *ctx, const int8_t *w, const float *w_scale, int64
     const int n_chunks = (C + QCC - 1) / QCC, n_kblocks = (K + k_blk - 1) / k_blk;
     const int64_t wp_bytes = int64_t(n_chunks) * n_kblocks * T * QCC * k_blk, kpad = int64_t(n_kblocks) * k_blk;
     const unsigned pb = unsigned(std::min<int64_t>(std::max<int64_t>(ceil_div64(wp_bytes, 256), ceil_div64(kpad, 4)), 1024));
-    hipLaunchKernelGGL(qpack_kernel, dim3(pb), dim3(256), 0, ctx->stream, w, w_scale, bias, wp, mult, corr, padvec,
-                       K, C, T, n_chunks, n_kblocks, k_blk, x_scale, y_scale, x_zp, int(n_wscale), 0, C);
+    const QPackJob job = {w, w_scale, bias, wp, mult, corr, padvec, K, C, T, n_chunks, n_kblocks, k_blk, x_scale, y_scale, x_zp, int(n_wscale), 0, C};
+    hipLaunchKernelGGL(qpack_kernel, dim3(pb), dim3(256), 0, ctx->stream, job);
     ZANT_LAUNCH_CHECK(ctx);
     return ZANT_OK;
 }
 
 int zant_qpack_depthwise(zant_ctx *ctx, const int8_t *w, const float *w_scale, int64_t n_wscale, const int32_t *bias, int K,
                          int kpad, float x_scale, int x_zp, float y_scale, uint32_t *wm, float *mult, int32_t *corr) {
-    hipLaunchKernelGGL(qdw_pack_kernel, dim3((kpad + 255) / 256), dim3(256), 0, ctx->stream, w, w_scale, bias, wm, mult, corr, K,
-                       kpad, x_scale, y_scale, x_zp, int(n_wscale));
+    const QdwPackJob job = {w, w_scale, bias, wm, mult, corr, K, kpad, x_scale, y_scale, x_zp, int(n_wscale)};
+    hipLaunchKernelGGL(qdw_pack_kernel, dim3((kpad + 255) / 256), dim3(256), 0, ctx->stream, job);
     ZANT_LAUNCH_CHECK(ctx);
     return ZANT_OK;
+}
+
+bool zant_blocked_job(const uint8_t *x, int64_t N, int64_t C, int64_t HW, void *xb, BlockedJob *j) {
+    const int64_t CB = (C + 15) / 16, HW4 = (HW + 3) / 4, quads = N * CB * HW4;
+    if (quads >= (int64_t(1) << 29) || C > INT32_MAX) return false;
+    j->x = x;
+    j->xb = static_cast<uint4 *>(xb);
+    j->quads = unsigned(quads);
+    j->CB = unsigned(CB); j->HW = unsigned(HW); j->HW4 = unsigned(HW4); j->C = int(C);
+    j->d_hw4 = make_fastdiv(j->HW4);
+    j->d_cb = make_fastdiv(j->CB);
+    return true;
 }
 
 int zant_to_blocked(zant_ctx *ctx, const uint8_t *x, int64_t N, int64_t C, int64_t HW, uint8_t *xb) {
@@ -1667,15 +1685,14 @@ int zant_to_blocked(zant_ctx *ctx, const uint8_t *x, int64_t N, int64_t C, int64
     if (N <= 0 || C <= 0 || HW <= 0) return ZANT_OK;
     if (!x || !xb) return ZANT_NullPointer;
     const int64_t CB = (C + 15) / 16;
-    const int vec_ok = (HW % 4 == 0) && (reinterpret_cast<uintptr_t>(x) % 4 == 0);
     KernelTimer kt(ctx);
-    const int64_t quads = N * CB * (HW / 4);  // (16-byte units of the blocked tensor, four at a time)
-    if (vec_ok && quads < (int64_t(1) << 29))
-        hipLaunchKernelGGL(to_blocked_s8_quads_kernel, dim3(unsigned((quads + 63) / 64)), dim3(256), 0, ctx->stream, x,
-                           reinterpret_cast<uint4 *>(xb), unsigned(quads), int(C), unsigned(CB), unsigned(HW / 4));
+    BlockedJob j;
+    if (zant_blocked_job(x, N, C, HW, xb, &j))
+        hipLaunchKernelGGL(to_blocked_kernel, dim3(j.blocks()), dim3(256), 0, ctx->stream, j);
     else
         hipLaunchKernelGGL(to_blocked_s8_kernel, dim3(to_blocked_grid(ctx, N, CB, HW)), dim3(256), 0, ctx->stream, x,
-                           reinterpret_cast<uint4 *>(xb), int(N), int(C), int(CB), HW, vec_ok);
+                           reinterpret_cast<uint4 *>(xb), int(N), int(C), int(CB), HW,
+                           (HW % 4 == 0) && (reinterpret_cast<uintptr_t>(x) % 4 == 0));
     ZANT_LAUNCH_CHECK(ctx);
     return ZANT_OK;
 }
@@ -1739,14 +1756,9 @@ int zant_qlinearconv_layout_pool(zant_ctx *ctx, const uint8_t *x, const int64_t 
         int rc = zant_pack_region(ctx, slot, qdw_table_bytes(g.C), dyn_bytes, &tables, &dyn, &need_pack);
         if (rc) return rc;
         char *base = static_cast<char *>(dyn);
-        const uint8_t *xin = x;
-        if (!xb) {
-            rc = zant_to_blocked(ctx, x, g.N, g.C, int64_t(g.H) * g.W, reinterpret_cast<uint8_t *>(base));
-            if (rc) return rc;
-            xin = reinterpret_cast<uint8_t *>(base);
-        }
+        uint8_t *xin = xb ? const_cast<uint8_t *>(x) : reinterpret_cast<uint8_t *>(base);
         uint8_t *yout = yb ? y : reinterpret_cast<uint8_t *>(base + o_y);
-        rc = run_qdw_blocked(ctx, xin, w, w_scale, bias, yout, g, q, tables, need_pack);
+        rc = run_qdw_blocked(ctx, xb ? nullptr : x, xin, w, w_scale, bias, yout, g, q, tables, need_pack);
         if (rc) return rc;
         return yb ? ZANT_OK : zant_from_blocked(ctx, yout, g.N, g.K, int64_t(g.OH) * g.OW, y);
     }

@@ -21,6 +21,7 @@
 
 #include "quant_common.h"
 #include "quant_layout.h"
+#include "to_blocked.h"
 
 namespace {
 
@@ -802,16 +803,27 @@ qconv_ps_kernel(const int8_t *__restrict__ xb, const int8_t *__restrict__ wp, co
 // which the kernel's steps consume them, so that the weight stream is one run of addresses.  Also writes the
 // per-channel requantisation multiplier, the integer correction (bias + (128 - x_zp) * sum of weights) and the 16-byte
 // padding vector (x_zp - 128 in every lane).
-__global__ void __launch_bounds__(256)
-ps_pack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, const int32_t *__restrict__ bias,
-               int8_t *__restrict__ wp, float *__restrict__ mult, int32_t *__restrict__ corr, int8_t *__restrict__ padvec,
-               int K, int C, int NC, int NKP, int KP, float x_scale, float y_scale, int x_zp, int n_wscale) {
+struct PsPackJob {
+    const int8_t *w;
+    const float *w_scale;
+    const int32_t *bias;
+    int8_t *wp;
+    float *mult;
+    int32_t *corr;
+    int8_t *padvec;
+    int K, C, NC, NKP, KP;
+    float x_scale, y_scale;
+    int x_zp, n_wscale;
+};
+// by workgroup `block` of `blocks`
+__device__ __forceinline__ void ps_pack(const PsPackJob &p, unsigned block, unsigned blocks) {
+    const int K = p.K, C = p.C, NC = p.NC, NKP = p.NKP, KP = p.KP;
     // (fewer than 2^31 packed bytes: the host checks; KP is 64 or 128)
     const unsigned total = unsigned(NKP) * unsigned(NC) * 9u * 32u * unsigned(KP);
-    const unsigned step = gridDim.x * blockDim.x;
-    const unsigned gid = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned step = blocks * 256u;
+    const unsigned gid = block * 256u + threadIdx.x;
     const int kp_shift = KP == 128 ? 7 : 6;
-    if (gid < 16) padvec[gid] = int8_t(x_zp - 128);
+    if (gid < 16) p.padvec[gid] = int8_t(p.x_zp - 128);
     for (unsigned i = gid; i < total; i += step) {
         unsigned r = i;
         const int j = int(r & 15u); r >>= 4;
@@ -822,7 +834,7 @@ ps_pack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, 
         const unsigned kp = r9 / unsigned(NC);
         const int chunk = int(r9 - kp * unsigned(NC));
         const int k = int(kp) * KP + kk, c = chunk * 32 + half * 16 + j;
-        wp[i] = (k < K && c < C) ? w[(int64_t(k) * C + c) * 9 + tap] : int8_t(0);
+        p.wp[i] = (k < K && c < C) ? p.w[(int64_t(k) * C + c) * 9 + tap] : int8_t(0);
     }
     // per output channel: one wavefront sums the channel's weights, as dwords where the rows are whole aligned dwords
     // (four signed bytes summed by one dot product with ones), every load of a round issued before the first add
@@ -830,11 +842,11 @@ ps_pack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, 
     const int lane = threadIdx.x & 63;
     const unsigned wave = gid >> 6, n_waves = step >> 6;
     const int row = C * 9;
-    const bool dwords = (row & 3) == 0 && (reinterpret_cast<uintptr_t>(w) & 3) == 0;
+    const bool dwords = (row & 3) == 0 && (reinterpret_cast<uintptr_t>(p.w) & 3) == 0;
     for (unsigned k = wave; k < unsigned(kpad); k += n_waves) {
         int sum = 0;
         if (k < unsigned(K)) {
-            const int8_t *wk = w + int64_t(k) * row;
+            const int8_t *wk = p.w + int64_t(k) * row;
             if (dwords) {
                 const int *wk4 = reinterpret_cast<const int *>(wk);
                 const int n4 = row >> 2;
@@ -854,10 +866,16 @@ ps_pack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_scale, 
         }
         for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
         if (lane == 0) {
-            corr[k] = k < unsigned(K) ? (bias ? bias[k] : 0) + (128 - x_zp) * sum : 0;
-            mult[k] = k < unsigned(K) ? (x_scale * w_scale[n_wscale == 1 ? 0 : k]) / y_scale : 0.0f;
+            p.corr[k] = k < unsigned(K) ? (p.bias ? p.bias[k] : 0) + (128 - p.x_zp) * sum : 0;
+            p.mult[k] = k < unsigned(K) ? (p.x_scale * p.w_scale[p.n_wscale == 1 ? 0 : k]) / p.y_scale : 0.0f;
         }
     }
+}
+__global__ void __launch_bounds__(256) ps_pack_kernel(PsPackJob p) { ps_pack(p, blockIdx.x, gridDim.x); }
+// Packing and the input's change of layout as one launch: workgroups [0, pack_blocks) pack.
+__global__ void __launch_bounds__(256) ps_pack_blocked_kernel(PsPackJob p, BlockedJob j, unsigned pack_blocks) {
+    if (blockIdx.x < pack_blocks) ps_pack(p, blockIdx.x, pack_blocks);
+    else blocked_tile(j, blockIdx.x - pack_blocks);
 }
 
 size_t ps_align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -1020,16 +1038,23 @@ int zant_qconv_ps(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float 
     float *mult = reinterpret_cast<float *>(base + o_mult);
     int32_t *corr = reinterpret_cast<int32_t *>(base + o_corr);
     int8_t *wp = reinterpret_cast<int8_t *>(base + o_wp);
-    if (need_pack) {
-        const unsigned pb = unsigned(std::min<int64_t>(std::max<int64_t>(ceil_div64(int64_t(wp_bytes), 256), ceil_div64(p.kpad, 4)), 1024));
-        hipLaunchKernelGGL(ps_pack_kernel, dim3(pb), dim3(256), 0, ctx->stream, w, w_scale, bias, wp, mult, corr, padvec, g.K, g.C,
-                           p.NC, p.NKP, p.KP, q.x_scale, q.y_scale, q.x_zp, q.n_wscale);
+    const unsigned pb = unsigned(std::min<int64_t>(std::max<int64_t>(ceil_div64(int64_t(wp_bytes), 256), ceil_div64(p.kpad, 4)), 1024));
+    const PsPackJob job = {w, w_scale, bias, wp, mult, corr, padvec, g.K, g.C, p.NC, p.NKP, p.KP, q.x_scale, q.y_scale, q.x_zp, q.n_wscale};
+    BlockedJob layout;
+    const bool one_launch = need_pack && !x_blocked && !x_direct && zant_blocked_job(x, g.N, g.C, int64_t(g.H) * g.W, dyn, &layout);
+    if (one_launch) {
+        hipLaunchKernelGGL(ps_pack_blocked_kernel, dim3(pb + layout.blocks()), dim3(256), 0, ctx->stream, job, layout, pb);
+        ZANT_LAUNCH_CHECK(ctx);
+    } else if (need_pack) {
+        hipLaunchKernelGGL(ps_pack_kernel, dim3(pb), dim3(256), 0, ctx->stream, job);
         ZANT_LAUNCH_CHECK(ctx);
     }
     const int8_t *xb = reinterpret_cast<const int8_t *>(x);
     if (!x_blocked && !x_direct) {
-        rc = zant_to_blocked(ctx, x, g.N, g.C, int64_t(g.H) * g.W, static_cast<uint8_t *>(dyn));
-        if (rc) return rc;
+        if (!one_launch) {
+            rc = zant_to_blocked(ctx, x, g.N, g.C, int64_t(g.H) * g.W, static_cast<uint8_t *>(dyn));
+            if (rc) return rc;
+        }
         xb = static_cast<const int8_t *>(dyn);
     }
     const int grid = std::min(p.n_tiles, ctx->num_cus);
