@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "conv_tile.h"
+#include "patch_reads.h"
 #include "quant_common.h"
 #include "quant_layout.h"
 #include "to_blocked.h"
@@ -749,14 +750,15 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
     {
         const size_t cap2 = plan.t.n_tiles <= ctx->num_cus ? 160 * 1024 : 80 * 1024;
         const int pw0 = plan.t.PW;
-        double best_c = zant_patch_read_cycles(plan, g, pool, pw0);
+        const PatchReads reads(plan.WM, plan.MT, plan.t.NB, plan.t.TH, plan.t.PH, g.OW, g.sh, g.sw, pool, plan.t.POW);
+        double best_c = reads.cycles(pw0);
         int best_pw = pw0;
         for (int pw = pw0 + 1; pw <= pw0 + 9 && best_c > 1.0; ++pw) {
             const int p1 = plan.t.NB * plan.t.PH * pw, p1s = ((p1 + NT - 1) / NT) * NT;
             const size_t need = 2 * (size_t(w_region_bytes(T * QCC * K_BLK, NT)) + size_t(QCC) * p1s) + size_t(p1s) * 8 + 512 +
                                 size_t(plan.t.n_kblocks) * K_BLK * 8;
             if (p1s / NT > QR_MAX || need > cap2) break;
-            const double c = zant_patch_read_cycles(plan, g, pool, pw);
+            const double c = reads.cycles(pw);
             if (c < best_c * 0.9) { best_c = c; best_pw = pw; }
         }
         plan.t.PW = best_pw;
