@@ -32,16 +32,18 @@ struct ReduceGeom {
 
 __device__ __forceinline__ int64_t kept_base(const ReduceGeom &g, int64_t o) {
     int64_t base = 0;
-    for (int i = g.nk - 1; i >= 0; --i) {
+    for (int i = g.nk - 1; i > 0; --i) {
         const int64_t q = o / g.ksize[i];
         base += (o - q * g.ksize[i]) * g.kstride[i];
         o = q;
     }
-    return base;
+    return g.nk ? base + o * g.kstride[0] : base;  // (what is left indexes the outermost group)
 }
 
 // The innermost group is reduced (unit stride): LANES lanes share one result and walk the contiguous run together.
 // `seg` > 1 splits the run of a result into segments (few results, long runs); partial sums go to `part`.
+// Bound by memory where a wave has enough of it in flight and few instructions around it: the usual form, planes of one kept group,
+// takes no 64-bit division (each is some hundred instructions), and what does not fill a round of loads is asked for all at once too.
 template <int LANES>
 __global__ void __launch_bounds__(kThreads) reduce_mean_lanes_kernel(const float *__restrict__ x, float *__restrict__ y,
                                                                     ReduceGeom g, int seg, int64_t seg_len, int vec4) {
@@ -53,18 +55,19 @@ __global__ void __launch_bounds__(kThreads) reduce_mean_lanes_kernel(const float
     int64_t outer = 1;
     for (int i = 0; i < g.nr - 1; ++i) outer *= g.rsize[i];
     for (int64_t it = int64_t(blockIdx.x) * (kThreads / LANES) + threadIdx.x / LANES; it < items; it += step) {
-        const int64_t o = it / seg;
+        const int64_t o = seg > 1 ? it / seg : it;
         const int s = int(it - o * seg);
         const float *row = x + kept_base(g, o);
         const int64_t lo = s * seg_len, hi = lo + seg_len < inner ? lo + seg_len : inner;
         float sum = 0.0f;
         for (int64_t c = 0; c < outer; ++c) {  // outer reduced groups (none in the common trailing-axes case)
             int64_t off = 0, r = c;
-            for (int i = g.nr - 2; i >= 0; --i) {
+            for (int i = g.nr - 2; i > 0; --i) {
                 const int64_t q = r / g.rsize[i];
                 off += (r - q * g.rsize[i]) * g.rstride[i];
                 r = q;
             }
+            if (g.nr > 1) off += r * g.rstride[0];
             const float *p = row + off;
             if (vec4) {  // the host checked: base 16-byte aligned, every run start and length a multiple of 4
                 const f4 *p4 = reinterpret_cast<const f4 *>(p);
@@ -77,18 +80,86 @@ __global__ void __launch_bounds__(kThreads) reduce_mean_lanes_kernel(const float
                     a0 += (v0.x + v1.x) + (v2.x + v3.x); a1 += (v0.y + v1.y) + (v2.y + v3.y);
                     a2 += (v0.z + v1.z) + (v2.z + v3.z); a3 += (v0.w + v1.w) + (v2.w + v3.w);
                 }
-                for (; j < j_end; j += LANES) {
-                    const f4 v = __builtin_nontemporal_load(p4 + j);
-                    a0 += v.x; a1 += v.y; a2 += v.z; a3 += v.w;
-                }
+                f4 v[3];  // (zeros where the run has ended: they change no sum)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) v[i] = j + i * LANES < j_end ? __builtin_nontemporal_load(p4 + j + i * LANES) : f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < 3; ++i) { a0 += v[i].x; a1 += v[i].y; a2 += v[i].z; a3 += v[i].w; }
                 sum += (a0 + a1) + (a2 + a3);
             } else {
-                for (int64_t j = lo + lane; j < hi; j += LANES) sum += p[j];
+                for (int64_t j = lo + lane; j < hi; j += 8 * LANES) {  // eight loads in flight per lane
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = j + i * LANES < hi ? p[j + i * LANES] : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) sum += v[i];
+                }
             }
         }
 #pragma unroll
         for (int m = LANES / 2; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
         if (lane == 0) y[it] = seg > 1 ? sum : sum / float(g.count);
+    }
+}
+
+// Planes: one kept group, one contiguous run of `inner` elements per result, at most U loads of a lane.  A wave takes 256 / LANES
+// results at once, four to a group of LANES lanes, and asks for all of their elements before it adds any: with one result at a time a
+// plane of some hundred elements leaves one or two loads in flight and the six exchanges of its sum behind each.  The four sums of a
+// group of 64 lanes meet in one register on the way (two half-wave swaps, one row swap), so four exchanges are left for four results.
+// Each result is the same sum, in the same order, as reduce_mean_lanes_kernel's.  Means of 270000 planes of 13x13: 92 us one at a time, 64
+// without the divisions, 41 here (4.4 TB/s); of 64064 planes of 26x26 34, 29 and 26.5 (6.5 TB/s).
+template <int LANES, int U, typename V>
+__global__ void __launch_bounds__(kThreads) reduce_mean_planes_kernel(const V *__restrict__ x, float *__restrict__ y, int64_t outputs,
+                                                                      int inner, float count) {
+    constexpr int GROUPS = 64 / LANES, ROWS = 4 * GROUPS;  // a wave's
+    const int lane = threadIdx.x % LANES, group = threadIdx.x % 64 / LANES;
+    const int64_t row0 = (int64_t(blockIdx.x) * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64)) * ROWS;
+    if (row0 >= outputs) return;
+    V v[4][U];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int64_t row = row0 + group * 4 + r;
+        const V *p = x + (row < outputs ? row : outputs - 1) * inner;  // (behind the last result: read again, not written)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[r][u] = V{};
+            if (u * LANES < inner && u * LANES + lane < inner) {
+                if constexpr (sizeof(V) == 16) v[r][u] = __builtin_nontemporal_load(p + u * LANES + lane);
+                else v[r][u] = p[u * LANES + lane];  // (rows share cache lines)
+            }
+        }
+    }
+    float sum[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if constexpr (sizeof(V) == 16) {
+            V a = v[r][0];
+#pragma unroll
+            for (int u = 1; u < U; ++u) a += v[r][u];
+            sum[r] = 0.0f + ((a.x + a.y) + (a.z + a.w));  // (+0 for a plane of -0, as from a sum that starts at +0)
+        } else {
+            sum[r] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < U; ++u) sum[r] += v[r][u];
+        }
+    }
+    if constexpr (LANES == 64) {
+        auto both = [](auto sw) { return __uint_as_float(sw[0]) + __uint_as_float(sw[1]); };
+        const float s02 = both(__builtin_amdgcn_permlane32_swap(__float_as_uint(sum[0]), __float_as_uint(sum[2]), false, false));
+        const float s13 = both(__builtin_amdgcn_permlane32_swap(__float_as_uint(sum[1]), __float_as_uint(sum[3]), false, false));
+        float s = both(__builtin_amdgcn_permlane16_swap(__float_as_uint(s02), __float_as_uint(s13), false, false));
+#pragma unroll
+        for (int m = 8; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+        const int64_t row = row0 + lane / 16;  // (16 lanes hold one result each)
+        if (lane % 16 == 0 && row < outputs) y[row] = s / count;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t row = row0 + group * 4 + r;
+#pragma unroll
+            for (int m = LANES / 2; m >= 1; m >>= 1) sum[r] += __shfl_xor(sum[r], m, 64);
+            if (lane == 0 && row < outputs) y[row] = sum[r] / count;
+        }
     }
 }
 
@@ -556,6 +627,24 @@ extern "C" int zant_hip_reduce_mean_f32(zant_ctx *ctx, const float *x, const int
     }
     const int64_t items = g.outputs * seg;
     const int64_t per_lane_run = vec4 ? inner / 4 : inner;
+    // planes that a group of lanes reads in few loads each (three of vectors, eight of elements): four of them at once.  Longer runs fill
+    // a lane's loads by themselves; runs under 16 elements are left to the four-lane groups.
+    const int64_t groups = per_lane_run >= 64 ? 1 : 4;
+    const int64_t blocks = ceil_div64(g.outputs, groups * 4 * (kThreads / 64));
+    if (g.nk == 1 && g.nr == 1 && seg == 1 && per_lane_run >= 16 && per_lane_run <= (vec4 ? 192 : 512) && blocks < (int64_t(1) << 31)) {
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        KernelTimer kt(ctx);
+#define ZANT_PLANES(LANES, U, V)                                                                                                    \
+    hipLaunchKernelGGL((reduce_mean_planes_kernel<LANES, U, V>), dim3(unsigned(blocks)), dim3(kThreads), 0, ctx->stream,            \
+                       reinterpret_cast<const V *>(x), y, g.outputs, int(per_lane_run), float(g.count))
+        if (vec4) ZANT_PLANES(64, 3, f4);
+        else if (groups == 4) ZANT_PLANES(16, 4, float);
+        else if (inner <= 256) ZANT_PLANES(64, 4, float);
+        else ZANT_PLANES(64, 8, float);
+#undef ZANT_PLANES
+        ZANT_LAUNCH_CHECK(ctx);
+        return ZANT_OK;
+    }
     {
         KernelTimer kt(ctx);
         if (per_lane_run >= 64)
