@@ -1,4 +1,4 @@
-"""The mean of planes whose sizes are not whole vectors, few loads a lane."""
+"""Operators on planes whose sizes are not whole vectors: the mean of a plane, batch normalisation, 2x2 pooling."""
 import numpy as np
 import pytest
 import torch
@@ -34,3 +34,30 @@ def test_mean_of_planes_keeps_infinities_and_nan_to_their_plane(G):
     want[3], want[4], want[20] = np.inf, np.nan, 0.0
     np.testing.assert_array_equal(y, want)
     assert not np.signbit(y[20])
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 4), (3, 5, 5), (1, 1, 6), (2, 7, 3), (5, 1, 7), (4, 3, 13, 13), (3, 50, 27, 27), (9, 2, 4099), (7, 5, 9)])
+def test_batchnorm_of_planes_that_end_inside_a_vector(G, shape):
+    g = torch.Generator("cuda").manual_seed(sum(shape))
+    F = shape[1]
+    x = torch.randn(shape, device="cuda", generator=g)
+    gamma, beta, mean = (torch.randn(F, device="cuda", generator=g) for _ in range(3))
+    var = torch.rand(F, device="cuda", generator=g) + 0.1
+    y = G.tm.batchnorm(x, gamma, beta, mean, var, 1e-5)
+    s = (1, F) + (1,) * (len(shape) - 2)
+    centred = (x - mean.view(s)).double()
+    scaled = centred / (var + 1e-5).double().sqrt().view(s) * gamma.double().view(s)
+    # root, quotient, product and sum are rounded once each: half a unit in the last place of each step's result
+    bound = 2.0 ** -24 * (4 * scaled.abs() + (scaled + beta.double().view(s)).abs())
+    assert ((y.double() - scaled - beta.double().view(s)).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 4, 5), (2, 3, 5, 5), (3, 7, 13, 11), (2, 4, 4, 255), (1, 5, 31, 33), (2, 3, 64, 65), (5, 1, 27, 27)])
+def test_pools_of_planes_of_odd_width(G, shape):
+    x = torch.randn(shape, device="cuda", generator=torch.Generator("cuda").manual_seed(shape[3]))
+    x[0, 0, 0, 0], x[-1, -1, 1, 2] = float("inf"), float("nan")
+    w = x[:, :, :shape[2] // 2 * 2, :shape[3] // 2 * 2]
+    a, b, c, d = w[:, :, ::2, ::2], w[:, :, ::2, 1::2], w[:, :, 1::2, ::2], w[:, :, 1::2, 1::2]
+    np.testing.assert_array_equal(G.host(G.tm.avgpool(x, [2, 2], [2, 2])), (((a + b) + c + d) / 4).cpu().numpy())
+    y = G.tm.onnx_maxpool(x, [2, 2], [2, 2], [1, 1], [0, 0, 0, 0])
+    np.testing.assert_array_equal(G.host(y), torch.fmax(torch.fmax(a, b), torch.fmax(c, d)).cpu().numpy())

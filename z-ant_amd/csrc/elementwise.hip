@@ -2,6 +2,7 @@
 // Reshape and MaxPool (f32 and u8).  All are HBM-bound: 16-byte vector accesses on the contiguous
 // axis, grid-stride loops sized to a few waves per CU.
 #include "common.h"
+#include "fastdiv.h"
 
 namespace {
 
@@ -430,7 +431,8 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T 
 // 2x2 / stride 2 on f32 planes that are not a whole number of vectors wide (26 x 26 -> 13 x 13 ...): a workgroup copies G
 // whole consecutive planes to LDS -- a contiguous run of the input, read as 16-byte vectors whatever the row length --
 // and writes their G * OH * OW results, also a contiguous run, as 16-byte vectors, four results per thread.  The rows of
-// a window are two 8-byte LDS reads (W is even).  G is a multiple of 4, so both runs start on 16-byte boundaries.
+// a window are two 8-byte LDS reads where W is even, four elements where it is odd.  G is a multiple of 4, so both runs start on
+// 16-byte boundaries.  Averages of 32064 planes of 27x27: 34 us by avgpool_f32_kernel, 22 here.
 constexpr int kPoolLdsFloats = 4 * 1024;  // 16 KB: eight workgroups (all 32 wave slots) share a CU
 template <bool AVG>  // AVG: the average in the reference's tap order (op_pooling.zig:373-408) instead of the maximum
 __global__ void __launch_bounds__(kThreads) pool_2x2s2_planes_f32_kernel(const float *__restrict__ x, float *__restrict__ y,
@@ -466,6 +468,10 @@ __global__ void __launch_bounds__(kThreads) pool_2x2s2_planes_f32_kernel(const f
         const int pz = small_div_host(o, OHW, inv_ohw), rem = o - pz * OHW;
         const int oh = small_div_host(rem, OW, inv_ow), ow = rem - oh * OW;
         const float *r = pl + pz * HW + 2 * oh * W + 2 * ow;
+        if (W & 1) {
+            if (AVG) return (((0.0f + r[0] + r[1]) + r[W]) + r[W + 1]) / 4.0f;
+            return fmaxf(fmaxf(r[0], r[1]), fmaxf(r[W], r[W + 1]));
+        }
         const f2 a = *reinterpret_cast<const f2 *>(r), b = *reinterpret_cast<const f2 *>(r + W);
         if (AVG) return (((a[0] + a[1]) + b[0]) + b[1]) / 4.0f;  // taps (0,0), (0,1), (1,0), (1,1), divided by their count
         return fmaxf(fmaxf(a[0], a[1]), fmaxf(b[0], b[1]));
@@ -579,7 +585,7 @@ int launch_maxpool(zant_ctx *ctx, const T *x, const int64_t xdim[4], T *y, const
                         (reinterpret_cast<uintptr_t>(x) % (sizeof(T) == 1 ? 16 : 8)) == 0 &&
                         (reinterpret_cast<uintptr_t>(y) % (sizeof(T) == 1 ? 8 : 4)) == 0 && g.OW / VEC < (1 << 18) && g.OH < (1 << 18);
     // f32 planes of a few KB whose rows are not whole vectors: the plane-staged kernel reads and writes 16-byte vectors
-    if (sizeof(T) == 4 && fast && g.W % 2 == 0 && g.W % 8 != 0 && int64_t(g.H) * g.W * 4 <= kPoolLdsFloats &&
+    if (sizeof(T) == 4 && fast && g.W % 8 != 0 && int64_t(g.H) * g.W * 4 <= kPoolLdsFloats &&
         int64_t(g.OH) * g.OW >= 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
         const int G = int(std::min<int64_t>((kPoolLdsFloats / (int64_t(g.H) * g.W)) & ~int64_t(3), 64));
         if (G >= 4 && ceil_div64(g.NC, G) < (int64_t(1) << 31)) {
@@ -727,6 +733,58 @@ __global__ void __launch_bounds__(kThreads) batchnorm_vec_f32_kernel(const float
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = (v[u][e] - m[u]) / sd[u] * ga[u] + be[u];
             __builtin_nontemporal_store(o, y4 + j);
+        }
+    }
+}
+
+// Any inner from 4 up, 16-byte aligned pointers: a vector lies in one (batch, feature) pair or two.  The parameters of the pairs that a
+// workgroup's elements lie in are gathered into LDS, the root taken once a pair, behind the loads of its vectors; the tensor's last
+// elements, short of a vector, are one thread's.  Bound by memory.  The scalar kernel divides in 64 bits for every element: 32064 planes
+// of 27x27 58 us, both pairs' parameters gathered and their roots taken by every vector 38, here 34.
+__global__ void __launch_bounds__(kThreads) batchnorm_pairs_f32_kernel(const float *__restrict__ x, float *__restrict__ y,
+                                                                       const float *__restrict__ gamma, const float *__restrict__ beta,
+                                                                       const float *__restrict__ mean, const float *__restrict__ var,
+                                                                       float eps, int64_t total, uint32_t inner, FastDiv by_inner,
+                                                                       uint32_t features) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    constexpr uint32_t ELEMS = kThreads * ZANT_STREAM_U * 4;
+    __shared__ f4 pairs[ELEMS / 4 + 2];  // deviation, mean, gamma, beta; inner >= 4: (inner - 1 + ELEMS - 1) / inner + 1 pairs at most
+    const f4 *x4 = reinterpret_cast<const f4 *>(x);
+    f4 *y4 = reinterpret_cast<f4 *>(y);
+    const int64_t total4 = total >> 2, base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
+    const int64_t pair0 = int64_t(blockIdx.x) * ELEMS / inner;
+    const uint32_t off0 = uint32_t(int64_t(blockIdx.x) * ELEMS - pair0 * inner), f0 = uint32_t(pair0 % features);
+    f4 v[ZANT_STREAM_U];
+#pragma unroll
+    for (int u = 0; u < ZANT_STREAM_U; ++u) {
+        const int64_t j = base + u * kThreads;
+        if (j < total4) v[u] = __builtin_nontemporal_load(x4 + j);
+    }
+    const uint32_t n_pairs = fastdiv(off0 + ELEMS - 1, by_inner) + 1;
+    for (uint32_t i = threadIdx.x; i < n_pairs; i += kThreads) {
+        const uint32_t f = (f0 + i) % features;
+        pairs[i] = f4{sqrtf(var[f] + eps), mean[f], gamma[f], beta[f]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < ZANT_STREAM_U; ++u) {
+        const int64_t j = base + u * kThreads;
+        const uint32_t local = off0 + (uint32_t(threadIdx.x) + uint32_t(u * kThreads)) * 4, q = fastdiv(local, by_inner);
+        if (j < total4) {
+            const uint32_t left = inner - (local - q * inner);  // elements of the first pair from here on
+            const f4 p = pairs[q], next = pairs[left < 4 ? q + 1 : q];
+            f4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const f4 a = uint32_t(e) < left ? p : next;
+                o[e] = (v[u][e] - a[1]) / a[0] * a[2] + a[3];
+            }
+            __builtin_nontemporal_store(o, y4 + j);
+        } else if (j == total4) {
+            for (uint32_t e = 0; e < uint32_t(total & 3); ++e) {
+                const f4 a = pairs[fastdiv(local + e, by_inner)];
+                y[total4 * 4 + e] = (x[total4 * 4 + e] - a[1]) / a[0] * a[2] + a[3];
+            }
         }
     }
 }
@@ -962,7 +1020,7 @@ extern "C" int zant_hip_avgpool2d_f32(zant_ctx *ctx, const float *x, const int64
     const bool fast = g.kh == 2 && g.kw == 2 && g.sh == 2 && g.sw == 2 && !g.pt && !g.pl && 2 * g.OH <= g.H && 2 * g.OW <= g.W &&
                       g.OW % 2 == 0 && g.W % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 8 == 0;
     // small planes, 2x2 / stride 2, no padding: the plane-staged kernel of the max pool
-    if (g.kh == 2 && g.kw == 2 && g.sh == 2 && g.sw == 2 && !g.pt && !g.pl && 2 * g.OH <= g.H && 2 * g.OW <= g.W && g.W % 2 == 0 &&
+    if (g.kh == 2 && g.kw == 2 && g.sh == 2 && g.sw == 2 && !g.pt && !g.pl && 2 * g.OH <= g.H && 2 * g.OW <= g.W &&
         int64_t(g.H) * g.W * 4 <= kPoolLdsFloats && int64_t(g.OH) * g.OW >= 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
         reinterpret_cast<uintptr_t>(y) % 16 == 0) {
         const int G = int(std::min<int64_t>((kPoolLdsFloats / (int64_t(g.H) * g.W)) & ~int64_t(3), 64));
@@ -1021,9 +1079,13 @@ extern "C" int zant_hip_batchnorm_f32(zant_ctx *ctx, const float *x, const int64
     if (xdim[1] > INT32_MAX) return ZANT_InvalidDimensions;
     if (!x || !y || !gamma || !beta || !mean || !var) return ZANT_NullPointer;
     KernelTimer kt(ctx);
-    if (inner % 4 == 0 && inner / 4 < (int64_t(1) << 31) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) {
+    const bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    if (aligned && inner % 4 == 0 && inner / 4 < (int64_t(1) << 31)) {
         hipLaunchKernelGGL(batchnorm_vec_f32_kernel, dim3(zant_stream_grid(total / 4)), dim3(kThreads), 0, ctx->stream,
                            x, y, gamma, beta, mean, var, epsilon, total / 4, uint32_t(inner / 4), uint32_t(xdim[1]));
+    } else if (aligned && inner >= 4 && inner < (int64_t(1) << 30)) {  // (a workgroup's offsets stay below 2^31)
+        hipLaunchKernelGGL(batchnorm_pairs_f32_kernel, dim3(zant_stream_grid(ceil_div64(total, 4))), dim3(kThreads), 0, ctx->stream,
+                           x, y, gamma, beta, mean, var, epsilon, total, uint32_t(inner), make_fastdiv(unsigned(inner)), uint32_t(xdim[1]));
     } else {
         hipLaunchKernelGGL(batchnorm_f32_kernel, dim3(grid_for(total, kThreads, ctx->num_cus)), dim3(kThreads), 0, ctx->stream, x, y,
                            gamma, beta, mean, var, epsilon, total, inner, int(xdim[1]));
