@@ -1,7 +1,9 @@
-"""Operators on planes whose sizes are not whole vectors: the mean of a plane, batch normalisation, 2x2 pooling."""
+"""Operators on planes whose sizes are not whole vectors: means, batch normalisation, 2x2 pooling, f32 and u8."""
 import numpy as np
 import pytest
 import torch
+
+from oracle import oracle as zo
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +63,31 @@ def test_pools_of_planes_of_odd_width(G, shape):
     np.testing.assert_array_equal(G.host(G.tm.avgpool(x, [2, 2], [2, 2])), (((a + b) + c + d) / 4).cpu().numpy())
     y = G.tm.onnx_maxpool(x, [2, 2], [2, 2], [1, 1], [0, 0, 0, 0])
     np.testing.assert_array_equal(G.host(y), torch.fmax(torch.fmax(a, b), torch.fmax(c, d)).cpu().numpy())
+
+
+# rows of 3 results (byte by byte), 4 to 7 (vectors of four), 8 up (of eight, the last moved back); odd heights, one row, one plane
+@pytest.mark.parametrize("shape", [(2, 3, 5, 7), (1, 1, 2, 8), (3, 2, 7, 9), (2, 5, 6, 15), (1, 1, 2, 16), (2, 3, 9, 17), (3, 7, 13, 11),
+                                   (4, 5, 27, 27), (3, 2, 50, 33), (1, 2, 4, 34), (2, 3, 48, 50), (40, 30, 21, 43)])
+def test_byte_pools_of_any_width(G, shape):
+    x = torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=torch.Generator("cuda").manual_seed(shape[3]))
+    w = x[:, :, :shape[2] // 2 * 2, :shape[3] // 2 * 2]
+    want = torch.maximum(torch.maximum(w[:, :, ::2, ::2], w[:, :, ::2, 1::2]), torch.maximum(w[:, :, 1::2, ::2], w[:, :, 1::2, 1::2]))
+    assert torch.equal(G.tm.onnx_maxpool(x, [2, 2], [2, 2], [1, 1], [0, 0, 0, 0]), want)
+    off = torch.cat([x.flatten(), x.flatten()[:3]])[3:].view(shape)  # from an odd address
+    assert off.data_ptr() % 4 == 3
+    y = torch.zeros(want.numel() + 5, dtype=torch.uint8, device="cuda")
+    G.tm.onnx_maxpool_lean(off, y[5:].view(want.shape), [2, 2], [2, 2], [1, 1], [0, 0, 0, 0])
+    w = off[:, :, :shape[2] // 2 * 2, :shape[3] // 2 * 2]
+    want = torch.maximum(torch.maximum(w[:, :, ::2, ::2], w[:, :, ::2, 1::2]), torch.maximum(w[:, :, 1::2, ::2], w[:, :, 1::2, 1::2]))
+    assert torch.equal(y[5:].view(want.shape), want) and not y[:5].any()
+
+
+@pytest.mark.parametrize("hw", [(1, 1), (3, 5), (4, 4), (1, 17), (7, 7), (8, 8), (5, 13), (13, 13), (31, 33), (32, 32), (25, 41), (57, 55), (90, 91)])
+@pytest.mark.parametrize("planes", [1, 3, 17, 260])
+def test_byte_means_of_any_plane(G, planes, hw):
+    g = np.random.default_rng(planes * 1000 + hw[0] * hw[1])
+    x = g.integers(0, 256, (1, planes) + hw, dtype=np.uint8)
+    want = zo.qlinear_global_avgpool(x, 0.05, 128, 0.02, 110)
+    np.testing.assert_array_equal(G.host(G.tm.qlinear_global_avgpool(G.dev(x), 0.05, 128, 0.02, 110)), want)
+    buf = G.dev(np.concatenate([np.zeros(3, np.uint8), x.ravel()]))  # from an odd address
+    np.testing.assert_array_equal(G.host(G.tm.qlinear_global_avgpool(buf[3:].view(x.shape), 0.05, 128, 0.02, 110)), want)

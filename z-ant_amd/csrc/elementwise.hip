@@ -361,7 +361,10 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_kernel(const T *__rest
 // kThreads * ZANT_STREAM_U consecutive output vectors of the flattened [NC * OH, OW / VEC] grid and issues all its
 // loads before its stores, nontemporal both ways (the streaming pattern of the elementwise kernels).  Needs W even
 // (f32) or a multiple of 16 (u8), OW a multiple of VEC and aligned bases; the host checks.
-template <typename T, int VEC>
+// ANY: any W and any alignment, OW >= VEC.  The last vector of a row starts early enough to end with the row (what it shares with the
+// one before is written twice, the same), and loads are plain: neighbours share cache lines.  1000x64x48x50 u8: 106 us with a thread's
+// inputs read byte by byte, 43 here; 48000 planes of 27x27 24 -> 12.
+template <typename T, int VEC, bool ANY>
 __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T *__restrict__ x, T *__restrict__ y, PoolGeom g,
                                                                       int64_t total_vec, int ow_vec, float inv_ow_vec,
                                                                       float inv_oh) {
@@ -375,6 +378,10 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T 
     const int col0 = int((int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U)) - row0 * ow_vec);
     const int64_t nc0 = row0 / g.OH;
     const int oh0 = int(row0 - nc0 * g.OH);
+    typedef f2 f2_any __attribute__((aligned(4)));
+    typedef u4 u4_any __attribute__((aligned(1)));
+    typedef u2 u2_any __attribute__((aligned(1)));
+    typedef unsigned u1_any __attribute__((aligned(1)));
     u4 r0[ZANT_STREAM_U], r1[ZANT_STREAM_U];
     int64_t dst[ZANT_STREAM_U];
 #pragma unroll
@@ -384,10 +391,22 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T 
         const int ohl = oh0 + drow;                                       // rows past this plane roll over
         const int dnc = small_div_host(ohl, g.OH, inv_oh), oh = ohl - dnc * g.OH;
         const int64_t nc = nc0 + dnc;
-        const T *p0 = x + (nc * g.H + 2 * oh) * int64_t(g.W) + int64_t(oc) * 2 * VEC;
-        dst[u] = (nc * g.OH + oh) * int64_t(g.OW) + int64_t(oc) * VEC;
+        const int64_t ow = ANY ? min(oc * VEC, g.OW - VEC) : int64_t(oc) * VEC;
+        const T *p0 = x + (nc * g.H + 2 * oh) * int64_t(g.W) + 2 * ow;
+        dst[u] = (nc * g.OH + oh) * int64_t(g.OW) + ow;
         if (base + u * kThreads < total_vec) {
-            if (F32) {
+            if constexpr (ANY && F32) {
+                const f2 a = *reinterpret_cast<const f2_any *>(p0), b = *reinterpret_cast<const f2_any *>(p0 + g.W);
+                r0[u][0] = __float_as_uint(a[0]); r0[u][1] = __float_as_uint(a[1]);
+                r1[u][0] = __float_as_uint(b[0]); r1[u][1] = __float_as_uint(b[1]);
+            } else if constexpr (ANY && VEC == 4) {
+                const u2 a = *reinterpret_cast<const u2_any *>(p0), b = *reinterpret_cast<const u2_any *>(p0 + g.W);
+                r0[u][0] = a[0]; r0[u][1] = a[1];
+                r1[u][0] = b[0]; r1[u][1] = b[1];
+            } else if constexpr (ANY) {
+                r0[u] = *reinterpret_cast<const u4_any *>(p0);
+                r1[u] = *reinterpret_cast<const u4_any *>(p0 + g.W);
+            } else if (F32) {
                 const f2 a = __builtin_nontemporal_load(reinterpret_cast<const f2 *>(p0));
                 const f2 b = __builtin_nontemporal_load(reinterpret_cast<const f2 *>(p0 + g.W));
                 r0[u][0] = __float_as_uint(a[0]); r0[u][1] = __float_as_uint(a[1]);
@@ -419,11 +438,14 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T 
             };
             u2 o;
 #pragma unroll
-            for (int d = 0; d < 2; ++d) {
+            for (int d = 0; d < (VEC == 4 ? 1 : 2); ++d) {
                 const uint32_t lo = window_max(r0[u][d * 2], r1[u][d * 2]), hi = window_max(r0[u][d * 2 + 1], r1[u][d * 2 + 1]);
                 o[d] = __builtin_amdgcn_perm(hi, lo, 0x06040200u);  // bytes 0, 2 of lo then bytes 0, 2 of hi
             }
-            __builtin_nontemporal_store(o, reinterpret_cast<u2 *>(reinterpret_cast<uint8_t *>(y) + dst[u]));
+            uint8_t *out = reinterpret_cast<uint8_t *>(y) + dst[u];
+            if constexpr (ANY && VEC == 4) *reinterpret_cast<u1_any *>(out) = o[0];
+            else if constexpr (ANY) *reinterpret_cast<u2_any *>(out) = o;
+            else __builtin_nontemporal_store(o, reinterpret_cast<u2 *>(out));
         }
     }
 }
@@ -611,12 +633,18 @@ int launch_maxpool(zant_ctx *ctx, const T *x, const int64_t xdim[4], T *y, const
             return ZANT_OK;
         }
     }
-    if (stream) {
-        const int ow_vec = g.OW / VEC;
+    // rows that are not whole vectors: vectors at any alignment, the last one of a row moved back (u8: eight results, four in rows under
+    // eight; f32: one)
+    const int any = !fast || g.OH >= (1 << 18) || g.OW >= (1 << 18) ? 0 : sizeof(T) == 4 ? 1 : g.OW >= 8 ? 8 : g.OW >= 4 ? 4 : 0;
+    if (stream || any) {
+        const int per = stream ? VEC : any, ow_vec = (g.OW + per - 1) / per;
         const int64_t total_vec = g.NC * g.OH * ow_vec;
         KernelTimer kt(ctx);
-        hipLaunchKernelGGL((maxpool_2x2s2_stream_kernel<T, VEC>), dim3(zant_stream_grid(total_vec)), dim3(kThreads), 0, ctx->stream,
-                           x, y, g, total_vec, ow_vec, 1.0f / float(ow_vec), 1.0f / float(g.OH));
+        auto *kernel = maxpool_2x2s2_stream_kernel<T, VEC, false>;
+        if (!stream) kernel = sizeof(T) == 1 && any == 4 ? maxpool_2x2s2_stream_kernel<T, sizeof(T) == 1 ? 4 : 1, true>
+                                                         : maxpool_2x2s2_stream_kernel<T, VEC, true>;
+        hipLaunchKernelGGL(kernel, dim3(zant_stream_grid(total_vec)), dim3(kThreads), 0, ctx->stream, x, y, g, total_vec, ow_vec,
+                           1.0f / float(ow_vec), 1.0f / float(g.OH));
     } else if (fast) {
         constexpr int PER = sizeof(T) == 1 ? 8 : 2;
         const int64_t items = g.NC * g.OH * ((g.OW + PER - 1) / PER);
