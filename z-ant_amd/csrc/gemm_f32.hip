@@ -179,30 +179,53 @@ __global__ void __launch_bounds__(256)
 gemm_f32_skinny_kernel(const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ C,
                        float *__restrict__ Y, GemmArgs g, int ldb_k, int ldb_n, int softmax) {
     __shared__ f32x4 bs[SK_KC * 4];  // [k][4 units of 4 columns]; unit u of row k at u ^ ((k >> 2) & 3): conflict-free reads
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row0 = (blockIdx.x * 4 + wave) * 4;
     float v[64];
 #pragma unroll
     for (int i = 0; i < 64; ++i) v[i] = 0.0f;
+    // rows and columns past the last one read the last one again: their results are not stored
+    const float *rows[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rows[r] = A + int64_t(min(row0 + r, g.M - 1)) * g.lda;
+    const float *col = B + int64_t(min(tid & 15, g.N - 1)) * ldb_n;
 
     for (int kc = 0; kc < g.K; kc += SK_KC) {
         const int kend = min(SK_KC, g.K - kc);
-        // this lane's A values of the whole stage first: 32 independent loads in flight while B is staged
-        float a[SK_KC / 64][4];
+        // this lane's A values of the whole stage first: 32 independent loads in flight while B is staged.  k past the end reads the
+        // last one and counts as zero: sixty-four loads under a branch each were more instructions, and more registers for their addresses
+        // (one workgroup a CU), than the arithmetic.  60000x512x7 72 -> 24 us (5 TB/s), 9000x2000x16 63 -> 28, 1x512x10 6.4 -> 4.7.
+        float a[SK_KC / 64][4], bv[SK_KC * 16 / 256];  // (B: all of a thread's loads are issued before the first LDS store, too)
+        auto load = [&](auto whole_tag) {
+            constexpr bool WHOLE = decltype(whole_tag)::value;
+            int t4 = tid >> 4;
+            asm volatile("" : "+v"(t4));  // (or what is made from it is kept in registers from stage to stage)
+            const float *p = col + int64_t(kc + (WHOLE ? t4 : min(t4, kend - 1))) * ldb_k;
+            const int64_t step = int64_t(16) * ldb_k;
 #pragma unroll
-        for (int it = 0; it < SK_KC / 64; ++it)
+            for (int it = 0; it < SK_KC / 64; ++it) {
+                const uint32_t k = WHOLE ? it * 64 + lane : min(it * 64 + lane, kend - 1);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int k = it * 64 + lane;
-                a[it][r] = (k < kend && row0 + r < g.M) ? A[int64_t(row0 + r) * g.lda + kc + k] : 0.0f;
+                for (int r = 0; r < 4; ++r) a[it][r] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(rows[r] + kc) + k * 4u);
             }
-        // B stage: all of a thread's loads are issued before the first LDS store (fixed trip count, unrolled)
-        float bv[SK_KC * 16 / 256];
 #pragma unroll
-        for (int i = 0; i < SK_KC * 16 / 256; ++i) {
-            const int idx = i * 256 + tid, k = idx >> 4, n = idx & 15;
-            bv[i] = (k < kend && n < g.N) ? B[int64_t(kc + k) * ldb_k + int64_t(n) * ldb_n] : 0.0f;
-        }
+            for (int i = 0; i < SK_KC * 16 / 256; ++i) {
+                bv[i] = *p;
+                p += WHOLE || t4 + (i + 1) * 16 < kend ? step : 0;
+            }
+            if (WHOLE) return;
+            asm volatile("" : "+v"(t4));  // (compared anew: thirty-two masks are more than there are registers for)
+#pragma unroll
+            for (int it = 0; it < SK_KC / 64; ++it)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (it * 64 + lane >= kend) a[it][r] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < SK_KC * 16 / 256; ++i)
+                if (t4 + i * 16 >= kend) bv[i] = 0.0f;
+        };
+        if (kend == SK_KC) load(std::true_type{});
+        else load(std::false_type{});
         if (kc) __syncthreads();
 #pragma unroll
         for (int i = 0; i < SK_KC * 16 / 256; ++i) {
