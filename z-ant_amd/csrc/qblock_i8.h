@@ -9,10 +9,11 @@ struct QBlockArgs {
     int Co;                            // output channels (the rest of the last block is padding)
     int NB, TH, PH, PW, P, Ppad, Q;    // tile: images, output rows, patch rows / columns / positions, output positions
     int n_row_tiles, n_tiles;
-    int o_xl, o_e, o_w1, o_w2, o_wdw, o_tab, o_ptab;  // LDS byte offsets
+    int o_xl, o_e, o_w1, o_w2, o_wdw, o_tab, o_act, o_ptab;  // LDS byte offsets
     int packed_units;                  // 16-byte units of weights and tables: the LDS bytes from o_w1 to o_ptab
     int split;                         // stage D deals (position tile, channel chunk) units to the waves (few position tiles)
-    float zp1f, zp2f, zp3f;            // zero points of the three convolutions' own outputs
+    int zp1, zp2;                      // zero points of the three convolutions' own outputs
+    float zp3f;
     QAct act1, act2;
     int has_act1, has_act2;
     uint32_t pad_e4;                   // the depthwise input zero point ^ 0x80 in every byte
@@ -23,13 +24,33 @@ struct QBlockArgs {
     int ra_zp, rb_zp, ry_zp;
 };
 
+// The activation part of a block's tables: QB_ACT_HEAD bytes of QBlockActHead, then the two activation tables, each at an address of
+// its convolution's zero point's parity (quant_common.h).
+constexpr int QB_ACT_HEAD = 32, QB_ACT_TABLE = 272, QB_ACT_BYTES = QB_ACT_HEAD + 2 * QB_ACT_TABLE;
+struct QBlockActHead {
+    int lo1, hi1, lo2, hi2;  // the entries between which each table changes
+    int unused[4];
+};
+static_assert(sizeof(QBlockActHead) == QB_ACT_HEAD && QB_ACT_BYTES % 16 == 0 && QB_ACT_TABLE >= 257, "layout of the tables");
+
+#ifdef __HIPCC__
+__device__ __forceinline__ RequantLut qb_lut(const char *act, int table, int lo, int hi, int zp) {
+    const int base = int(lds_address(act)) + QB_ACT_HEAD + table * QB_ACT_TABLE + (zp & 1);
+    RequantLut t;
+    t.t0 = zq_as_float(unsigned(base + zp));
+    t.lo = zq_as_float(unsigned(base + lo));
+    t.hi = zq_as_float(unsigned(base + hi));
+    return t;
+}
+#endif
+
 // What a launch needs of one block: its kernel arguments, LDS bytes, instantiation and packed weights.
 struct QBlockPrep {
     QBlockArgs a;
     size_t lds_bytes;
     int CO32, MQv;
-    const uint4 *packed;  // weights, requantisation tables, then (see o_lut) what qblock_image_i8.hip wants beside them
-    int o_lut;            // bytes from `packed` to the two activation tables and the table of a whole image's patch positions
+    const uint4 *packed;  // weights, requantisation and activation tables, then (see o_img) what qblock_image_i8.hip wants beside them
+    int o_img;            // bytes from `packed` to the table of a whole image's patch positions
 };
 
 // Plans a block's tile, (re)packs its weights and tables into `slot` (or the context workspace) and fills the kernel

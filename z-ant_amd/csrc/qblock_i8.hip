@@ -35,36 +35,28 @@ __device__ __forceinline__ i32x4 as_i32x4(const uint4 &v) {
     return r;
 }
 
-// One block for the tiles of this workgroup; `lds` is the workgroup's dynamic LDS (256-byte aligned: the activation
-// tables need it).
+// One block for the tiles of this workgroup; `lds` is the workgroup's dynamic LDS.
 template <int CO32, int MQ, bool PF, bool SPLIT>
 __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t *__restrict__ y, const uint4 *__restrict__ packed,
                                             const QBlockArgs &a, char *lds) {
-    uint8_t *lut1 = reinterpret_cast<uint8_t *>(lds), *lut2 = lut1 + 256;
     uint4 *XL = reinterpret_cast<uint4 *>(lds + a.o_xl);   // [Cin32*2][Ppad] units of 16 channels
     uint4 *E = reinterpret_cast<uint4 *>(lds + a.o_e);     // [Ce32*2][Ppad]
     uint4 *W1 = reinterpret_cast<uint4 *>(lds + a.o_w1);   // [Cin32][Ce32][2][32] units
     uint4 *W2 = reinterpret_cast<uint4 *>(lds + a.o_w2);   // [Ce32][CO32][2][32] units
     uint32_t *WDW = reinterpret_cast<uint32_t *>(lds + a.o_wdw);  // [Ce/4][9][4] dwords
     const int Ce = a.Ce32 * 32;
-    float *m1 = reinterpret_cast<float *>(lds + a.o_tab);
-    int *c1 = reinterpret_cast<int *>(m1 + Ce);
-    float *m2 = reinterpret_cast<float *>(c1 + Ce);
-    int *c2 = reinterpret_cast<int *>(m2 + Ce);
-    float *m3 = reinterpret_cast<float *>(c2 + Ce);
-    int *c3 = reinterpret_cast<int *>(m3 + CO32 * 32);
+    const float *m1 = reinterpret_cast<const float *>(lds + a.o_tab);
+    const int *c1 = reinterpret_cast<const int *>(m1 + Ce);
+    const float *m2 = reinterpret_cast<const float *>(c1 + Ce);
+    const int *c2 = reinterpret_cast<const int *>(m2 + Ce);
+    const float *m3 = reinterpret_cast<const float *>(c2 + Ce);
+    const int *c3 = reinterpret_cast<const int *>(m3 + CO32 * 32);
     int *ptab = reinterpret_cast<int *>(lds + a.o_ptab);   // [Ppad] patch row; bit 31: a halo column or past the patch
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, lh = lane >> 5;
-    const unsigned lut1_a = lds_address(lut1), lut2_a = lds_address(lut2);
 
     // ---- once per workgroup: tables and weights into LDS ----
-    {
-        const uint8_t b = uint8_t(tid);
-        lut1[tid] = uint8_t((a.has_act1 ? qact_apply(b, a.act1) : b) ^ 0x80);
-        lut2[tid] = uint8_t((a.has_act2 ? qact_apply(b, a.act2) : b) ^ 0x80);
-    }
-    // weights and requantisation tables: `packed` holds them in the order and spacing of their LDS region, so they are
+    // `packed` holds them in the order and spacing of their LDS region, so they are
     // one copy, eight 16-byte units per thread in flight at a time.  The first eight are loaded here and written to LDS
     // behind the first tile's input patch, whose loads thereby travel with them.
     i32x4 *wdst = reinterpret_cast<i32x4 *>(lds + a.o_w1);
@@ -141,6 +133,9 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     }
     __syncthreads();
 
+    const QBlockActHead *head = reinterpret_cast<const QBlockActHead *>(lds + a.o_act);
+    const RequantLut lut1 = qb_lut(lds + a.o_act, 0, __builtin_amdgcn_readfirstlane(head->lo1), __builtin_amdgcn_readfirstlane(head->hi1), a.zp1);
+    const RequantLut lut2 = qb_lut(lds + a.o_act, 1, __builtin_amdgcn_readfirstlane(head->lo2), __builtin_amdgcn_readfirstlane(head->hi2), a.zp2);
     for (int tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
         const int ig = tile / a.n_row_tiles, rt = tile - ig * a.n_row_tiles;
         const int n0 = ig * a.NB, oh0 = rt * a.TH, ih0 = oh0 * a.stride - 1;
@@ -219,8 +214,8 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                     }
                     // a last block with at most 16 real channels: accumulator rows 16..31 (values 8..15) are padding
                     uint32_t d[NU][4];
-                    if (half) qb_requant_lookup_n<2, NU>(acc, mv, a.zp1f, lut1_a, d);
-                    else qb_requant_lookup_n<4, NU>(acc, mv, a.zp1f, lut1_a, d);
+                    if (half) qb_requant_lookup_n<2, NU>(acc, mv, lut1, d);
+                    else qb_requant_lookup_n<4, NU>(acc, mv, lut1, d);
 #pragma unroll
                     for (int j = 0; j < NU; ++j) {
                         // the half-wave swap leaves the lower lane with the 16 bytes of the first block of 16 channels and
@@ -340,8 +335,8 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                     }
                     if (j + 1 < MQ && !SPLIT) issue_taps(j + 1);
                     uint32_t d[4];
-                    if (half) qb_requant_lookup<2>(acc2, mv, a.zp2f, lut2_a, d);
-                    else qb_requant_lookup<4>(acc2, mv, a.zp2f, lut2_a, d);
+                    if (half) qb_requant_lookup<2>(acc2, mv, lut2, d);
+                    else qb_requant_lookup<4>(acc2, mv, lut2, d);
                     // lane (p, 0) gathers channels 0..15 of the chunk, lane (p, 1) channels 16..31
                     const auto s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
                     const auto s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
@@ -494,14 +489,33 @@ qblock_chain_kernel(QBlockChain c) {
     }
 }
 
-// A block's two activation tables and the table of patch positions of a whole image (row; bit 31: a halo column or past the patch),
-// for qblock_image_i8.hip.
-__global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, int P, uint8_t *out) {
+// A block's two activation tables with their windows, and the table of patch positions of a whole image (row; bit 31: a halo column or
+// past the patch) for qblock_image_i8.hip.
+__global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, int P, char *act, int *ptab) {
     const int tid = threadIdx.x;
+    __shared__ uint8_t lut[2][256];
+    __shared__ int win[4];  // lo1 hi1 lo2 hi2
     const uint8_t b = uint8_t(tid);
-    out[tid] = uint8_t((a.has_act1 ? qact_apply(b, a.act1) : b) ^ 0x80);
-    out[256 + tid] = uint8_t((a.has_act2 ? qact_apply(b, a.act2) : b) ^ 0x80);
-    int *ptab = reinterpret_cast<int *>(out + 512);
+    lut[0][tid] = uint8_t((a.has_act1 ? qact_apply(b, a.act1) : b) ^ 0x80);
+    lut[1][tid] = uint8_t((a.has_act2 ? qact_apply(b, a.act2) : b) ^ 0x80);
+    if (tid < 4) win[tid] = tid & 1 ? 0 : 255;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        // the last entry before the first change, the first one behind the last change
+        if (tid < 255 && lut[t][tid] != lut[t][tid + 1]) {
+            atomicMin(&win[2 * t], tid);
+            atomicMax(&win[2 * t + 1], tid + 1);
+        }
+        act[QB_ACT_HEAD + t * QB_ACT_TABLE + ((t ? a.zp2 : a.zp1) & 1) + tid] = char(lut[t][tid]);
+    }
+    __syncthreads();
+    if (tid == 0) {
+        QBlockActHead h = {0, 0, 0, 0, {0, 0, 0, 0}};  // (a constant table: its first entry)
+        if (win[0] < win[1]) { h.lo1 = win[0]; h.hi1 = win[1]; }
+        if (win[2] < win[3]) { h.lo2 = win[2]; h.hi2 = win[3]; }
+        *reinterpret_cast<QBlockActHead *>(act) = h;
+    }
     for (int p = tid; p < ((P + 31) & ~31); p += 256) {
         const int pp = min(p, P - 1), ph = pp / a.PW, pw = pp - ph * a.PW;
         ptab[p] = ph | ((p >= P || pw == 0 || pw == a.PW - 1) ? int(0x80000000u) : 0);
@@ -509,7 +523,6 @@ __global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, int P,
 }
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
-size_t align16(size_t v) { return (v + 15) & ~size_t(15); }
 
 bool conv1x1(const zant_qconv_desc *d) { return d && d->K > 0 && d->C > 0 && (d->n_wscale == 1 || d->n_wscale == d->K); }
 
@@ -547,7 +560,7 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
     const int64_t p_img = ((OH - 1) * dw_stride + 3) * a.PW;
     auto lds_for = [&](int64_t P) {
         const int64_t Ppad = (P + 31) & ~int64_t(31);
-        return size_t(512) + size_t(a.Cin32 * 2 + a.Ce32 * 2) * size_t(Ppad) * 16 + w1_bytes + w2_bytes + wdw_bytes + tab_bytes +
+        return size_t(QB_ACT_BYTES) + size_t(a.Cin32 * 2 + a.Ce32 * 2) * size_t(Ppad) * 16 + w1_bytes + w2_bytes + wdw_bytes + tab_bytes +
                size_t(Ppad) * 4;
     };
     auto tile_cost = [&](int64_t P, int64_t Q) {
@@ -610,13 +623,14 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         const int64_t n_tiles = ((N + bNB - 1) / bNB) * t.n_row_tiles;
         if (n_tiles > INT32_MAX || t.P >= (1 << 20) || t.Q >= (1 << 20)) continue;
         t.n_tiles = int(n_tiles);
-        size_t o = 512;
+        size_t o = 0;
         t.o_xl = int(o); o += size_t(t.Cin32) * 2 * t.Ppad * 16;
         t.o_e = int(o); o += size_t(t.Ce32) * 2 * t.Ppad * 16;
         t.o_w1 = int(o); o += w1_bytes;
         t.o_w2 = int(o); o += w2_bytes;
         t.o_wdw = int(o); o += wdw_bytes;
         t.o_tab = int(o); o += tab_bytes;
+        t.o_act = int(o); o += QB_ACT_BYTES;
         t.o_ptab = int(o); o += size_t(t.Ppad) * 4;
         if (o > cap) continue;
         a = t;
@@ -643,7 +657,7 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         out->CO32 = CO32;
         out->lds_bytes = cap_used;
     }
-    out->o_lut = int(align256(w1_bytes + w2_bytes + wdw_bytes + tab_bytes));
+    out->o_img = int(w1_bytes + w2_bytes + wdw_bytes + tab_bytes + QB_ACT_BYTES);
     if (plan_only) {
         out->a = a;
         out->packed = nullptr;
@@ -655,11 +669,11 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
     // packed weights and tables of the three convolutions
     const size_t kp1 = size_t(CeP), kp3 = size_t(CO32) * 32;
     // in the order and spacing of the kernel's LDS region [o_w1, o_ptab): weights of the expansion, of the projection, of
-    // the depthwise convolution, then the tables m1 c1 m2 c2 (CeP entries each) m3 c3 (kp3 entries each)
+    // the depthwise convolution, then the tables m1 c1 m2 c2 (CeP entries each) m3 c3 (kp3 entries each), the activations
     const size_t o_w1p = 256, o_w2p = o_w1p + w1_bytes, o_wm = o_w2p + w2_bytes, o_m1 = o_wm + wdw_bytes, o_c1 = o_m1 + kp1 * 4,
-                 o_m2 = o_c1 + kp1 * 4, o_c2 = o_m2 + kp1 * 4, o_m3 = o_c2 + kp1 * 4, o_c3 = o_m3 + kp3 * 4,
-                 o_tables = o_w1p + size_t(out->o_lut), static_bytes = align256(o_tables + 512 + size_t((p_img + 31) & ~int64_t(31)) * 4);
-    if (o_c3 + kp3 * 4 - o_w1p != w1_bytes + w2_bytes + wdw_bytes + tab_bytes || size_t(a.o_ptab - a.o_w1) != o_c3 + kp3 * 4 - o_w1p)
+                 o_m2 = o_c1 + kp1 * 4, o_c2 = o_m2 + kp1 * 4, o_m3 = o_c2 + kp1 * 4, o_c3 = o_m3 + kp3 * 4, o_actp = o_m1 + tab_bytes,
+                 o_imgp = o_w1p + size_t(out->o_img), static_bytes = align256(o_imgp + size_t((p_img + 31) & ~int64_t(31)) * 4);
+    if (o_c3 + kp3 * 4 != o_actp || size_t(a.o_ptab - a.o_w1) != size_t(out->o_img) || size_t(a.o_act - a.o_w1) + o_w1p != o_actp)
         return ZANT_InvalidInput;  // the two layouts must stay in step
     void *ws = nullptr, *dyn = nullptr;
     bool need_pack = true;
@@ -672,7 +686,7 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
     int32_t *c1 = reinterpret_cast<int32_t *>(base + o_c1), *c2 = reinterpret_cast<int32_t *>(base + o_c2),
             *c3 = reinterpret_cast<int32_t *>(base + o_c3);
     uint32_t *wmk = reinterpret_cast<uint32_t *>(base + o_wm);
-    a.zp1f = float(expand->y_zp); a.zp2f = float(dw->y_zp); a.zp3f = float(project->y_zp);
+    a.zp1 = expand->y_zp; a.zp2 = dw->y_zp; a.zp3f = float(project->y_zp);
     a.has_act1 = expand->act != ZANT_ACT_NONE;
     a.act1.act = expand->act; a.act1.alpha = expand->act_alpha; a.act1.in_scale = expand->y_scale; a.act1.in_zp = expand->y_zp;
     a.act1.out_scale = expand->act_scale; a.act1.out_zp = uint8_t(expand->act_zp);
@@ -699,7 +713,8 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         rc = zant_qpack_dense(ctx, project->w, project->w_scale, project->n_wscale, project->bias, int(Co), int(Ce), 1, 32,
                               project->x_scale, project->x_zp, project->y_scale, w2p, m3, c3, padvec + 16);
         if (rc) return rc;
-        hipLaunchKernelGGL(qblock_tables_kernel, dim3(1), dim3(256), 0, ctx->stream, a, int(p_img), reinterpret_cast<uint8_t *>(base + o_tables));
+        hipLaunchKernelGGL(qblock_tables_kernel, dim3(1), dim3(256), 0, ctx->stream, a, int(p_img), base + o_actp,
+                           reinterpret_cast<int *>(base + o_imgp));
         ZANT_LAUNCH_CHECK(ctx);
     }
 

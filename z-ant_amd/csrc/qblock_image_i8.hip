@@ -34,7 +34,6 @@ struct ImageLink {
     uint8_t *y;
     QBlockArgs a;
     int co32;      // blocks of 32 output channels
-    int o_lut;     // the two activation tables, behind the weights; the table of patch positions (a.o_ptab) follows them
     int o_r;       // projection sums: [32-position tile][32-channel block][accumulator register][lane]
     int late;      // LDS has no room for this block's weights while the block before it runs: they are loaded after it
 };
@@ -85,7 +84,9 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
     const int *c3 = reinterpret_cast<const int *>(m3 + co32 * 32);
     const int *ptab = reinterpret_cast<const int *>(lds + a.o_ptab);
     int *R = reinterpret_cast<int *>(lds + l.o_r);
-    const unsigned lut1_a = lds_address(lds + l.o_lut), lut2_a = lut1_a + 256;
+    const QBlockActHead *head = reinterpret_cast<const QBlockActHead *>(lds + a.o_act);
+    const RequantLut lut1 = qb_lut(lds + a.o_act, 0, __builtin_amdgcn_readfirstlane(head->lo1), __builtin_amdgcn_readfirstlane(head->hi1), a.zp1);
+    const RequantLut lut2 = qb_lut(lds + a.o_act, 1, __builtin_amdgcn_readfirstlane(head->lo2), __builtin_amdgcn_readfirstlane(head->hi2), a.zp2);
     const unsigned xl_a = lds_address(lds + a.o_xl), e_a = lds_address(lds + a.o_e);  // expanded patch: [Ce32*2][Ppad] units
     const int n_ptiles = a.Ppad >> 5, nq_tiles = (a.Q + 31) >> 5;
 
@@ -123,8 +124,8 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
                                                            as_i32x4(XL[(2 * chunk + lh) * a.Ppad + ptile * 32 + l32]), acc[0], 0, 0, 0);
         const bool half = a.half_last && kb == a.Ce32 - 1;  // at most 16 real channels: the upper half is padding
         uint32_t d[1][4];
-        if (half) qb_requant_lookup_n<2, 1>(acc, mv, a.zp1f, lut1_a, d);
-        else qb_requant_lookup_n<4, 1>(acc, mv, a.zp1f, lut1_a, d);
+        if (half) qb_requant_lookup_n<2, 1>(acc, mv, lut1, d);
+        else qb_requant_lookup_n<4, 1>(acc, mv, lut1, d);
         const auto s0 = __builtin_amdgcn_permlane32_swap(d[0][0], d[0][2], false, false);
         const auto s1 = __builtin_amdgcn_permlane32_swap(d[0][1], d[0][3], false, false);
         i32x4 out;
@@ -181,8 +182,8 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
                 acc2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa, tap[t], acc2, 0, 0, 0);
             }
             uint32_t d[4];
-            if (half) qb_requant_lookup<2>(acc2, mv, a.zp2f, lut2_a, d);
-            else qb_requant_lookup<4>(acc2, mv, a.zp2f, lut2_a, d);
+            if (half) qb_requant_lookup<2>(acc2, mv, lut2, d);
+            else qb_requant_lookup<4>(acc2, mv, lut2, d);
             const auto s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
             const auto s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
             i32x4 db;
@@ -336,7 +337,7 @@ size_t plan_lds(ImageChain &c) {
         const size_t xl = low ? 0 : total - n.xl, w = low ? n.xl : xl - n.w, e = low ? w + n.w : w - n.e, r = low ? e + n.e : e - n.r;
         const int move = int(w) - a.o_w1;  // (what lies behind the weights keeps its distance from them)
         a.o_xl = int(xl); a.o_e = int(e); l.o_r = int(r);
-        a.o_w1 += move; a.o_w2 += move; a.o_wdw += move; a.o_tab += move; l.o_lut += move; a.o_ptab += move;
+        a.o_w1 += move; a.o_w2 += move; a.o_wdw += move; a.o_tab += move; a.o_act += move; a.o_ptab += move;
     }
     return total;
 }
@@ -377,9 +378,8 @@ int zant_qblock_image_chain(zant_ctx *ctx, int n, const zant_qblock_call *calls,
         l.packed = prep.packed;
         l.y = k.y;
         l.a = prep.a;
-        l.o_lut = l.a.o_w1 + prep.o_lut;
-        l.a.o_ptab = l.o_lut + 512;
-        l.a.packed_units = (prep.o_lut + 512 + l.a.Ppad * 4) / 16;
+        l.a.o_ptab = l.a.o_w1 + prep.o_img;
+        l.a.packed_units = (prep.o_img + l.a.Ppad * 4) / 16;
         l.co32 = prep.CO32;
     }
     const size_t lds = plan_lds(c);
