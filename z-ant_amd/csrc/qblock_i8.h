@@ -5,12 +5,12 @@
 
 struct QBlockArgs {
     int N, H, W, OH, OW, stride;
-    int CBin, Cin32, Ce32, CBo;        // input channel blocks (16) / chunks (32); expanded chunks; output blocks
+    int CBin, Cin32, Ce32, CBe, CBo;   // input channel blocks (16) / chunks (32); expanded chunks / blocks; output blocks
     int Co;                            // output channels (the rest of the last block is padding)
     int NB, TH, PH, PW, P, Ppad, Q;    // tile: images, output rows, patch rows / columns / positions, output positions
     int n_row_tiles, n_tiles;
-    int o_xl, o_e, o_w1, o_w2, o_wdw, o_tab, o_act, o_ptab;  // LDS byte offsets
-    int packed_units;                  // 16-byte units of weights and tables: the LDS bytes from o_w1 to o_ptab
+    int o_xl, o_e, o_w1, o_w2, o_wdw, o_tab, o_act, o_ptab, o_qtab;  // LDS byte offsets
+    int packed_units;                  // 16-byte units of weights and tables: the LDS bytes from o_w1 to the end of the position tables
     int split;                         // stage D deals (position tile, channel chunk) units to the waves (few position tiles)
     int zp1, zp2;                      // zero points of the three convolutions' own outputs
     float zp3f;
@@ -31,6 +31,10 @@ struct QBlockActHead {
     int lo1, hi1, lo2, hi2;  // the entries between which each table changes
     int unused[4];
 };
+// The position tables.  Of a patch position (Ppad entries): x the patch row, bit 31 set for a halo column or past the patch; y the byte
+// offset of its first unit from that of the tile's first image, patch row 0, column 0.  Of an output position (Q rounded up to 32): x
+// the byte offset of its top-left tap in the patch, y that of its first output unit from the tile's first one.
+typedef int2 QBlockPos;
 static_assert(sizeof(QBlockActHead) == QB_ACT_HEAD && QB_ACT_BYTES % 16 == 0 && QB_ACT_TABLE >= 257, "layout of the tables");
 
 #ifdef __HIPCC__
@@ -49,8 +53,7 @@ struct QBlockPrep {
     QBlockArgs a;
     size_t lds_bytes;
     int CO32, MQv;
-    const uint4 *packed;  // weights, requantisation and activation tables, then (see o_img) what qblock_image_i8.hip wants beside them
-    int o_img;            // bytes from `packed` to the table of a whole image's patch positions
+    const uint4 *packed;  // weights, requantisation, activation and position tables
 };
 
 // Plans a block's tile, (re)packs its weights and tables into `slot` (or the context workspace) and fills the kernel

@@ -35,12 +35,31 @@ __device__ __forceinline__ i32x4 as_i32x4(const uint4 &v) {
     return r;
 }
 
+// Table entries of patch position p and output position q of a tile.
+__device__ __forceinline__ QBlockPos qb_patch_pos(const QBlockArgs &a, int p, float inv_patch_hw, float inv_pw) {
+    const int pp = min(p, a.P - 1), img = small_div(pp, a.PH * a.PW, inv_patch_hw), rem = pp - img * a.PH * a.PW;
+    const int ph = small_div(rem, a.PW, inv_pw), pw = rem - ph * a.PW;
+    QBlockPos e;
+    e.x = ph | (p >= a.P || pw == 0 || pw == a.PW - 1 ? int(0x80000000u) : 0);
+    e.y = ((img * a.CBin * a.H + ph) * a.W + pw - 1) * 16;
+    return e;
+}
+__device__ __forceinline__ QBlockPos qb_out_pos(const QBlockArgs &a, int q) {
+    const int qq = min(q, a.Q - 1), img = qq / (a.TH * a.OW), rem = qq - img * a.TH * a.OW, r = rem / a.OW, c = rem - r * a.OW;
+    QBlockPos e;
+    e.x = ((img * a.PH + r * a.stride) * a.PW + c * a.stride) * 16;
+    e.y = ((img * a.CBo * a.OH + r) * a.OW + c) * 16;
+    return e;
+}
+
 // One block for the tiles of this workgroup; `lds` is the workgroup's dynamic LDS.
 template <int CO32, int MQ, bool PF, bool SPLIT>
 __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t *__restrict__ y, const uint4 *__restrict__ packed,
                                             const QBlockArgs &a, char *lds) {
-    uint4 *XL = reinterpret_cast<uint4 *>(lds + a.o_xl);   // [Cin32*2][Ppad] units of 16 channels
-    uint4 *E = reinterpret_cast<uint4 *>(lds + a.o_e);     // [Ce32*2][Ppad]
+    // A chunk of 32 channels is two blocks of 16; where the last chunk has one block only, the lanes of its second half read the first
+    // one again: whatever integers they hold meet zero weights.
+    uint4 *XL = reinterpret_cast<uint4 *>(lds + a.o_xl);   // [CBin][Ppad] units of 16 channels
+    uint4 *E = reinterpret_cast<uint4 *>(lds + a.o_e);     // [CBe][Ppad]
     uint4 *W1 = reinterpret_cast<uint4 *>(lds + a.o_w1);   // [Cin32][Ce32][2][32] units
     uint4 *W2 = reinterpret_cast<uint4 *>(lds + a.o_w2);   // [Ce32][CO32][2][32] units
     uint32_t *WDW = reinterpret_cast<uint32_t *>(lds + a.o_wdw);  // [Ce/4][9][4] dwords
@@ -51,7 +70,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     const int *c2 = reinterpret_cast<const int *>(m2 + Ce);
     const float *m3 = reinterpret_cast<const float *>(c2 + Ce);
     const int *c3 = reinterpret_cast<const int *>(m3 + CO32 * 32);
-    int *ptab = reinterpret_cast<int *>(lds + a.o_ptab);   // [Ppad] patch row; bit 31: a halo column or past the patch
+    const QBlockPos *ptab = reinterpret_cast<const QBlockPos *>(lds + a.o_ptab), *qtab = reinterpret_cast<const QBlockPos *>(lds + a.o_qtab);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, lh = lane >> 5;
 
@@ -63,19 +82,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     i32x4 w0[8];
 #pragma unroll
     for (int r = 0; r < 8; ++r) w0[r] = *reinterpret_cast<const i32x4 *>(packed + min(r * 256 + tid, a.packed_units - 1));
-    {
-        const int patch = a.PH * a.PW;
-        const float inv_patch = 1.0f / float(patch), inv_pw = 1.0f / float(a.PW);
-        for (int p = tid; p < a.Ppad; p += 256) {
-            const int pp = min(p, a.P - 1);
-            const int img = small_div(pp, patch, inv_patch), rem = pp - img * patch;
-            const int ph = small_div(rem, a.PW, inv_pw), pw = rem - ph * a.PW;
-            ptab[p] = ph | ((p >= a.P || pw == 0 || pw == a.PW - 1) ? int(0x80000000u) : 0);
-        }
-    }
-
-    const float inv_p = 1.0f / float(a.P), inv_nptiles = 1.0f / float(a.Ppad >> 5);
-    const float inv_tile_img = 1.0f / float(a.TH * a.OW), inv_ow = 1.0f / float(a.OW);
+    const float inv_nptiles = 1.0f / float(a.Ppad >> 5);
     const int n_ptiles = a.Ppad >> 5, nq_tiles = (a.Q + 31) >> 5;
     // the diagonal element of row l32 lies in this lane's half of the columns; which dword of the 16-byte operand
     const bool diag_mine = (l32 >> 4) == lh;
@@ -87,39 +94,57 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     // first tile's patch is copied before the loop; every later one is loaded into registers before stage B of the tile
     // in front of it and written to LDS after that stage (the input patch is dead once B is done), so its global
     // latency passes under B.  Patches of more than QB_PF units per thread are copied in place instead. ----
+    // A round is 256 positions of one channel block.  The first tile's positions are taken apart by division, while the tables are on their
+    // way; every later tile's come from the table (8 instead of 60 vector instructions a unit, six of them quarter rate).
     constexpr int QB_PF = 4;
     const int patch_hw = a.PH * a.PW;
-    const float inv_patch_hw = 1.0f / float(patch_hw), inv_pw_ = 1.0f / float(a.PW);
-    const int a_units = a.CBin * a.P;
-    const bool prefetch = PF && a_units <= QB_PF * 256;  // PF is off for the instantiations without registers to spare
-    auto patch_unit = [&](int tile_, int u, int &dst) -> const uint4 * {  // source of unit u of a tile's patch, or null
-        const int ig_ = tile_ / a.n_row_tiles, rt_ = tile_ - ig_ * a.n_row_tiles;
-        const int cb = small_div(u, a.P, inv_p), p = u - cb * a.P;
-        const int img = small_div(p, patch_hw, inv_patch_hw), rem = p - img * patch_hw;   // (not from the position table: the
-        const int ph = small_div(rem, a.PW, inv_pw_), pw = rem - ph * a.PW;               // first patch is fetched before it exists)
-        const int n = ig_ * a.NB + img, ih = rt_ * a.TH * a.stride - 1 + ph, iw = pw - 1;
-        dst = cb * a.Ppad + p;
-        if (n < a.N && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W) return x + ((int64_t(n) * a.CBin + cb) * a.H + ih) * int64_t(a.W) + iw;
-        return nullptr;
+    const int p_rounds = (a.Ppad + 255) >> 8, a_rounds = a.CBin * p_rounds;
+    const bool prefetch = PF && a_rounds <= QB_PF;  // PF is off for the instantiations without registers to spare
+    const int64_t in_plane = int64_t(a.H) * a.W * 16;
+    struct Source { const char *base; int ih0, positions; unsigned valid; };  // `valid`: an offset that lies inside the tensor
+    auto source_of = [&](int tile_) {
+        const int ig_ = tile_ / a.n_row_tiles, rt_ = tile_ - ig_ * a.n_row_tiles, n_ = ig_ * a.NB;
+        Source s;
+        s.ih0 = rt_ * a.TH * a.stride - 1;
+        s.positions = a.n_row_tiles > 1 ? a.P : min(a.NB, a.N - n_) * patch_hw;
+        s.base = reinterpret_cast<const char *>(x) + (int64_t(n_) * a.CBin * a.H + s.ih0) * int64_t(a.W) * 16;
+        s.valid = s.ih0 < 0 ? unsigned(a.W) * 16u : 0u;
+        return s;
     };
-    auto copy_patch = [&](int tile_) {  // four loads in flight per thread, then their four LDS writes
-        for (int u0 = tid; u0 < a_units; u0 += 4 * 256) {
+    // every lane loads (from a place inside the tensor when it has nothing to fetch): no divergent branch around the load, so nothing
+    // waits for it before the values are written to LDS
+    auto fetch = [&](const Source &s, int cb, int p, const QBlockPos &e, i32x4 &v) {
+        const bool ok = p < s.positions && e.x >= 0 && unsigned(s.ih0 + (e.x & 0xffff)) < unsigned(a.H);
+        v = *reinterpret_cast<const i32x4 *>(s.base + cb * in_plane + (ok ? unsigned(e.y) : s.valid));
+        return ok;
+    };
+    auto copy_patch = [&](int tile_, auto entry) {  // four loads in flight per thread, then their four LDS writes
+        const Source s = source_of(tile_);
+        int cb = 0, pr = 0;
+        for (int r0 = 0; r0 < a_rounds; r0 += 4) {
             i32x4 v[4];  // (a native vector type: arrays of it are kept in registers)
             int dst[4];
             bool ok[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int u = min(u0 + r * 256, a_units - 1);
-                const uint4 *src = patch_unit(tile_, u, dst[r]);
-                ok[r] = src != nullptr && u0 + r * 256 < a_units;
-                v[r] = *reinterpret_cast<const i32x4 *>(ok[r] ? src : x);
+                const int p = pr * 256 + tid;
+                dst[r] = cb * a.Ppad + p;
+                ok[r] = false;
+                if (r0 + r < a_rounds) {
+                    ok[r] = fetch(s, cb, p, entry(p), v[r]);
+                    if (++pr == p_rounds) { pr = 0; ++cb; }
+                }
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 if (ok[r]) *reinterpret_cast<i32x4 *>(XL + dst[r]) = v[r];
         }
     };
-    if (int(blockIdx.x) < a.n_tiles) copy_patch(blockIdx.x);
+    if (int(blockIdx.x) < a.n_tiles) {
+        const float inv_patch_hw = 1.0f / float(patch_hw), inv_pw = 1.0f / float(a.PW);
+        copy_patch(blockIdx.x, [&](int p) { return qb_patch_pos(a, p, inv_patch_hw, inv_pw); });
+    }
+    auto from_table = [&](int p) { return ptab[min(p, a.Ppad - 1)]; };
 #pragma unroll
     for (int r = 0; r < 8; ++r)
         if (r * 256 + tid < a.packed_units) wdst[r * 256 + tid] = w0[r];
@@ -142,22 +167,17 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         const int next_tile = tile + int(gridDim.x);
         const bool has_next = next_tile < a.n_tiles;
         i32x4 nxt[QB_PF];
-        int nxt_dst[QB_PF];
         unsigned nxt_ok = 0;
         if (PF && prefetch && has_next) {
+            const Source s = source_of(next_tile);
+            int cb = 0, pr = 0;
 #pragma unroll
-            for (int r = 0; r < QB_PF; ++r) {
-                nxt_dst[r] = 0;
-                if (r * 256 < a_units) {
-                    // every lane loads (from the tensor's first unit when it has nothing to fetch): no divergent branch
-                    // around the load, so nothing waits for it before the values are written to LDS
-                    const int u = min(r * 256 + tid, a_units - 1);
-                    const uint4 *src = patch_unit(next_tile, u, nxt_dst[r]);
-                    const bool ok = src != nullptr && r * 256 + tid < a_units;
-                    nxt[r] = *reinterpret_cast<const i32x4 *>(ok ? src : x);
-                    nxt_ok |= ok ? 1u << r : 0u;
+            for (int r = 0; r < QB_PF; ++r)
+                if (r < a_rounds) {
+                    const int p = pr * 256 + tid;
+                    nxt_ok |= fetch(s, cb, p, from_table(p), nxt[r]) ? 1u << r : 0u;
+                    if (++pr == p_rounds) { pr = 0; ++cb; }
                 }
-            }
         }
 
         // ---- B: expansion.  A wave keeps one block of 32 expanded channels (its multipliers, corrections and, for one
@@ -183,7 +203,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                 const bool half = a.half_last && kb == a.Ce32 - 1;
                 // this lane's operand of input chunk 0 and the 16-byte unit it writes: lane (p, 0) the block of expanded
                 // channels 32 kb .. + 15 of its position, lane (p, 1) the block of channels 32 kb + 16 .. + 31
-                const unsigned x_addr = lds_address(XL) + unsigned(lh * a.Ppad + l32) * 16u;
+                const unsigned x_addr = lds_address(XL) + unsigned(min(lh, a.CBin - 1) * a.Ppad + l32) * 16u;
                 const unsigned e_addr = lds_address(E) + unsigned((2 * kb + lh) * a.Ppad + l32) * 16u;
                 // Two position tiles at a time (then a single one): the second tile's operand read, MFMA and table lookups
                 // travel under the first one's arithmetic.  A position of the depthwise convolution's padding -- a halo
@@ -193,7 +213,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                     bool padp[NU];
 #pragma unroll
                     for (int j = 0; j < NU; ++j) {
-                        const int e = ptab[(ptile + j) * 32 + l32];
+                        const int e = ptab[(ptile + j) * 32 + l32].x;
                         padp[j] = e < 0 || unsigned(ih0 + (e & 0xffff)) >= unsigned(a.H);
                     }
                     i32x4 xb[NU];
@@ -209,7 +229,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                         const i32x4 wc = as_i32x4(W1[(chunk * a.Ce32 + kb) * 64 + lh * 32 + l32]);
 #pragma unroll
                         for (int j = 0; j < NU; ++j)
-                            acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wc, as_i32x4(XL[(2 * chunk + lh) * a.Ppad + (ptile + j) * 32 + l32]),
+                            acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wc, as_i32x4(XL[min(2 * chunk + lh, a.CBin - 1) * a.Ppad + (ptile + j) * 32 + l32]),
                                                                            acc[j], 0, 0, 0);
                     }
                     // a last block with at most 16 real channels: accumulator rows 16..31 (values 8..15) are padding
@@ -242,11 +262,15 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         // ---- the next tile's input patch goes to LDS (the current one is dead; stage D reads the expanded patch only) ----
         if (has_next) {
             if (PF && prefetch) {
+                int cb = 0, pr = 0;
 #pragma unroll
                 for (int r = 0; r < QB_PF; ++r)
-                    if ((nxt_ok >> r) & 1u) *reinterpret_cast<i32x4 *>(XL + nxt_dst[r]) = nxt[r];
+                    if (r < a_rounds) {
+                        if ((nxt_ok >> r) & 1u) *reinterpret_cast<i32x4 *>(XL + cb * a.Ppad + pr * 256 + tid) = nxt[r];
+                        if (++pr == p_rounds) { pr = 0; ++cb; }
+                    }
             } else {
-                copy_patch(next_tile);
+                copy_patch(next_tile, from_table);
             }
         }
 
@@ -260,18 +284,40 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         const int q_end = SPLIT ? nq_tiles : min(nq_tiles, (wave + 1) * q_per_wave);
         const int n_units = nq_tiles * a.Ce32, u_begin = (n_units * wave) >> 2, u_end = (n_units * (wave + 1)) >> 2;
         for (int q0 = SPLIT ? 0 : wave * q_per_wave; q0 < q_end; q0 += MQ) {
-            int p0[MQ], qimg[MQ], qr[MQ], qc[MQ];
-            bool qvalid[MQ];
+            // an output position's top-left tap and its place in y, from the table.  Tiles of rows of one image end at the image's last
+            // row, tiles of images at the last image.
+            constexpr int SJ = SPLIT ? 1 : MQ;  // position tiles this wave stores: its own of those all waves share
+            int p0[MQ];
+            unsigned ybase[SJ];  // byte offset of this lane's four channels in block 0 of its position (the host checks that the
+            bool ok[SJ];         // blocked tensors stay below 2^31 bytes); a block of 16 channels further on is one plane further
+            auto place = [&](int tile_) { return qtab[min(tile_, nq_tiles - 1) * 32 + l32]; };
 #pragma unroll
-            for (int j = 0; j < MQ; ++j) {
-                const int q = (q0 + j) * 32 + l32;
-                qvalid[j] = q0 + j < q_end && q < a.Q;
-                const int qq = qvalid[j] ? q : 0;
-                qimg[j] = small_div(qq, a.TH * a.OW, inv_tile_img);
-                const int rem = qq - qimg[j] * a.TH * a.OW;
-                qr[j] = small_div(rem, a.OW, inv_ow);
-                qc[j] = rem - qr[j] * a.OW;
-                p0[j] = (qimg[j] * a.PH + qr[j] * a.stride) * a.PW + qc[j] * a.stride;  // top-left tap in the patch
+            for (int j = 0; j < MQ; ++j) p0[j] = place(q0 + j).x;
+            auto set_out = [&] {
+                const int q_valid = a.n_row_tiles > 1 ? min(a.TH, a.OH - oh0) * a.OW : min(a.NB, a.N - n0) * a.TH * a.OW;
+                const unsigned y_tile = ((unsigned(n0) * unsigned(a.CBo) * unsigned(a.OH) + unsigned(oh0)) * unsigned(a.OW)) * 16u;
+#pragma unroll
+                for (int j = 0; j < SJ; ++j) {
+                    const int qt = SPLIT ? wave : q0 + j;
+                    ok[j] = qt < q_end && qt * 32 + l32 < q_valid;
+                    ybase[j] = y_tile + unsigned(place(qt).y) + unsigned(lh) * 4u;
+                }
+            };
+            // The residual's bytes of every (tile, group), as one batch of loads; where registers allow, ahead of the chunks.
+            constexpr bool XR_EARLY = CO32 == 1 && MQ <= 3;
+            const unsigned plane16 = unsigned(a.OH * a.OW) * 16u;
+            uint32_t xr[SJ][CO32 * 4];
+            auto load_residual = [&] {
+#pragma unroll
+                for (int j = 0; j < SJ; ++j)
+#pragma unroll
+                    for (int g = 0; g < CO32 * 4; ++g)
+                        if (g * 8 < a.Co)
+                            xr[j][g] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(x) + (ok[j] ? ybase[j] + unsigned(g >> 1) * plane16 + unsigned(g & 1) * 8u : 0u));
+            };
+            if (XR_EARLY) {
+                set_out();
+                if (a.has_res) load_residual();
             }
             i32x16 acc3[MQ][CO32];
 #pragma unroll
@@ -305,16 +351,20 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                     const uint32_t wd = wk[t * 4];
                     wa[t][0] = int(wd & dm0); wa[t][1] = int(wd & dm1); wa[t][2] = int(wd & dm2); wa[t][3] = int(wd & dm3);
                 }
+                constexpr bool W2_KEPT = CO32 * MQ < 4;  // (no registers to keep two blocks' operands beside two tiles' sums)
                 i32x4 w2a[CO32];
+                auto load_w2 = [&] {
 #pragma unroll
-                for (int kb3 = 0; kb3 < CO32; ++kb3) w2a[kb3] = as_i32x4(W2[(ch * CO32 + kb3) * 64 + lh * 32 + l32]);
+                    for (int kb3 = 0; kb3 < CO32; ++kb3) w2a[kb3] = as_i32x4(W2[(ch * CO32 + kb3) * 64 + lh * 32 + l32]);
+                };
+                if (W2_KEPT) load_w2();
                 // The nine taps of a position tile are issued as one batch and consumed by the MFMAs as they arrive; the
                 // taps of the next tile are issued before this tile's requantisation, so they travel under its arithmetic.
-                const unsigned e_ch = lds_address(E) + unsigned((2 * ch + lh) * a.Ppad) * 16u;
+                const unsigned e_ch = lds_address(E) + unsigned(min(2 * ch + lh, a.CBe - 1) * a.Ppad) * 16u;
                 const unsigned row_b = unsigned(a.PW) * 16u;
                 i32x4 tap[9];
                 auto issue_taps = [&](int j) {
-                    const unsigned r0 = e_ch + unsigned(p0[j]) * 16u, r1 = r0 + row_b, r2 = r1 + row_b;
+                    const unsigned r0 = e_ch + unsigned(p0[j]), r1 = r0 + row_b, r2 = r1 + row_b;
                     qb_read128(tap[0], r0, 0); qb_read128(tap[1], r0, 16); qb_read128(tap[2], r0, 32);
                     qb_read128(tap[3], r1, 0); qb_read128(tap[4], r1, 16); qb_read128(tap[5], r1, 32);
                     qb_read128(tap[6], r2, 0); qb_read128(tap[7], r2, 16); qb_read128(tap[8], r2, 32);
@@ -342,6 +392,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                     const auto s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
                     i32x4 db;
                     db[0] = int(s0[0]); db[1] = int(s0[1]); db[2] = int(s1[0]); db[3] = int(s1[1]);
+                    if (!W2_KEPT) load_w2();
 #pragma unroll
                     for (int kb3 = 0; kb3 < CO32; ++kb3)
                         acc3[j][kb3] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w2a[kb3], db, acc3[j][kb3], 0, 0, 0);
@@ -363,41 +414,18 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                         for (int v = 0; v < 16; ++v) atomicAdd(R + ((j * CO32 + kb3) * 16 + v) * 64 + lane, acc3[j][kb3][v]);
                 }
                 __syncthreads();
-#pragma unroll
-                for (int j = 0; j < MQ; ++j) {
-                    if (j != wave) continue;
+                if (wave < nq_tiles) {
 #pragma unroll
                     for (int kb3 = 0; kb3 < CO32; ++kb3)
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            acc3[j][kb3][v] = R[((j * CO32 + kb3) * 16 + v) * 64 + lane] + c3[kb3 * 32 + lh * 4 + (v >> 2) * 8 + (v & 3)];
+                            acc3[0][kb3][v] = R[((wave * CO32 + kb3) * 16 + v) * 64 + lane] + c3[kb3 * 32 + lh * 4 + (v >> 2) * 8 + (v & 3)];
                 }
             }
+            if (!XR_EARLY) set_out();
             auto store_tiles = [&](auto res_tag, auto fast_tag) {
                 constexpr bool RES = decltype(res_tag)::value, FAST = decltype(fast_tag)::value;
-                // byte offset of this lane's four channels in block 0 of its position (the host checks that the blocked
-                // tensors stay below 2^31 bytes); a block of 16 channels further on is one plane further
-                unsigned ybase[MQ];
-                bool ok[MQ];
-                const unsigned plane16 = unsigned(a.OH * a.OW) * 16u;
-#pragma unroll
-                for (int j = 0; j < MQ; ++j) {
-                    const int n = n0 + qimg[j], oh = oh0 + qr[j];
-                    ok[j] = qvalid[j] && n < a.N && oh < a.OH && (!SPLIT || j == wave);
-                    ybase[j] = ((unsigned(n) * unsigned(a.CBo) * unsigned(a.OH) + unsigned(oh)) * unsigned(a.OW) + unsigned(qc[j])) * 16u + unsigned(lh) * 4u;
-                }
-                // the residual's bytes of every (tile, group) first, as one batch of loads
-                uint32_t xr[MQ][CO32 * 4];
-                if (RES) {
-#pragma unroll
-                    for (int j = 0; j < MQ; ++j)
-#pragma unroll
-                        for (int g = 0; g < CO32 * 4; ++g) {
-                            xr[j][g] = 0;
-                            if (ok[j] && g * 8 < a.Co)
-                                xr[j][g] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(x) + (ybase[j] + unsigned(g >> 1) * plane16 + unsigned(g & 1) * 8u));
-                        }
-                }
+                if (RES && !XR_EARLY) load_residual();
 #pragma unroll
                 for (int kb3 = 0; kb3 < CO32; ++kb3) {
 #pragma unroll
@@ -409,7 +437,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                         // layout (no kernel reads it against a non-zero weight): no arithmetic, zeros stored
                         if (kb3 * 32 + gq * 8 >= a.Co) {
 #pragma unroll
-                            for (int j = 0; j < MQ; ++j)
+                            for (int j = 0; j < SJ; ++j)
                                 if (ok[j]) *reinterpret_cast<uint32_t *>(y + (ybase[j] + goff)) = 0u;
                             continue;
                         }
@@ -417,7 +445,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
 #pragma unroll
                         for (int e = 0; e < 4; ++e) mq[e] = m3[kb3 * 32 + gq * 8 + lh * 4 + e];
 #pragma unroll
-                        for (int j = 0; j < MQ; ++j) {
+                        for (int j = 0; j < SJ; ++j) {
                             uint32_t o = 0;
 #pragma unroll
                             for (int e = 0; e < 4; ++e) {
@@ -489,9 +517,8 @@ qblock_chain_kernel(QBlockChain c) {
     }
 }
 
-// A block's two activation tables with their windows, and the table of patch positions of a whole image (row; bit 31: a halo column or
-// past the patch) for qblock_image_i8.hip.
-__global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, int P, char *act, int *ptab) {
+// A block's two activation tables with their windows, and the position tables of its tiles.
+__global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, char *act, QBlockPos *ptab, QBlockPos *qtab) {
     const int tid = threadIdx.x;
     __shared__ uint8_t lut[2][256];
     __shared__ int win[4];  // lo1 hi1 lo2 hi2
@@ -516,10 +543,9 @@ __global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, int P,
         if (win[2] < win[3]) { h.lo2 = win[2]; h.hi2 = win[3]; }
         *reinterpret_cast<QBlockActHead *>(act) = h;
     }
-    for (int p = tid; p < ((P + 31) & ~31); p += 256) {
-        const int pp = min(p, P - 1), ph = pp / a.PW, pw = pp - ph * a.PW;
-        ptab[p] = ph | ((p >= P || pw == 0 || pw == a.PW - 1) ? int(0x80000000u) : 0);
-    }
+    const float inv_patch_hw = 1.0f / float(a.PH * a.PW), inv_pw = 1.0f / float(a.PW);
+    for (int p = tid; p < a.Ppad; p += 256) ptab[p] = qb_patch_pos(a, p, inv_patch_hw, inv_pw);
+    for (int q = tid; q < ((a.Q + 31) & ~31); q += 256) qtab[q] = qb_out_pos(a, q);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -545,7 +571,7 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
 
     QBlockArgs a;
     a.N = int(N); a.H = int(H); a.W = int(W); a.OH = int(OH); a.OW = int(OW); a.stride = int(dw_stride);
-    a.CBin = int((Cin + 15) / 16); a.Cin32 = int((Cin + 31) / 32); a.Ce32 = int((Ce + 31) / 32); a.CBo = int((Co + 15) / 16); a.Co = int(Co);
+    a.CBin = int((Cin + 15) / 16); a.Cin32 = int((Cin + 31) / 32); a.Ce32 = int((Ce + 31) / 32); a.CBe = int((Ce + 15) / 16); a.CBo = int((Co + 15) / 16); a.Co = int(Co);
     const int CO32 = int((Co + 31) / 32), CeP = a.Ce32 * 32;
     a.PW = int(W) + 2;
     // LDS: fixed part, then per patch position the input and expanded bytes and one table entry
@@ -558,10 +584,10 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
     // positions, MQ at a time per wave; partly filled units and the halo rows cost as much as full ones.
     const int mq_cap = CO32 == 1 ? 4 : CO32 == 2 ? 2 : 1;
     const int64_t p_img = ((OH - 1) * dw_stride + 3) * a.PW;
-    auto lds_for = [&](int64_t P) {
-        const int64_t Ppad = (P + 31) & ~int64_t(31);
-        return size_t(QB_ACT_BYTES) + size_t(a.Cin32 * 2 + a.Ce32 * 2) * size_t(Ppad) * 16 + w1_bytes + w2_bytes + wdw_bytes + tab_bytes +
-               size_t(Ppad) * 4;
+    auto lds_for = [&](int64_t P, int64_t Q) {
+        const int64_t Ppad = (P + 31) & ~int64_t(31), Qpad = (Q + 31) & ~int64_t(31);
+        return size_t(QB_ACT_BYTES) + size_t(a.CBin + a.CBe) * size_t(Ppad) * 16 + w1_bytes + w2_bytes + wdw_bytes + tab_bytes +
+               size_t(Ppad + Qpad) * sizeof(QBlockPos);
     };
     auto tile_cost = [&](int64_t P, int64_t Q) {
         const int64_t b_units = int64_t(a.Ce32) * ((P + 31) / 32), nq = (Q + 31) / 32, qpw = (nq + 3) / 4;
@@ -591,17 +617,19 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         const int64_t slots = int64_t(ctx->num_cus) * (two ? 2 : 1);
         double best = 0.0;
         int bNB = 0, bTH = 0;
-        if (lds_for(p_img) <= cap) {
-            for (int64_t nb = 1; nb <= std::min<int64_t>(N, 2047) && lds_for(nb * p_img) <= cap; ++nb) {
+        if (lds_for(p_img, OH * OW) <= cap) {
+            for (int64_t nb = 1; nb <= std::min<int64_t>(N, 2047) && lds_for(nb * p_img, nb * OH * OW) <= cap; ++nb) {
                 if (force_nb > 0 && nb != force_nb) continue;
                 const int64_t tiles = (N + nb - 1) / nb, waves = (tiles + slots - 1) / slots;
                 const double c = tile_cost(nb * p_img, nb * OH * OW) * double(waves);  // time of the busiest workgroup slot
                 if (!bNB || c < best * 0.98) { best = c; bNB = int(nb); bTH = int(OH); }
             }
-        } else if (force_nb <= 0) {
-            for (int64_t th = 1; th <= OH; ++th) {
+        }
+        // rows of an image where a whole one does not fit, or where there are fewer images than CUs (one image of 24x24: 15.5 us whole, 6.6 in rows)
+        if (force_nb <= 0 && (!bNB || N < ctx->num_cus)) {
+            for (int64_t th = 1; th < OH || (th == OH && !bNB); ++th) {
                 const int64_t P = ((th - 1) * dw_stride + 3) * a.PW;
-                if (lds_for(P) > cap) break;
+                if (lds_for(P, th * OW) > cap) break;
                 const int64_t nrt = (OH + th - 1) / th;
                 if ((OH + nrt - 1) / nrt != th) continue;  // only evened-out row tiles
                 const int64_t tiles = N * nrt, waves = (tiles + slots - 1) / slots;
@@ -624,14 +652,15 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         if (n_tiles > INT32_MAX || t.P >= (1 << 20) || t.Q >= (1 << 20)) continue;
         t.n_tiles = int(n_tiles);
         size_t o = 0;
-        t.o_xl = int(o); o += size_t(t.Cin32) * 2 * t.Ppad * 16;
-        t.o_e = int(o); o += size_t(t.Ce32) * 2 * t.Ppad * 16;
+        t.o_xl = int(o); o += size_t(t.CBin) * t.Ppad * 16;
+        t.o_e = int(o); o += size_t(t.CBe) * t.Ppad * 16;
         t.o_w1 = int(o); o += w1_bytes;
         t.o_w2 = int(o); o += w2_bytes;
         t.o_wdw = int(o); o += wdw_bytes;
         t.o_tab = int(o); o += tab_bytes;
         t.o_act = int(o); o += QB_ACT_BYTES;
-        t.o_ptab = int(o); o += size_t(t.Ppad) * 4;
+        t.o_ptab = int(o); o += size_t(t.Ppad) * sizeof(QBlockPos);
+        t.o_qtab = int(o); o += size_t((t.Q + 31) & ~31) * sizeof(QBlockPos);
         if (o > cap) continue;
         a = t;
         cap_used = o;
@@ -652,12 +681,12 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         const int rounds = (q_per_wave + mq_cap - 1) / mq_cap;
         // fewer position tiles than waves: the waves share them chunk by chunk (their sums meet in the expanded patch's LDS)
         a.split = CO32 <= 2 && nq_tiles < 4 && nq_tiles <= mq_cap && a.Ce32 >= 2 &&
-                  size_t(nq_tiles) * CO32 * 4096 <= size_t(a.Ce32) * 2 * a.Ppad * 16;
+                  size_t(nq_tiles) * CO32 * 4096 <= size_t(a.CBe) * a.Ppad * 16;
         out->MQv = a.split ? nq_tiles : std::max(1, (q_per_wave + rounds - 1) / rounds);
         out->CO32 = CO32;
         out->lds_bytes = cap_used;
     }
-    out->o_img = int(w1_bytes + w2_bytes + wdw_bytes + tab_bytes + QB_ACT_BYTES);
+    a.packed_units = (a.o_qtab - a.o_w1 + ((a.Q + 31) & ~31) * int(sizeof(QBlockPos))) / 16;
     if (plan_only) {
         out->a = a;
         out->packed = nullptr;
@@ -668,17 +697,20 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
 
     // packed weights and tables of the three convolutions
     const size_t kp1 = size_t(CeP), kp3 = size_t(CO32) * 32;
-    // in the order and spacing of the kernel's LDS region [o_w1, o_ptab): weights of the expansion, of the projection, of
-    // the depthwise convolution, then the tables m1 c1 m2 c2 (CeP entries each) m3 c3 (kp3 entries each), the activations
+    // in the order and spacing of the kernel's LDS region from o_w1 on: weights of the expansion, of the projection, of
+    // the depthwise convolution, then the tables m1 c1 m2 c2 (CeP entries each) m3 c3 (kp3 entries each), the
+    // activations, the position tables
     const size_t o_w1p = 256, o_w2p = o_w1p + w1_bytes, o_wm = o_w2p + w2_bytes, o_m1 = o_wm + wdw_bytes, o_c1 = o_m1 + kp1 * 4,
                  o_m2 = o_c1 + kp1 * 4, o_c2 = o_m2 + kp1 * 4, o_m3 = o_c2 + kp1 * 4, o_c3 = o_m3 + kp3 * 4, o_actp = o_m1 + tab_bytes,
-                 o_imgp = o_w1p + size_t(out->o_img), static_bytes = align256(o_imgp + size_t((p_img + 31) & ~int64_t(31)) * 4);
-    if (o_c3 + kp3 * 4 != o_actp || size_t(a.o_ptab - a.o_w1) != size_t(out->o_img) || size_t(a.o_act - a.o_w1) + o_w1p != o_actp)
+                 o_ptabp = o_actp + QB_ACT_BYTES, o_qtabp = o_ptabp + size_t(a.Ppad) * sizeof(QBlockPos),
+                 end = o_qtabp + size_t((a.Q + 31) & ~31) * sizeof(QBlockPos), static_bytes = align256(end);
+    if (o_c3 + kp3 * 4 != o_actp || size_t(a.o_act - a.o_w1) + o_w1p != o_actp || size_t(a.o_qtab - a.o_w1) + o_w1p != o_qtabp || size_t(a.packed_units) * 16 != end - o_w1p)
         return ZANT_InvalidInput;  // the two layouts must stay in step
     void *ws = nullptr, *dyn = nullptr;
     bool need_pack = true;
     int rc = zant_pack_region(ctx, slot, static_bytes, 0, &ws, &dyn, &need_pack);
     if (rc) return rc;
+    need_pack = need_pack || !cached;  // (the position tables are the tiling's)
     char *base = static_cast<char *>(ws);
     int8_t *w1p = reinterpret_cast<int8_t *>(base + o_w1p), *w2p = reinterpret_cast<int8_t *>(base + o_w2p);
     float *m1 = reinterpret_cast<float *>(base + o_m1), *m2 = reinterpret_cast<float *>(base + o_m2),
@@ -713,12 +745,12 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         rc = zant_qpack_dense(ctx, project->w, project->w_scale, project->n_wscale, project->bias, int(Co), int(Ce), 1, 32,
                               project->x_scale, project->x_zp, project->y_scale, w2p, m3, c3, padvec + 16);
         if (rc) return rc;
-        hipLaunchKernelGGL(qblock_tables_kernel, dim3(1), dim3(256), 0, ctx->stream, a, int(p_img), base + o_actp,
-                           reinterpret_cast<int *>(base + o_imgp));
+        hipLaunchKernelGGL(qblock_tables_kernel, dim3(1), dim3(256), 0, ctx->stream, a, base + o_actp,
+                           reinterpret_cast<QBlockPos *>(base + o_ptabp), reinterpret_cast<QBlockPos *>(base + o_qtabp));
         ZANT_LAUNCH_CHECK(ctx);
     }
 
-    a.packed_units = int((a.o_ptab - a.o_w1) / 16);
+
     out->a = a;
     out->packed = reinterpret_cast<const uint4 *>(base + o_w1p);
     return ZANT_OK;
@@ -748,7 +780,7 @@ int zant_qblock_blocked(zant_ctx *ctx, const uint8_t *x, const int64_t xdim[4], 
     switch ((a.split ? 100 : 0) + CO32 * 10 + MQv) {
     case 11: ZANT_QBLOCK_LAUNCH(1, 1, true, false); break;
     case 12: ZANT_QBLOCK_LAUNCH(1, 2, true, false); break;
-    case 13: ZANT_QBLOCK_LAUNCH(1, 3, false, false); break;
+    case 13: ZANT_QBLOCK_LAUNCH(1, 3, true, false); break;
     case 14: ZANT_QBLOCK_LAUNCH(1, 4, false, false); break;
     case 21: ZANT_QBLOCK_LAUNCH(2, 1, true, false); break;
     case 22: ZANT_QBLOCK_LAUNCH(2, 2, false, false); break;

@@ -82,7 +82,7 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
     const int *c2 = reinterpret_cast<const int *>(m2 + Ce);
     const float *m3 = reinterpret_cast<const float *>(c2 + Ce);
     const int *c3 = reinterpret_cast<const int *>(m3 + co32 * 32);
-    const int *ptab = reinterpret_cast<const int *>(lds + a.o_ptab);
+    const QBlockPos *ptab = reinterpret_cast<const QBlockPos *>(lds + a.o_ptab), *qtab = reinterpret_cast<const QBlockPos *>(lds + a.o_qtab);
     int *R = reinterpret_cast<int *>(lds + l.o_r);
     const QBlockActHead *head = reinterpret_cast<const QBlockActHead *>(lds + a.o_act);
     const RequantLut lut1 = qb_lut(lds + a.o_act, 0, __builtin_amdgcn_readfirstlane(head->lo1), __builtin_amdgcn_readfirstlane(head->hi1), a.zp1);
@@ -107,7 +107,7 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
         i32x4 xb;
         qb_read128(xb, xl_a + unsigned(lh * a.Ppad + ptile * 32 + l32) * 16u, 0);
         const i32x4 wa0 = as_i32x4(W1[kb * 64 + lh * 32 + l32]);
-        const int e = ptab[ptile * 32 + l32];
+        const int e = ptab[ptile * 32 + l32].x;
         i32x16 acc[1];
         float mv[16];
 #pragma unroll
@@ -151,13 +151,12 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
         const uint32_t dm0 = diag_mine && diag_q == 0 ? 0xffffffffu : 0u, dm1 = diag_mine && diag_q == 1 ? 0xffffffffu : 0u,
                        dm2 = diag_mine && diag_q == 2 ? 0xffffffffu : 0u, dm3 = diag_mine && diag_q == 3 ? 0xffffffffu : 0u;
         const int d_units = nq_tiles * a.Ce32;
-        const float inv_ce = 1.0f / float(a.Ce32), inv_ow = 1.0f / float(a.OW);
+        const float inv_ce = 1.0f / float(a.Ce32);
         const unsigned row_b = unsigned(a.PW) * 16u;
         for (int u = wave; u < d_units; u += kWaves) {
             const int j = small_div(u, a.Ce32, inv_ce), ch = u - j * a.Ce32, kch = ch * 32 + lh * 4;
-            const int qq = min(j * 32 + l32, a.Q - 1), qr = small_div(qq, a.OW, inv_ow), qc = qq - qr * a.OW;
             const bool half = a.half_last && ch == a.Ce32 - 1;
-            const unsigned r0 = e_a + unsigned((2 * ch + lh) * a.Ppad + qr * a.stride * a.PW + qc * a.stride) * 16u,  // top-left tap
+            const unsigned r0 = e_a + unsigned((2 * ch + lh) * a.Ppad) * 16u + unsigned(qtab[j * 32 + l32].x),  // top-left tap
                            r1 = r0 + row_b, r2 = r1 + row_b;
             const uint32_t *wk = WDW + ((ch * 32 + l32) >> 2) * 36 + (l32 & 3);
             uint32_t wd[9];
@@ -337,7 +336,7 @@ size_t plan_lds(ImageChain &c) {
         const size_t xl = low ? 0 : total - n.xl, w = low ? n.xl : xl - n.w, e = low ? w + n.w : w - n.e, r = low ? e + n.e : e - n.r;
         const int move = int(w) - a.o_w1;  // (what lies behind the weights keeps its distance from them)
         a.o_xl = int(xl); a.o_e = int(e); l.o_r = int(r);
-        a.o_w1 += move; a.o_w2 += move; a.o_wdw += move; a.o_tab += move; a.o_act += move; a.o_ptab += move;
+        a.o_w1 += move; a.o_w2 += move; a.o_wdw += move; a.o_tab += move; a.o_act += move; a.o_ptab += move; a.o_qtab += move;
     }
     return total;
 }
@@ -378,8 +377,6 @@ int zant_qblock_image_chain(zant_ctx *ctx, int n, const zant_qblock_call *calls,
         l.packed = prep.packed;
         l.y = k.y;
         l.a = prep.a;
-        l.a.o_ptab = l.a.o_w1 + prep.o_img;
-        l.a.packed_units = (prep.o_img + l.a.Ppad * 4) / 16;
         l.co32 = prep.CO32;
     }
     const size_t lds = plan_lds(c);

@@ -171,7 +171,8 @@ __device__ __forceinline__ void qb_requant_lookup_n(const zq_i32x16 (&acc)[NU], 
         if (G > 2) qb_ready8(b[j] + 8);
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-            d[j][g] = g < G ? (b[j][4 * g] | (b[j][4 * g + 1] << 8) | (b[j][4 * g + 2] << 16) | (b[j][4 * g + 3] << 24)) : 0u;
+            d[j][g] = g < G ? __builtin_amdgcn_perm(b[j][4 * g + 1], b[j][4 * g], 0x0c0c0400u) |  // (0x0c: a zero byte)
+                                  __builtin_amdgcn_perm(b[j][4 * g + 3], b[j][4 * g + 2], 0x04000c0cu) : 0u;
     }
 }
 template <int G>
