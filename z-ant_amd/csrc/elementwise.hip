@@ -32,6 +32,7 @@ __global__ void __launch_bounds__(kThreads) unary_f32_kernel(const float *__rest
                                                             int64_t n, float slope) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     const int64_t n4 = n >> 2;
+    const bool kept = zant_out_kept(n * 4);
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
     f4 *y4 = reinterpret_cast<f4 *>(y);
@@ -50,7 +51,7 @@ __global__ void __launch_bounds__(kThreads) unary_f32_kernel(const float *__rest
             r.y = unary_op<OP>(v[u].y, slope);
             r.z = unary_op<OP>(v[u].z, slope);
             r.w = unary_op<OP>(v[u].w, slope);
-            __builtin_nontemporal_store(r, y4 + j);
+            zant_store_out(r, y4 + j, kept);
         }
     }
     if (blockIdx.x == 0) {  // the 0..3 elements behind the last full vector
@@ -140,6 +141,7 @@ __global__ void __launch_bounds__(kThreads) softmax_small_f32_kernel(const float
     typedef float f4 __attribute__((ext_vector_type(4)));
     __shared__ __attribute__((aligned(16))) float buf[2][kThreads * 16];
     const int64_t n_chunks = (rows + kThreads - 1) / kThreads;
+    const bool kept = zant_out_kept(rows * cols * 4);
     f4 pre[kSoftmaxVecs];
     // a chunk's vectors into registers (vec: spans start on 16-byte boundaries; otherwise the scalar path below)
     auto fetch = [&](int64_t chunk) {
@@ -196,7 +198,7 @@ __global__ void __launch_bounds__(kThreads) softmax_small_f32_kernel(const float
 #pragma unroll
         for (int u = 0; u < kSoftmaxVecs; ++u) {
             const int i = u * kThreads + int(threadIdx.x);
-            if (i < nvec) __builtin_nontemporal_store(reinterpret_cast<const f4 *>(b)[i], reinterpret_cast<f4 *>(yb) + i);
+            if (i < nvec) zant_store_out(reinterpret_cast<const f4 *>(b)[i], reinterpret_cast<f4 *>(yb) + i, kept);
         }
         for (int i = (nvec << 2) + threadIdx.x; i < nel; i += kThreads) yb[i] = b[i];
     }
@@ -216,6 +218,7 @@ __global__ void __launch_bounds__(kThreads) add_same_f32_kernel(const float *__r
         return;
     }
     const int64_t n4 = n >> 2;
+    const bool kept = zant_out_kept(n * 4);
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     const f4 *a4 = reinterpret_cast<const f4 *>(a);
     const f4 *b4 = reinterpret_cast<const f4 *>(b);
@@ -229,7 +232,7 @@ __global__ void __launch_bounds__(kThreads) add_same_f32_kernel(const float *__r
 #pragma unroll
     for (int u = 0; u < ZANT_STREAM_U; ++u) {
         const int64_t j = base + u * kThreads;
-        if (j < n4) __builtin_nontemporal_store(va[u] + vb[u], y4 + j);
+        if (j < n4) zant_store_out(va[u] + vb[u], y4 + j, kept);
     }
     if (blockIdx.x == 0) {
         const int64_t j = (n4 << 2) + threadIdx.x;
@@ -264,6 +267,7 @@ __global__ void __launch_bounds__(kThreads) add_bcast_f32_kernel(const float *__
 __global__ void __launch_bounds__(kThreads) add_channel_f32_kernel(const float *__restrict__ big, const float *__restrict__ small,
                                                                   float *__restrict__ y, uint32_t n4, uint32_t inner4, uint32_t C) {
     typedef float f4 __attribute__((ext_vector_type(4)));
+    const bool kept = zant_out_kept(int64_t(n4) * 16);
     const uint32_t base = blockIdx.x * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     const f4 *b4 = reinterpret_cast<const f4 *>(big);
     f4 *y4 = reinterpret_cast<f4 *>(y);
@@ -280,7 +284,7 @@ __global__ void __launch_bounds__(kThreads) add_channel_f32_kernel(const float *
 #pragma unroll
     for (int u = 0; u < ZANT_STREAM_U; ++u) {
         const uint32_t j = base + u * kThreads;
-        if (j < n4) __builtin_nontemporal_store(v[u] + c[u], y4 + j);
+        if (j < n4) zant_store_out(v[u] + c[u], y4 + j, kept);
     }
 }
 
@@ -372,6 +376,7 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T 
     typedef unsigned u2 __attribute__((ext_vector_type(2)));
     typedef float f2 __attribute__((ext_vector_type(2)));
     constexpr bool F32 = sizeof(T) == 4;
+    const bool kept = zant_out_kept(total_vec * int64_t(VEC * sizeof(T)));
     static_assert(!(ANY && F32), "f32 rows of odd lengths are no faster this way than element by element");
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     // flat row index of the first vector of this workgroup, then block-local arithmetic in 32 bits
@@ -419,7 +424,7 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T 
         if (F32) {
             const float m = fmaxf(fmaxf(__uint_as_float(r0[u][0]), __uint_as_float(r0[u][1])),
                                   fmaxf(__uint_as_float(r1[u][0]), __uint_as_float(r1[u][1])));
-            __builtin_nontemporal_store(m, reinterpret_cast<float *>(y) + dst[u]);
+            zant_store_out(m, reinterpret_cast<float *>(y) + dst[u], kept);
         } else {
             // bytes as 16-bit lanes (even bytes and odd bytes of a dword apart): the vertical maximum is one packed
             // 16-bit max per half, the horizontal one (bytes 0|1 and 2|3) the packed max of the two halves, and one byte
@@ -441,7 +446,7 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_stream_kernel(const T 
             uint8_t *out = reinterpret_cast<uint8_t *>(y) + dst[u];
             if constexpr (ANY && VEC == 4) *reinterpret_cast<u1_any *>(out) = o[0];
             else if constexpr (ANY) *reinterpret_cast<u2_any *>(out) = o;
-            else __builtin_nontemporal_store(o, reinterpret_cast<u2 *>(out));
+            else zant_store_out(o, reinterpret_cast<u2 *>(out), kept);
         }
     }
 }
@@ -462,6 +467,7 @@ __global__ void __launch_bounds__(kThreads) pool_2x2s2_planes_f32_kernel(const f
     const int64_t p0 = int64_t(blockIdx.x) * G;
     const int planes = int(min<int64_t>(G, NC - p0));
     const int HW = H * W, OHW = OH * OW;
+    const bool kept = zant_out_kept(NC * OHW * 4);
     const int n_in = planes * HW, n_out = planes * OHW;  // n_in is a multiple of 4 unless this is the tensor's tail
     const float *src = x + p0 * HW;
     const int n_in4 = n_in >> 2;
@@ -499,7 +505,7 @@ __global__ void __launch_bounds__(kThreads) pool_2x2s2_planes_f32_kernel(const f
         f4 o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = one(4 * i + e);
-        __builtin_nontemporal_store(o, reinterpret_cast<f4 *>(dst) + i);
+        zant_store_out(o, reinterpret_cast<f4 *>(dst) + i, kept);
     }
     for (int o = (n_out4 << 2) + int(threadIdx.x); o < n_out; o += kThreads) dst[o] = one(o);
 }
@@ -516,6 +522,7 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_planes_u8_kernel(const
     const int64_t p0 = int64_t(blockIdx.x) * G;
     const int planes = int(min<int64_t>(G, NC - p0));
     const int HW = H * W, OHW = OH * OW;
+    const bool kept = zant_out_kept(NC * OHW);
     const int n_in16 = planes * HW / 16, n_out16 = planes * OHW / 16;
     const u4 *src = reinterpret_cast<const u4 *>(x + p0 * HW);
     constexpr int B = kPoolLdsFloats / 4 / kThreads;
@@ -554,7 +561,7 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_planes_u8_kernel(const
             o[2 * h] = __builtin_amdgcn_perm(window_max(a[1], b[1]), window_max(a[0], b[0]), 0x06040200u);
             o[2 * h + 1] = __builtin_amdgcn_perm(window_max(a[3], b[3]), window_max(a[2], b[2]), 0x06040200u);
         }
-        __builtin_nontemporal_store(o, dst + i);
+        zant_store_out(o, dst + i, kept);
     }
 }
 
@@ -734,6 +741,7 @@ __global__ void __launch_bounds__(kThreads) batchnorm_vec_f32_kernel(const float
                                                                      float eps, int64_t total4, uint32_t inner4, uint32_t features) {
     // the streaming pattern: a workgroup's ZANT_STREAM_U x 256 vectors are all loaded before any is stored
     typedef float f4 __attribute__((ext_vector_type(4)));
+    const bool kept = zant_out_kept(total4 * 16);
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
     f4 *y4 = reinterpret_cast<f4 *>(y);
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
@@ -759,7 +767,7 @@ __global__ void __launch_bounds__(kThreads) batchnorm_vec_f32_kernel(const float
             f4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = (v[u][e] - m[u]) / sd[u] * ga[u] + be[u];
-            __builtin_nontemporal_store(o, y4 + j);
+            zant_store_out(o, y4 + j, kept);
         }
     }
 }
@@ -774,6 +782,7 @@ __global__ void __launch_bounds__(kThreads) batchnorm_pairs_f32_kernel(const flo
                                                                        float eps, int64_t total, uint32_t inner, FastDiv by_inner,
                                                                        uint32_t features) {
     typedef float f4 __attribute__((ext_vector_type(4)));
+    const bool kept = zant_out_kept(total * 4);
     constexpr uint32_t ELEMS = kThreads * ZANT_STREAM_U * 4;
     __shared__ f4 pairs[ELEMS / 4 + 2];  // deviation, mean, gamma, beta; inner >= 4: (inner - 1 + ELEMS - 1) / inner + 1 pairs at most
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
@@ -806,7 +815,7 @@ __global__ void __launch_bounds__(kThreads) batchnorm_pairs_f32_kernel(const flo
                 const f4 a = uint32_t(e) < left ? p : next;
                 o[e] = (v[u][e] - a[1]) / a[0] * a[2] + a[3];
             }
-            __builtin_nontemporal_store(o, y4 + j);
+            zant_store_out(o, y4 + j, kept);
         } else if (j == total4) {
             for (uint32_t e = 0; e < uint32_t(total & 3); ++e) {
                 const f4 a = pairs[fastdiv(local + e, by_inner)];

@@ -53,6 +53,7 @@ __global__ void __launch_bounds__(kThreads) quantize_vec_kernel(const float *__r
     const float s = scale[0];
     const uint8_t z = zp ? zp[0] : uint8_t(0);
     const int64_t n4 = n >> 2;
+    const bool kept = zant_out_kept(n);
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     const f4 *x4 = reinterpret_cast<const f4 *>(x);
     uint32_t *y4 = reinterpret_cast<uint32_t *>(y);
@@ -68,7 +69,7 @@ __global__ void __launch_bounds__(kThreads) quantize_vec_kernel(const float *__r
         if (j < n4) {
             const uint32_t r = uint32_t(sat_u8_rne(v[u].x / s, z)) | (uint32_t(sat_u8_rne(v[u].y / s, z)) << 8) |
                                (uint32_t(sat_u8_rne(v[u].z / s, z)) << 16) | (uint32_t(sat_u8_rne(v[u].w / s, z)) << 24);
-            __builtin_nontemporal_store(r, y4 + j);
+            zant_store_out(r, y4 + j, kept);
         }
     }
     if (blockIdx.x == 0) {
@@ -84,6 +85,7 @@ __global__ void __launch_bounds__(kThreads) dequantize_vec_kernel(const uint8_t 
     const float s = scale[0];
     const int z = zp ? int(zp[0]) : 0;
     const int64_t n4 = n >> 2;
+    const bool kept = zant_out_kept(n * 4);
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     const uint32_t *x4 = reinterpret_cast<const uint32_t *>(x);
     f4 *y4 = reinterpret_cast<f4 *>(y);
@@ -102,7 +104,7 @@ __global__ void __launch_bounds__(kThreads) dequantize_vec_kernel(const uint8_t 
             r.y = float(int((v[u] >> 8) & 255) - z) * s;
             r.z = float(int((v[u] >> 16) & 255) - z) * s;
             r.w = float(int(v[u] >> 24) - z) * s;
-            __builtin_nontemporal_store(r, y4 + j);
+            zant_store_out(r, y4 + j, kept);
         }
     }
     if (blockIdx.x == 0) {
@@ -140,6 +142,7 @@ __global__ void __launch_bounds__(kThreads) qlinear_act_kernel(const uint8_t *__
         return;
     }
     const int64_t n16 = n >> 4;
+    const bool kept = zant_out_kept(n);
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     const u4 *x16 = reinterpret_cast<const u4 *>(x);
     u4 *y16 = reinterpret_cast<u4 *>(y);
@@ -160,7 +163,7 @@ __global__ void __launch_bounds__(kThreads) qlinear_act_kernel(const uint8_t *__
                 r[k] = uint32_t(lut[w & 255]) | (uint32_t(lut[(w >> 8) & 255]) << 8) | (uint32_t(lut[(w >> 16) & 255]) << 16) |
                        (uint32_t(lut[w >> 24]) << 24);
             }
-            __builtin_nontemporal_store(r, y16 + j);
+            zant_store_out(r, y16 + j, kept);
         }
     }
     if (blockIdx.x == 0) {
@@ -202,6 +205,7 @@ __global__ void __launch_bounds__(kThreads) qlinear_add_kernel(const uint8_t *__
     // the kernel's time, two thirds of that in bank conflicts).
     const float za = float(q.a_zp), zb = float(q.b_zp);
     const int64_t n16 = n >> 4;
+    const bool kept = zant_out_kept(n);
     const int64_t base = int64_t(blockIdx.x) * (kThreads * ZANT_STREAM_U) + threadIdx.x;
     const u4 *a16 = reinterpret_cast<const u4 *>(a);
     const u4 *b16 = reinterpret_cast<const u4 *>(b);
@@ -239,7 +243,7 @@ __global__ void __launch_bounds__(kThreads) qlinear_add_kernel(const uint8_t *__
                     }
                     r[w] = o ^ flip4;
                 }
-                __builtin_nontemporal_store(r, y16 + j);
+                zant_store_out(r, y16 + j, kept);
             }
         }
     };

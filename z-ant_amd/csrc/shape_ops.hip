@@ -202,6 +202,7 @@ __global__ void __launch_bounds__(kThreads) concat_copy_kernel(const U *__restri
                                                               int64_t pitch, int64_t offset) {
     // streaming pattern: ZANT_STREAM_U x 256 consecutive units per workgroup, all loads before the stores
     const I base = I(blockIdx.x) * I(kThreads * ZANT_STREAM_U) + threadIdx.x;
+    const bool kept = zant_out_kept(int64_t(total) / int64_t(chunk) * pitch * int64_t(sizeof(U)));
     U v[ZANT_STREAM_U];
 #pragma unroll
     for (int k = 0; k < ZANT_STREAM_U; ++k) {
@@ -213,7 +214,7 @@ __global__ void __launch_bounds__(kThreads) concat_copy_kernel(const U *__restri
         const I u = base + I(k * kThreads);
         if (u < total) {
             const I sl = u / chunk, r = u - sl * chunk;
-            __builtin_nontemporal_store(v[k], y + (int64_t(sl) * pitch + offset + int64_t(r)));
+            zant_store_out(v[k], y + (int64_t(sl) * pitch + offset + int64_t(r)), kept);
         }
     }
 }
@@ -294,6 +295,7 @@ __global__ void __launch_bounds__(kThreads) resize_gather_vec_kernel(const U *__
                                                                     const int *__restrict__ tab, ResizeGeom g,
                                                                     unsigned nvec, unsigned ow_vec, int lds_axes, unsigned n_chunks) {
     typedef U UV __attribute__((ext_vector_type(VEC)));
+    const bool kept = zant_out_kept(int64_t(nvec) * int64_t(sizeof(UV)));
     __shared__ __attribute__((aligned(16))) int tab_lds[kResizeLdsEntries];
     const int first = g.rank - lds_axes;  // axes first .. rank-1 are looked up in LDS
     const int lds_base = first < g.rank ? int(g.tab_off[first]) : int(g.tab_total);
@@ -360,7 +362,7 @@ __global__ void __launch_bounds__(kThreads) resize_gather_vec_kernel(const U *__
 #pragma unroll
     for (int u = 0; u < ZANT_STREAM_U; ++u) {
         const unsigned v = base + unsigned(u * kThreads);
-        if (v < nvec) __builtin_nontemporal_store(out[u], reinterpret_cast<UV *>(y) + v);
+        if (v < nvec) zant_store_out(out[u], reinterpret_cast<UV *>(y) + v, kept);
     }
     }
 }
@@ -382,6 +384,7 @@ struct ResizePlanes {
 template <typename U, int VEC>
 __global__ void __launch_bounds__(kThreads) resize_planes_kernel(const U *__restrict__ x, U *__restrict__ y, ResizePlanes g) {
     typedef U UV __attribute__((ext_vector_type(VEC)));
+    const bool kept = zant_out_kept(int64_t(g.total) * int64_t(sizeof(U)));
     extern __shared__ __attribute__((aligned(16))) char lds[];
     U *span = reinterpret_cast<U *>(lds);
     int *rows = reinterpret_cast<int *>(lds + ((size_t(g.span_cap) * sizeof(U) + 15) & ~size_t(15)));
@@ -417,7 +420,7 @@ __global__ void __launch_bounds__(kThreads) resize_planes_kernel(const U *__rest
                 v[k] = from[at + cols[col]];
                 ++col;
             }
-            if (o + VEC - 1 <= o1) __builtin_nontemporal_store(v, reinterpret_cast<UV *>(y + o));
+            if (o + VEC - 1 <= o1) zant_store_out(v, reinterpret_cast<UV *>(y + o), kept);
             else
                 for (int k = 0; k < VEC; ++k)
                     if (o + k <= o1) y[o + k] = v[k];
