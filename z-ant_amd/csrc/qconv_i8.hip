@@ -1047,12 +1047,17 @@ qfirst_pack_kernel(const int8_t *__restrict__ w, const float *__restrict__ w_sca
     }
 }
 
-template <int C, int S, bool POOL, int NV>  // NV: accumulator values per lane that are real channels (8 when K <= 16)
-__global__ void __launch_bounds__(256, 2)
+// NV: accumulator values per lane that are real channels (8 when K <= 16).  A pooled layer of up to 16 filters has them in the upper half of
+// the matrix rows once more, moved by a column: one chain gives a window's left and right member, half the matrix instructions and
+// accumulators, and with 128 registers four wavefronts share a SIMD.
+template <int C, int S, bool POOL, int NV>
+__global__ void __launch_bounds__(256, NV == 8 ? 4 : 2)
 qfirst_mfma_kernel(const uint8_t *__restrict__ x, const uint4 *__restrict__ wpk, const float *__restrict__ mult,
                    const int32_t *__restrict__ corr, uint8_t *__restrict__ y, ConvGeom g, QConvArgs q, int y_blocked, int kb32) {
     constexpr int RW = C * 3, NCH = (RW + 7) / 8;
-    constexpr int PR = POOL ? 4 : 3, NWIN = POOL ? 4 : 1;
+    constexpr bool BOTH = POOL && NV == 8;
+    const int n_kb = NV == 8 ? 1 : kb32;
+    constexpr int PR = POOL ? 4 : 3, NWIN = BOTH ? 2 : POOL ? 4 : 1, DX = POOL && !BOTH ? 2 : 1;
     __shared__ __attribute__((aligned(256))) uint8_t lut[256];  // the fused activation as a byte table, in the byte values the output stores
     lut[threadIdx.x] = uint8_t((q.has_act ? qact_apply(uint8_t(threadIdx.x), q.act) : uint8_t(threadIdx.x)) ^ (y_blocked ? 0x80 : 0));
     __syncthreads();
@@ -1149,22 +1154,26 @@ qfirst_mfma_kernel(const uint8_t *__restrict__ x, const uint4 *__restrict__ wpk,
             for (int c = 0; c < C; ++c) row[c][r] = __builtin_amdgcn_perm(raw[c][r] ^ 0x80808080u, pad4, sel_r);
         }
         if (pt + n_waves < n_ptiles) issue(nxt);
-        for (int kb = 0; kb < kb32; ++kb) {
+        for (int kb = 0; kb < n_kb; ++kb) {
             const int kch = kb * 32 + lh * 4;
-            if (kb32 > 1 || !tables_loaded) {  // one block of output channels: the tables stay in registers across tiles
+            if (n_kb > 1 || !tables_loaded) {  // one block of output channels: the tables stay in registers across tiles
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
-                    cvec[v] = corr[kch + (v >> 2) * 8 + (v & 3)];
-                    mv[v] = mult[kch + (v >> 2) * 8 + (v & 3)];
+                    const int k = kch + ((BOTH ? v & 7 : v) >> 2) * 8 + (v & 3);
+                    cvec[v] = corr[k];
+                    mv[v] = mult[k];
                 }
 #pragma unroll
                 for (int ch = 0; ch < NCH; ++ch) {
-                    wa_all[ch] = as_i32x4_q(wpk[((kb * NCH + ch) * 2 + lh) * 32 + l32]);
+                    wa_all[ch] = as_i32x4_q(wpk[((kb * NCH + ch) * 2 + lh) * 32 + (BOTH ? l32 & 15 : l32)]);
                     // the window member one column to the right reads the same four input columns against the filter
                     // row moved up one byte (columns 1..3 instead of 0..2): the shift is in the weights, once per table
                     // load, instead of in every activation operand
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) wa_dx1[ch][e] = int(uint32_t(wa_all[ch][e]) << 8);
+                    for (int e = 0; e < 4; ++e) {
+                        if (BOTH) wa_all[ch][e] = int(uint32_t(wa_all[ch][e]) << (l32 & 16 ? 8 : 0));
+                        else wa_dx1[ch][e] = int(uint32_t(wa_all[ch][e]) << 8);
+                    }
                 }
                 any_negative = false;
 #pragma unroll
@@ -1187,8 +1196,8 @@ qfirst_mfma_kernel(const uint8_t *__restrict__ x, const uint4 *__restrict__ wpk,
                         b[j] = int(lh ? vb : va);
                     }
 #pragma unroll
-                    for (int dx = 0; dx < (POOL ? 2 : 1); ++dx) {
-                        const int wd = dy * 2 + dx;
+                    for (int dx = 0; dx < DX; ++dx) {
+                        const int wd = dy * DX + dx;
                         acc[wd] = __builtin_amdgcn_mfma_i32_32x32x32_i8(dx ? wa_dx1[ch] : wa_all[ch], b, ch == 0 ? cvec : acc[wd], 0, 0, 0);
                     }
                 }
@@ -1196,13 +1205,14 @@ qfirst_mfma_kernel(const uint8_t *__restrict__ x, const uint4 *__restrict__ wpk,
             if (POOL) {
                 // requantisation and the activation keep (multiplier >= 0) or reverse (< 0) the order of the accumulators;
                 // scales are positive in practice, and then the minima are never computed
+                auto member = [&](int m, int v) { return BOTH ? acc[m >> 1][v + (m & 1) * 8] : acc[m % NWIN][v]; };
                 if (!any_negative) {
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) acc[0][v] = max(max(acc[0][v], acc[1][v]), max(acc[2][v], acc[3][v]));
+                    for (int v = 0; v < NV; ++v) acc[0][v] = max(max(acc[0][v], member(1, v)), max(member(2, v), member(3, v)));
                 } else {
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
-                        const int a0 = acc[0][v], a1 = acc[1][v], a2 = acc[2][v], a3 = acc[3][v];
+                        const int a0 = acc[0][v], a1 = member(1, v), a2 = member(2, v), a3 = member(3, v);
                         const int mx = max(max(a0, a1), max(a2, a3)), mn = min(min(a0, a1), min(a2, a3));
                         acc[0][v] = mv[v] >= 0.0f ? mx : mn;
                     }
@@ -1227,7 +1237,7 @@ qfirst_mfma_kernel(const uint8_t *__restrict__ x, const uint4 *__restrict__ wpk,
                 // channel kch of the position; the lane's other channels are whole planes further on
                 const unsigned pos = out0 + __umul24(unsigned(oho), unsigned(OWo)) + unsigned(owo) + unsigned(kch) * per_img;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
+                for (int v = 0; v < NV; ++v) {
                     const int dk = (v >> 2) * 8 + (v & 3);
                     if (kch + dk < g.K) y[pos + unsigned(dk) * per_img] = uint8_t(d[v >> 2] >> (8 * (v & 3)));
                 }
