@@ -1598,6 +1598,86 @@ size_t qdw_table_bytes(int C) {
     return 2 * align256(size_t(CB) * 64) + size_t(CB) * 144 * 4;
 }
 
+// Fully connected layers (1x1 on a 1x1 map) of few images: what they take is their weights, once from memory.  A wave computes one output
+// channel of all images: its row of weights, as it is stored, stays in registers (no packing), a lane holding 16 channels of every 1024.
+// The matrix-core kernel deals 64 channels to a workgroup, which reads their weights on its own: 1280 -> 1000 of one image on 16 of 256
+// CUs (9.9 us of MobileNetV2's pass; here the pass of one image takes 121.4 -> 114.6 us, a call by itself 17.7 -> 12.2, 4096 -> 4096 94 -> 12
+// and, with 64 images, 2076 -> 47).  C is a multiple of 16: a blocked tensor is then its channels in a row, like an NCHW one (flip: 0x80 in every byte for that).
+template <int U>
+__global__ void __launch_bounds__(256) qfc_kernel(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const float *__restrict__ w_scale,
+                                                  const int32_t *__restrict__ bias, uint8_t *__restrict__ y, int N, int units, int K, int y_pitch,
+                                                  QConvArgs q, uint32_t flip, int y_flip) {
+    const int lane = threadIdx.x & 63, k = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    if (k >= y_pitch) return;
+    if (k >= K) {  // (the rest of a blocked output's last 16 channels)
+        if (lane < N) y[lane * y_pitch + k] = 0;
+        return;
+    }
+    uint4 wv[U];
+    int sum = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int at = u * 64 + lane;
+        wv[u] = at < units ? w[int64_t(k) * units + at] : uint4{0u, 0u, 0u, 0u};
+        sum = __builtin_amdgcn_sdot4(int(wv[u].x), 0x01010101, sum, false);
+        sum = __builtin_amdgcn_sdot4(int(wv[u].y), 0x01010101, sum, false);
+        sum = __builtin_amdgcn_sdot4(int(wv[u].z), 0x01010101, sum, false);
+        sum = __builtin_amdgcn_sdot4(int(wv[u].w), 0x01010101, sum, false);
+    }
+    const float m = (q.x_scale * w_scale[q.n_wscale == 1 ? 0 : k]) / q.y_scale;
+    const int b = bias ? bias[k] : 0;
+    // (128 - x_zp) * sum of weights joins every lane's part of the sum of products
+    const int own = (128 - q.x_zp) * sum;
+    int mine = 0;  // lane n: image n's sum
+    constexpr int G = 4;
+    for (int n0 = 0; n0 < N; n0 += G) {
+        int acc[G];
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const uint4 *xn = x + int64_t(min(n0 + i, N - 1)) * units;
+            acc[i] = own;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint4 v = xn[min(u * 64 + lane, units - 1)];  // (past the row: against zero weights)
+                acc[i] = __builtin_amdgcn_sdot4(int(v.x ^ flip), int(wv[u].x), acc[i], false);
+                acc[i] = __builtin_amdgcn_sdot4(int(v.y ^ flip), int(wv[u].y), acc[i], false);
+                acc[i] = __builtin_amdgcn_sdot4(int(v.z ^ flip), int(wv[u].z), acc[i], false);
+                acc[i] = __builtin_amdgcn_sdot4(int(v.w ^ flip), int(wv[u].w), acc[i], false);
+            }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int i = 0; i < G; ++i) acc[i] += __shfl_xor(acc[i], o, 64);
+#pragma unroll
+        for (int i = 0; i < G; ++i) mine = lane == n0 + i ? acc[i] : mine;
+    }
+    if (lane < N) y[lane * y_pitch + k] = uint8_t(requant(mine + b, m, q) ^ y_flip);
+}
+constexpr int QFC_MAX_N = 64;
+bool qfc_eligible(const ConvGeom &g, const void *x, const void *w) {
+    return g.groups == 1 && g.H == 1 && g.W == 1 && g.KH == 1 && g.KW == 1 && g.OH == 1 && g.OW == 1 && g.pt == 0 && g.pl == 0 && g.C % 16 == 0 &&
+           g.C <= 4096 && g.N <= QFC_MAX_N && g.K <= (1 << 24) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+}
+int run_qfc(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float *w_scale, const int32_t *bias, uint8_t *y, const ConvGeom &g,
+            const QConvArgs &q, bool xb, bool yb) {
+    const int pitch = yb ? (g.K + 15) / 16 * 16 : g.K, units = g.C / 16;
+    KernelTimer kt(ctx);
+    ZANT_KERNEL_NAME(ctx, "qfc_kernel<%d>", (units + 63) / 64);
+#define ZANT_QFC(U)                                                                                                                    \
+    hipLaunchKernelGGL(qfc_kernel<U>, dim3(unsigned(pitch + 3) / 4), dim3(256), 0, ctx->stream, reinterpret_cast<const uint4 *>(x),    \
+                       reinterpret_cast<const uint4 *>(w), w_scale, bias, y, g.N, units, g.K, pitch, q, xb ? 0u : 0x80808080u, yb ? 0x80 : 0)
+    switch ((units + 63) / 64) {
+    case 1: ZANT_QFC(1); break;
+    case 2: ZANT_QFC(2); break;
+    case 3: ZANT_QFC(3); break;
+    default: ZANT_QFC(4); break;
+    }
+#undef ZANT_QFC
+    ZANT_LAUNCH_CHECK(ctx);
+    return ZANT_OK;
+}
+
 // x, y blocked; `tables` holds qdw_table_bytes(C) bytes that are (re)filled when need_pack is set.  x_nchw: the input as it came, still to
 // be written to xb (null: xb holds it).
 int run_qdw_blocked(zant_ctx *ctx, const uint8_t *x_nchw, uint8_t *xb, const int8_t *w, const float *w_scale, const int32_t *bias, uint8_t *yb,
@@ -1774,6 +1854,7 @@ int zant_qlinearconv_layout_pool(zant_ctx *ctx, const uint8_t *x, const int64_t 
         if (rc) return rc;
         return yb ? ZANT_OK : zant_from_blocked(ctx, yout, g.N, g.K, int64_t(g.OH) * g.OW, y);
     }
+    if (w_zp == nullptr && qfc_eligible(g, x, w)) return run_qfc(ctx, x, w, w_scale, bias, y, g, q, xb, yb);
     if (w_zp == nullptr) {  // a non-zero weight zero point makes the correction position dependent: direct kernel
         const int rc = run_qconv_mfma(ctx, x, w, w_scale, bias, y, g, q, xb, yb, slot);
         if (rc <= 0) return rc;
