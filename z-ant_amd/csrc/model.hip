@@ -1286,12 +1286,16 @@ extern "C" int zant_model_predict_host(zant_model *m, const void *input_host, vo
     if (!m || !input_host || !output_host) return ZANT_NullPointer;
     if (!m->finalized) return ZANT_NotFinalized;
     zant_ctx *ctx = m->ctx;
-    int rc = zant_hip_upload(ctx, tensor_ptr(m, m->input), input_host, m->t[m->input].bytes());
-    if (rc) return rc;
+    // Not waited for here: the caller has the buffer back after the last copy's wait, or after this one on a failure.  The nodes are enqueued
+    // while the input travels: README CNN on one image 67.5 -> 57.5 us.
+    ZANT_HIP_TRY(ctx, hipMemcpyAsync(tensor_ptr(m, m->input), input_host, m->t[m->input].bytes(), hipMemcpyHostToDevice, ctx->stream));
     for (const MNode &nd : m->n) {
         if (nd.skip) continue;
-        rc = run_node(m, nd);
-        if (rc) return rc;
+        const int rc = run_node(m, nd);
+        if (rc) {
+            (void)hipStreamSynchronize(ctx->stream);
+            return rc;
+        }
     }
     return zant_hip_download(ctx, output_host, tensor_ptr(m, m->output), m->t[m->output].bytes());
 }
