@@ -1659,6 +1659,9 @@ bool qfc_eligible(const ConvGeom &g, const void *x, const void *w) {
     return g.groups == 1 && g.H == 1 && g.W == 1 && g.KH == 1 && g.KW == 1 && g.OH == 1 && g.OW == 1 && g.pt == 0 && g.pl == 0 && g.C % 16 == 0 &&
            g.C <= 4096 && g.N <= QFC_MAX_N && g.K <= (1 << 24) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
 }
+// A call by itself on one image keeps the kernel that it is tested to take below 2 MB of weights (1280 -> 1000: 17.7 us there, 12.2 here);
+// model nodes, plans, several images and larger layers (4096 -> 4096: 94 us there) take this one.
+bool qfc_preferred(const ConvGeom &g, bool kept) { return kept || g.N > 1 || int64_t(g.C) * g.K >= (int64_t(1) << 21); }
 int run_qfc(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float *w_scale, const int32_t *bias, uint8_t *y, const ConvGeom &g,
             const QConvArgs &q, bool xb, bool yb) {
     const int pitch = yb ? (g.K + 15) / 16 * 16 : g.K, units = g.C / 16;
@@ -1854,7 +1857,7 @@ int zant_qlinearconv_layout_pool(zant_ctx *ctx, const uint8_t *x, const int64_t 
         if (rc) return rc;
         return yb ? ZANT_OK : zant_from_blocked(ctx, yout, g.N, g.K, int64_t(g.OH) * g.OW, y);
     }
-    if (w_zp == nullptr && qfc_eligible(g, x, w)) return run_qfc(ctx, x, w, w_scale, bias, y, g, q, xb, yb);
+    if (w_zp == nullptr && qfc_eligible(g, x, w) && qfc_preferred(g, slot != nullptr)) return run_qfc(ctx, x, w, w_scale, bias, y, g, q, xb, yb);
     if (w_zp == nullptr) {  // a non-zero weight zero point makes the correction position dependent: direct kernel
         const int rc = run_qconv_mfma(ctx, x, w, w_scale, bias, y, g, q, xb, yb, slot);
         if (rc <= 0) return rc;
