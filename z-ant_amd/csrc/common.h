@@ -118,8 +118,8 @@ static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b;
 constexpr int64_t ZANT_MAX_BLOCKS_256 = (int64_t(1) << 24) - 1;
 
 // Streaming pattern of the HBM-bound elementwise kernels: a workgroup of 256 threads handles ZANT_STREAM_U x 256
-// consecutive vectors, issuing all its loads before its stores, with nontemporal hints on both (measured on a
-// 354 MB f32 stream: 6.7 TB/s against 5.0 TB/s for a grid-stride loop of plain 16-byte accesses).
+// consecutive vectors, issuing all its loads, nontemporal ones, before its stores (a 354 MB f32 stream, nontemporal both ways: 6.7 TB/s
+// against 5.0 for a grid-stride loop of plain 16-byte accesses; for the stores see zant_store_out).
 constexpr int ZANT_STREAM_U = 4;
 static inline unsigned zant_stream_grid(int64_t vectors) {
     const int64_t b = ceil_div64(vectors, int64_t(256) * ZANT_STREAM_U);

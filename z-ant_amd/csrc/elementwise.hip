@@ -363,7 +363,7 @@ __global__ void __launch_bounds__(kThreads) maxpool_2x2s2_kernel(const T *__rest
 // 2x2 / stride 2 with even rows of inputs read as vectors: a thread turns two row segments of 2 * VEC inputs into VEC
 // outputs (f32: VEC = 1, two 8-byte loads; u8: VEC = 8, two 16-byte loads, one 8-byte store).  A workgroup covers
 // kThreads * ZANT_STREAM_U consecutive output vectors of the flattened [NC * OH, OW / VEC] grid and issues all its
-// loads before its stores, nontemporal both ways (the streaming pattern of the elementwise kernels).  Needs W even
+// loads before its stores (the streaming pattern of the elementwise kernels).  Needs W even
 // (f32) or a multiple of 16 (u8), OW a multiple of VEC and aligned bases; the host checks.
 // ANY (u8): any W and any alignment, OW >= VEC.  The last vector of a row starts early enough to end with the row (what it shares with the
 // one before is written twice, the same), and loads are plain: neighbours share cache lines.  1000x64x48x50: 106 us with a thread's

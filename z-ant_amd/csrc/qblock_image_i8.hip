@@ -9,7 +9,7 @@
 // projection stage, (32 positions x 8 output channels) in the last -- are dealt to the waves one by one, and the projection's
 // sums meet in LDS by integer additions, whose order does not matter.  The arithmetic is qblock_kernel's: the same bytes.
 // MobileNetV2-0.35's last 14 blocks, one image: 139 us as two tile chains and a block, 97 with eight waves, 82 with sixteen, 71 with the
-// tables packed beside the weights (they were the longest unit) and the arguments prefetched.  Of a block's 5 us the expansion
+// tables packed beside the weights (they were the longest unit) and the arguments prefetched, 69 with lookups by address.  Of a block's 5 us the expansion
 // takes 1.3, depthwise and projection 2, the last stage 1.2, mostly vector instructions of three or four waves a SIMD.
 #include <algorithm>
 #include <cstring>

@@ -1101,7 +1101,7 @@ qfirst_mfma_kernel(const uint8_t *__restrict__ x, const uint4 *__restrict__ wpk,
     const unsigned d_n = step / per_img, step_r = step - d_n * per_img;
     const int d_oho = int(step_r / unsigned(OWo)), d_owo = int(step_r - unsigned(d_oho) * unsigned(OWo));
     const unsigned d_in = d_n * img_in, d_out = d_n * out_img;
-    // The row loads of the NEXT tile are issued before this tile's arithmetic: with two wavefronts per SIMD the load
+    // The row loads of the NEXT tile are issued before this tile's arithmetic: with two to four wavefronts per SIMD the load
     // latency would otherwise sit on the critical path of every tile.
     struct TileMeta { unsigned out0; int oho, owo, ih0, sh; bool valid; };  // out0: the image's first output element
     uint32_t raw[C][PR];
