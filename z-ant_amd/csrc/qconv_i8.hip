@@ -142,6 +142,7 @@ struct QPackJob {
     int K, C, T, n_chunks, n_kblocks, k_blk;
     float x_scale, y_scale;
     int x_zp, n_wscale, fc_g, c_orig;
+    int pair;  // 3x3 of up to 16 channels, two taps of a row an operand (TAPS_PAIRED)
 };
 // by workgroup `block` of `blocks`
 __device__ __forceinline__ void qpack(const QPackJob &p, unsigned block, unsigned blocks) {
@@ -163,6 +164,9 @@ __device__ __forceinline__ void qpack(const QPackJob &p, unsigned block, unsigne
             // regrouped 1x1 layer: "tap" t of 16-channel block b is channel block b * fc_g + t of the c_orig real channels
             const int oc = ((c >> 4) * fc_g + tap) * 16 + j;
             p.wp[i] = (k < K && oc < c_orig) ? p.w[int64_t(k) * c_orig + oc] : int8_t(0);
+        } else if (p.pair) {
+            const int kw = 2 * (tap & 1) + half;  // the fourth column of a row is none
+            p.wp[i] = (k < K && j < C && kw < 3) ? p.w[(int64_t(k) * C + j) * 9 + (tap >> 1) * 3 + kw] : int8_t(0);
         } else {
             p.wp[i] = (k < K && c < C) ? p.w[(int64_t(k) * C + c) * T + tap] : int8_t(0);
         }
@@ -174,7 +178,7 @@ __device__ __forceinline__ void qpack(const QPackJob &p, unsigned block, unsigne
     for (int64_t k = wave; k < kpad; k += n_waves) {
         int sum = 0;
         if (k < K) {
-            const int row = fc_g ? c_orig : C * T;
+            const int row = fc_g ? c_orig : C * (p.pair ? 9 : T);
             const int8_t *wk = p.w + k * int64_t(row);
             for (int e = lane; e < row; e += 64) sum += int(wk[e]);
         }
@@ -198,6 +202,13 @@ __global__ void __launch_bounds__(256) qpack_blocked_kernel(QPackJob p, BlockedJ
 }
 
 // Bytes of the weight region of a staging buffer: the slab rounded up to one 16-byte unit per thread and round.
+// 3x3 layers of up to 16 channels: a matrix instruction takes 32 of the sum, two neighbouring taps of a filter row -- the halves of a wave read
+// positions one (dilated) column apart instead of two channel blocks -- and a row is two such pairs, the fourth tap's weights zero: six
+// instructions and operand reads instead of nine half empty ones.  What a fourth tap reads past a row or the patch is in the copy's unused
+// second half at most (PW > 2 dw) and meets zero weights.  16 -> 96 channels on 512 maps of 48x48 112.5 -> 105 us a call, 16 -> 32 52.6 ->
+// 49.6, with stride 2 33.4 -> 32.2, 256 maps of 64x64 8 -> 64 67 -> 63.4; tiny-YOLO's pass 125 -> 122.
+constexpr int TAPS_PAIRED = 6;
+__device__ __host__ __forceinline__ bool taps_paired(const ConvGeom &g) { return g.C <= 16 && g.KH == 3 && g.KW == 3; }
 __device__ __host__ __forceinline__ int w_region_bytes(int w_chunk, int nt) { return ((w_chunk / 16 + nt - 1) / nt) * nt * 16; }
 
 // Where this thread's patch slots of one tile come from: byte offset of the first 16-channel half of chunk 0 from the
@@ -326,7 +337,8 @@ __device__ __forceinline__ void qconv_step(char *__restrict__ dma, const char *_
     __builtin_amdgcn_sched_barrier(0);
 
     const char *wl = cmp + (lh * K_BLK + wn * 32 + l32) * 16;
-    const char *xl = cmp + w_region_bytes(w_chunk, NT) + lh * t.P1s * 16;
+    constexpr int KW_STEP = TT == TAPS_PAIRED ? 2 : 1;
+    const char *xl = cmp + w_region_bytes(w_chunk, NT) + lh * (TT == TAPS_PAIRED ? g.dw : t.P1s) * 16;
     i32x4 a0, a1, b0[MT], b1[MT];
     int lkh = 0, lkw = 0, ltap = 0;
     auto load_tap = [&](i32x4 &a, i32x4 (&b)[MT]) {
@@ -335,7 +347,7 @@ __device__ __forceinline__ void qconv_step(char *__restrict__ dma, const char *_
 #pragma unroll
         for (int i = 0; i < MT; ++i) b[i] = *reinterpret_cast<const i32x4 *>(xl + lds_off[i] * 16 + off);
         ++ltap;
-        if (++lkw == g.KW) { lkw = 0; ++lkh; }
+        if ((lkw += KW_STEP) >= g.KW) { lkw = 0; ++lkh; }
     };
     auto mfma_tap = [&](const i32x4 &a, const i32x4 (&b)[MT]) {
         __builtin_amdgcn_s_setprio(1);
@@ -634,7 +646,8 @@ void launch_qmfma(zant_ctx *ctx, const int8_t *xb, const int8_t *wp, const float
                   const int8_t *padvec, uint8_t *y, const ConvGeom &g, const TilePlan &p, int CB, const QConvArgs &q,
                   int grid, int yb, int n_stages) {
     const int T = g.KH * g.KW;
-    if (T == 9) launch_qmfma_tt<MT, WM, WN, 9>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
+    if (taps_paired(g)) launch_qmfma_tt<MT, WM, WN, TAPS_PAIRED>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
+    else if (T == 9) launch_qmfma_tt<MT, WM, WN, 9>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
     else if (T == 1) launch_qmfma_tt<MT, WM, WN, 1>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
     else launch_qmfma_tt<MT, WM, WN, 0>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
 }
@@ -646,7 +659,8 @@ bool dispatch_qmt(zant_ctx *ctx, const int8_t *xb, const int8_t *wp, const float
     if (pool) {  // four window members per lane: MT = 4
         if (p.MT != 4) return false;
         const int T = g.KH * g.KW;
-        if (T == 9) launch_qmfma_tt<4, WM, WN, 9, true>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
+        if (taps_paired(g)) launch_qmfma_tt<4, WM, WN, TAPS_PAIRED, true>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
+        else if (T == 9) launch_qmfma_tt<4, WM, WN, 9, true>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
         else if (T == 1) launch_qmfma_tt<4, WM, WN, 1, true>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
         else launch_qmfma_tt<4, WM, WN, 0, true>(ctx, xb, wp, mult, corr, padvec, y, g, p, CB, q, grid, yb, n_stages);
         return true;
@@ -739,7 +753,7 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
         }
     }
     if (!have) return 1;
-    const int T = g.KH * g.KW, K_BLK = WN * 32;
+    const int T = taps_paired(g) ? TAPS_PAIRED : g.KH * g.KW, K_BLK = WN * 32;
     plan.t.n_chunks = (g.C + QCC - 1) / QCC;
     // Ring of staging buffers: as many stages as fit beside the tables in the LDS share of a workgroup -- half a CU's
     // 160 KB when two workgroups share a CU, all of it when the layer has no more tiles than the GPU has CUs (short
@@ -782,7 +796,7 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
         }
     }
     const int CB = (g.C + 15) / 16;
-    const int T = g.KH * g.KW, K_BLK = WN * 32;
+    const int T = taps_paired(g) ? TAPS_PAIRED : g.KH * g.KW, K_BLK = WN * 32;
     const size_t buf_bytes = size_t(w_region_bytes(T * QCC * K_BLK, NT)) + size_t(QCC) * plan.t.P1s;
     const size_t fixed_bytes = size_t(plan.t.P1s) * 8 + 512 + size_t(plan.t.n_kblocks) * K_BLK * 8;  // 256: table, 256: its alignment
     if (plan_only) return ZANT_OK;
@@ -806,7 +820,7 @@ int run_qconv_mfma(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float
     const int grid = int(std::min<int64_t>(plan.t.n_tiles, int64_t(ctx->num_cus) * 2));
     const unsigned pb = unsigned(std::min<int64_t>(std::max<int64_t>(ceil_div64(int64_t(wp_bytes), 256), ceil_div64(int64_t(kpad), 4)), 1024));
     const QPackJob job = {w, w_scale, bias, wp, mult, corr, padvec, g.K, g.C, T, plan.t.n_chunks, plan.t.n_kblocks, K_BLK,
-                          q.x_scale, q.y_scale, q.x_zp, q.n_wscale, fc_g, g0.C};
+                          q.x_scale, q.y_scale, q.x_zp, q.n_wscale, fc_g, g0.C, taps_paired(g)};
     BlockedJob layout;
     const bool one_launch = need_pack && !x_blocked && zant_blocked_job(x, g0.N, g0.C, int64_t(g0.H) * g0.W, dyn, &layout);
     if (one_launch) {
@@ -1749,7 +1763,7 @@ int zant_qpack_dense(zant_ctx *ctx, const int8_t *w, const float *w_scale, int64
     const int n_chunks = (C + QCC - 1) / QCC, n_kblocks = (K + k_blk - 1) / k_blk;
     const int64_t wp_bytes = int64_t(n_chunks) * n_kblocks * T * QCC * k_blk, kpad = int64_t(n_kblocks) * k_blk;
     const unsigned pb = unsigned(std::min<int64_t>(std::max<int64_t>(ceil_div64(wp_bytes, 256), ceil_div64(kpad, 4)), 1024));
-    const QPackJob job = {w, w_scale, bias, wp, mult, corr, padvec, K, C, T, n_chunks, n_kblocks, k_blk, x_scale, y_scale, x_zp, int(n_wscale), 0, C};
+    const QPackJob job = {w, w_scale, bias, wp, mult, corr, padvec, K, C, T, n_chunks, n_kblocks, k_blk, x_scale, y_scale, x_zp, int(n_wscale), 0, C, 0};
     hipLaunchKernelGGL(qpack_kernel, dim3(pb), dim3(256), 0, ctx->stream, job);
     ZANT_LAUNCH_CHECK(ctx);
     return ZANT_OK;
