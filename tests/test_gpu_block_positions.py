@@ -1,0 +1,35 @@
+"""Position tables of the fused inverted residual block: tiles of several images of odd and even maps under both strides, the last one partly
+filled, rows that do not divide a map, and a block whose weights leave room for a row or two.  Bit for bit against the oracle, layer by layer."""
+import numpy as np
+import pytest
+
+import int8_ref
+from test_gpu_qblock import _arch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (H, W), stem channels, blocks (hidden, cout, stride, activations, depthwise padding), batch
+    ((7, 7), 96, [(576, 96, 1, "relu6", "relu6", 1)], 3),
+    ((4, 6), 8, [(48, 16, 2, "relu6", "relu6", 1)], 701),
+    ((5, 3), 16, [(64, 24, 2, "relu6", "leaky", 1)], 1027),
+    ((6, 5), 40, [(80, 40, 1, "leaky", "relu6", 1)], 515),
+    ((11, 30), 24, [(72, 24, 1, "relu6", "relu6", 1)], 2),
+    ((23, 9), 20, [(60, 40, 2, "relu6", "relu6", 1)], 5),
+]
+
+
+@pytest.mark.parametrize("hw,c0,blocks,batch", CASES, ids=[str(i) for i in range(len(CASES))])
+def test_blocks_match_the_oracle(hw, c0, blocks, batch):
+    import gpu_util as G
+    from zant_amd import networks as nets
+    arch = _arch(hw, c0, blocks)
+    params = nets.int8_params(arch, seed=7)
+    rng = np.random.default_rng(batch)
+    quant = int8_ref.calibrate(arch, params, rng.integers(0, 256, (2,) + arch["input"], dtype=np.uint8))
+    x = rng.integers(0, 256, (batch,) + arch["input"], dtype=np.uint8)
+    sample = np.unique(np.r_[0:min(batch, 5), max(batch - 5, 0):batch])
+    m = nets.build_int8_model(G.tm.context(), arch, params, quant, batch)
+    assert m.num_launches == 3
+    np.testing.assert_array_equal(m.predict_host(x)[sample], int8_ref.forward(arch, params, quant, x[sample]))
+    m.close()

@@ -14,32 +14,36 @@ struct QBlockArgs {
     int split;                         // stage D deals (position tile, channel chunk) units to the waves (few position tiles)
     int zp1, zp2;                      // zero points of the three convolutions' own outputs
     float zp3f;
-    QAct act1, act2;
-    int has_act1, has_act2;
     uint32_t pad_e4;                   // the depthwise input zero point ^ 0x80 in every byte
     int half_last;                     // the last chunk of expanded channels holds at most 16 real ones
     int has_res, fast_div;             // fast_div: the scales allow the unscaled division sequence
     float ry_rcp;                      // refined reciprocal of ry_scale
     float ra_scale, rb_scale, ry_scale;  // residual add: a = projection output, b = block input, y = sum
     int ra_zp, rb_zp, ry_zp;
+    QAct act1, act2;                   // what only the tables are made from comes last: the kernels load their arguments in wide pieces
+    int has_act1, has_act2;
 };
 
 // The activation part of a block's tables: QB_ACT_HEAD bytes of QBlockActHead, then the two activation tables, each at an address of
 // its convolution's zero point's parity (quant_common.h).
-constexpr int QB_ACT_HEAD = 32, QB_ACT_TABLE = 272, QB_ACT_BYTES = QB_ACT_HEAD + 2 * QB_ACT_TABLE;
+constexpr int QB_ACT_HEAD = 4, QB_ACT_TABLE = 258, QB_ACT_BYTES = (QB_ACT_HEAD + 2 * QB_ACT_TABLE + 15) / 16 * 16;
 struct QBlockActHead {
-    int lo1, hi1, lo2, hi2;  // the entries between which each table changes
-    int unused[4];
+    uint8_t lo1, hi1, lo2, hi2;  // the entries between which each table changes
 };
-// The position tables.  Of a patch position (Ppad entries): x the patch row, bit 31 set for a halo column or past the patch; y the byte
-// offset of its first unit from that of the tile's first image, patch row 0, column 0.  Of an output position (Q rounded up to 32): x
-// the byte offset of its top-left tap in the patch, y that of its first output unit from the tile's first one.
-typedef int2 QBlockPos;
-static_assert(sizeof(QBlockActHead) == QB_ACT_HEAD && QB_ACT_BYTES % 16 == 0 && QB_ACT_TABLE >= 257, "layout of the tables");
+static_assert(sizeof(QBlockActHead) == QB_ACT_HEAD && QB_ACT_TABLE % 2 == 0 && QB_ACT_TABLE >= 257, "layout of the tables");
+// The position tables, 16 bits an entry: what is more in LDS is a smaller tile, a workgroup less on a CU or a block that does not fit (with
+// 8 bytes an entry 96 -> 576 -> 96 channels did not, 64 -> 192 -> 64 on 1024 maps of 20x20 took 171 us instead of 141).  Of a patch
+// position (Ppad entries): its row among those of the tile's images, QB_POS_PAD set for a halo column, past the patch and, in tiles of
+// whole images, for the rows above and below an image.  Of an output position (Q rounded up to 32): its top-left tap's patch position.
+typedef uint16_t QBlockPos;
+constexpr int QB_POS_PAD = 0x8000;
 
 #ifdef __HIPCC__
-__device__ __forceinline__ RequantLut qb_lut(const char *act, int table, int lo, int hi, int zp) {
+// `head`: the four bytes of QBlockActHead, in a scalar register
+__device__ __forceinline__ unsigned qb_act_head(const char *act) { return __builtin_amdgcn_readfirstlane(*reinterpret_cast<const unsigned *>(act)); }
+__device__ __forceinline__ RequantLut qb_lut(const char *act, unsigned head, int table, int zp) {
     const int base = int(lds_address(act)) + QB_ACT_HEAD + table * QB_ACT_TABLE + (zp & 1);
+    const int lo = (head >> (16 * table)) & 255, hi = (head >> (16 * table + 8)) & 255;
     RequantLut t;
     t.t0 = zq_as_float(unsigned(base + zp));
     t.lo = zq_as_float(unsigned(base + lo));
@@ -61,6 +65,13 @@ struct QBlockPrep {
 int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_desc *expand, const zant_qconv_desc *dw, int64_t dw_stride,
                         const zant_qconv_desc *project, int residual, float add_scale, int add_zp, const int64_t ydim[4], bool plan_only,
                         zant_pack_slot *slot, int force_nb, QBlockPrep *out);
+
+// LDS bytes that a block takes of a chain on one image a workgroup: input patch of `positions`, `weights` and tables, expanded patch,
+// projection sums of `outputs`.
+static inline size_t zant_qblock_image_bytes(int Cin32, int Ce32, int co32, int64_t positions, int64_t outputs, int64_t weights) {
+    const size_t Ppad = size_t(positions + 31) & ~size_t(31), Qpad = size_t(outputs + 31) & ~size_t(31);
+    return size_t(Cin32 + Ce32) * 2 * Ppad * 16 + size_t(weights) + QB_ACT_BYTES + (Ppad + Qpad) * sizeof(QBlockPos) + Qpad / 32 * co32 * 4096;
+}
 
 // zant_qblock_chain on one image a workgroup, activations in LDS from block to block (qblock_image_i8.hip); 1 when the blocks do not
 // fit that or there are too many images.

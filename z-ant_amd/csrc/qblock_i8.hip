@@ -35,21 +35,25 @@ __device__ __forceinline__ i32x4 as_i32x4(const uint4 &v) {
     return r;
 }
 
-// Table entries of patch position p and output position q of a tile.
-__device__ __forceinline__ QBlockPos qb_patch_pos(const QBlockArgs &a, int p, float inv_patch_hw, float inv_pw) {
-    const int pp = min(p, a.P - 1), img = small_div(pp, a.PH * a.PW, inv_patch_hw), rem = pp - img * a.PH * a.PW;
-    const int ph = small_div(rem, a.PW, inv_pw), pw = rem - ph * a.PW;
-    QBlockPos e;
-    e.x = ph | (p >= a.P || pw == 0 || pw == a.PW - 1 ? int(0x80000000u) : 0);
-    e.y = ((img * a.CBin * a.H + ph) * a.W + pw - 1) * 16;
-    return e;
+// p / d for 0 <= p < 2^15 with inv = 1.0f / d to within a few units in the last place: (p + 1/2) / d is at least 1 / 2d away from a whole
+// number, further than reciprocal and fma err.
+__device__ __forceinline__ int quick_div(int p, float inv) { return int(__builtin_fmaf(float(p), inv, 0.5f * inv)); }
+
+// 1 / d, taken anew where it is used: two instructions, but registers are scarce from one tile to the next
+__device__ __forceinline__ float fresh_rcp(int d) {
+    asm volatile("" : "+s"(d));
+    return __builtin_amdgcn_rcpf(float(d));
 }
-__device__ __forceinline__ QBlockPos qb_out_pos(const QBlockArgs &a, int q) {
+
+// Table entries of patch position p and output position q of a tile.
+__device__ __forceinline__ int qb_patch_pos(const QBlockArgs &a, int p) {
+    const int row = p / a.PW, pw = p - row * a.PW, ph = row % a.PH;
+    const bool pad = p >= a.P || pw == 0 || pw == a.PW - 1 || (a.n_row_tiles == 1 && unsigned(ph - 1) >= unsigned(a.H));
+    return row | (pad ? QB_POS_PAD : 0);
+}
+__device__ __forceinline__ int qb_out_pos(const QBlockArgs &a, int q) {
     const int qq = min(q, a.Q - 1), img = qq / (a.TH * a.OW), rem = qq - img * a.TH * a.OW, r = rem / a.OW, c = rem - r * a.OW;
-    QBlockPos e;
-    e.x = ((img * a.PH + r * a.stride) * a.PW + c * a.stride) * 16;
-    e.y = ((img * a.CBo * a.OH + r) * a.OW + c) * 16;
-    return e;
+    return (img * a.PH + r * a.stride) * a.PW + c * a.stride;
 }
 
 // One block for the tiles of this workgroup; `lds` is the workgroup's dynamic LDS.
@@ -94,18 +98,25 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     // first tile's patch is copied before the loop; every later one is loaded into registers before stage B of the tile
     // in front of it and written to LDS after that stage (the input patch is dead once B is done), so its global
     // latency passes under B.  Patches of more than QB_PF units per thread are copied in place instead. ----
-    // A round is 256 positions of one channel block.  The first tile's positions are taken apart by division, while the tables are on their
-    // way; every later tile's come from the table (8 instead of 60 vector instructions a unit, six of them quarter rate).
+    // A round is 256 positions of one channel block.  A position's row, which with the position itself gives its place in x, is divided out
+    // for the first tile, while the tables are on their way; every later tile's comes from the table (60 vector instructions a unit, six of
+    // them quarter rate, when positions were taken apart for each).
     constexpr int QB_PF = 4;
     const int patch_hw = a.PH * a.PW;
     const int p_rounds = (a.Ppad + 255) >> 8, a_rounds = a.CBin * p_rounds;
     const bool prefetch = PF && a_rounds <= QB_PF;  // PF is off for the instantiations without registers to spare
     const int64_t in_plane = int64_t(a.H) * a.W * 16;
-    struct Source { const char *base; int ih0, positions; unsigned valid; };  // `valid`: an offset that lies inside the tensor
+    // a row of the patch is in the map (tiles of whole images: as the table says)
+    const int rows_in = a.n_row_tiles > 1 ? a.H : QB_POS_PAD;
+    // valid: an offset that lies inside the tensor; img_gap: units from an image's rows to the next one's beyond those of the patch
+    struct Source { const char *base; int ih0, row0, positions, img_gap; unsigned valid; float inv_ph; };
     auto source_of = [&](int tile_) {
         const int ig_ = tile_ / a.n_row_tiles, rt_ = tile_ - ig_ * a.n_row_tiles, n_ = ig_ * a.NB;
         Source s;
         s.ih0 = rt_ * a.TH * a.stride - 1;
+        s.row0 = a.n_row_tiles > 1 ? s.ih0 : 0;
+        s.img_gap = (a.CBin * a.H - a.PH) * a.W;
+        s.inv_ph = fresh_rcp(a.PH);
         s.positions = a.n_row_tiles > 1 ? a.P : min(a.NB, a.N - n_) * patch_hw;
         s.base = reinterpret_cast<const char *>(x) + (int64_t(n_) * a.CBin * a.H + s.ih0) * int64_t(a.W) * 16;
         s.valid = s.ih0 < 0 ? unsigned(a.W) * 16u : 0u;
@@ -113,12 +124,20 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     };
     // every lane loads (from a place inside the tensor when it has nothing to fetch): no divergent branch around the load, so nothing
     // waits for it before the values are written to LDS
-    auto fetch = [&](const Source &s, int cb, int p, const QBlockPos &e, i32x4 &v) {
-        const bool ok = p < s.positions && e.x >= 0 && unsigned(s.ih0 + (e.x & 0xffff)) < unsigned(a.H);
-        v = *reinterpret_cast<const i32x4 *>(s.base + cb * in_plane + (ok ? unsigned(e.y) : s.valid));
+    auto fetch = [&](const Source &s, int cb, int p, auto place, i32x4 &v) {
+        int unit;
+        const bool ok = place(s, p, unit) && p < s.positions;
+        v = *reinterpret_cast<const i32x4 *>(s.base + cb * in_plane + (ok ? unsigned(unit) * 16u : s.valid));
         return ok;
     };
-    auto copy_patch = [&](int tile_, auto entry) {  // four loads in flight per thread, then their four LDS writes
+    // whether patch position p lies in the map, and its unit from the patch's first row, column 0, on
+    auto from_table = [&](const Source &s, int p, int &unit) {
+        const int e = ptab[min(p, a.Ppad - 1)], row = e & (QB_POS_PAD - 1);
+        unit = p - 2 * row - 1;  // = row * W + column
+        if (a.NB > 1) unit += quick_div(row, s.inv_ph) * s.img_gap;
+        return !(e & QB_POS_PAD) && unsigned(s.row0 + row) < unsigned(rows_in);
+    };
+    auto copy_patch = [&](int tile_, auto place) {  // four loads in flight per thread, then their four LDS writes
         const Source s = source_of(tile_);
         int cb = 0, pr = 0;
         for (int r0 = 0; r0 < a_rounds; r0 += 4) {
@@ -131,7 +150,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                 dst[r] = cb * a.Ppad + p;
                 ok[r] = false;
                 if (r0 + r < a_rounds) {
-                    ok[r] = fetch(s, cb, p, entry(p), v[r]);
+                    ok[r] = fetch(s, cb, p, place, v[r]);
                     if (++pr == p_rounds) { pr = 0; ++cb; }
                 }
             }
@@ -141,10 +160,19 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         }
     };
     if (int(blockIdx.x) < a.n_tiles) {
-        const float inv_patch_hw = 1.0f / float(patch_hw), inv_pw = 1.0f / float(a.PW);
-        copy_patch(blockIdx.x, [&](int p) { return qb_patch_pos(a, p, inv_patch_hw, inv_pw); });
+        const float inv_pw = fresh_rcp(a.PW);
+        copy_patch(blockIdx.x, [&](const Source &s, int p, int &unit) {
+            const int row = quick_div(p, inv_pw), column = p - row * a.PW - 1;
+            int ph = row;
+            unit = row * a.W + column;
+            if (a.NB > 1) {
+                const int img = quick_div(row, s.inv_ph);
+                ph -= img * a.PH;
+                unit += img * s.img_gap;
+            }
+            return unsigned(column) < unsigned(a.W) && unsigned(s.ih0 + ph) < unsigned(a.H);
+        });
     }
-    auto from_table = [&](int p) { return ptab[min(p, a.Ppad - 1)]; };
 #pragma unroll
     for (int r = 0; r < 8; ++r)
         if (r * 256 + tid < a.packed_units) wdst[r * 256 + tid] = w0[r];
@@ -158,12 +186,11 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     }
     __syncthreads();
 
-    const QBlockActHead *head = reinterpret_cast<const QBlockActHead *>(lds + a.o_act);
-    const RequantLut lut1 = qb_lut(lds + a.o_act, 0, __builtin_amdgcn_readfirstlane(head->lo1), __builtin_amdgcn_readfirstlane(head->hi1), a.zp1);
-    const RequantLut lut2 = qb_lut(lds + a.o_act, 1, __builtin_amdgcn_readfirstlane(head->lo2), __builtin_amdgcn_readfirstlane(head->hi2), a.zp2);
+    const unsigned head = qb_act_head(lds + a.o_act);
+    const RequantLut lut1 = qb_lut(lds + a.o_act, head, 0, a.zp1), lut2 = qb_lut(lds + a.o_act, head, 1, a.zp2);
     for (int tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
         const int ig = tile / a.n_row_tiles, rt = tile - ig * a.n_row_tiles;
-        const int n0 = ig * a.NB, oh0 = rt * a.TH, ih0 = oh0 * a.stride - 1;
+        const int n0 = ig * a.NB, oh0 = rt * a.TH, row0 = a.n_row_tiles > 1 ? oh0 * a.stride - 1 : 0;
         const int next_tile = tile + int(gridDim.x);
         const bool has_next = next_tile < a.n_tiles;
         i32x4 nxt[QB_PF];
@@ -175,7 +202,7 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
             for (int r = 0; r < QB_PF; ++r)
                 if (r < a_rounds) {
                     const int p = pr * 256 + tid;
-                    nxt_ok |= fetch(s, cb, p, from_table(p), nxt[r]) ? 1u << r : 0u;
+                    nxt_ok |= fetch(s, cb, p, from_table, nxt[r]) ? 1u << r : 0u;
                     if (++pr == p_rounds) { pr = 0; ++cb; }
                 }
         }
@@ -213,8 +240,8 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
                     bool padp[NU];
 #pragma unroll
                     for (int j = 0; j < NU; ++j) {
-                        const int e = ptab[(ptile + j) * 32 + l32].x;
-                        padp[j] = e < 0 || unsigned(ih0 + (e & 0xffff)) >= unsigned(a.H);
+                        const int e = ptab[(ptile + j) * 32 + l32];
+                        padp[j] = (e & QB_POS_PAD) || unsigned(row0 + (e & (QB_POS_PAD - 1))) >= unsigned(rows_in);
                     }
                     i32x4 xb[NU];
 #pragma unroll
@@ -284,23 +311,26 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         const int q_end = SPLIT ? nq_tiles : min(nq_tiles, (wave + 1) * q_per_wave);
         const int n_units = nq_tiles * a.Ce32, u_begin = (n_units * wave) >> 2, u_end = (n_units * (wave + 1)) >> 2;
         for (int q0 = SPLIT ? 0 : wave * q_per_wave; q0 < q_end; q0 += MQ) {
-            // an output position's top-left tap and its place in y, from the table.  Tiles of rows of one image end at the image's last
+            // an output position's top-left tap, from the table, and its place in y.  Tiles of rows of one image end at the image's last
             // row, tiles of images at the last image.
             constexpr int SJ = SPLIT ? 1 : MQ;  // position tiles this wave stores: its own of those all waves share
             int p0[MQ];
             unsigned ybase[SJ];  // byte offset of this lane's four channels in block 0 of its position (the host checks that the
             bool ok[SJ];         // blocked tensors stay below 2^31 bytes); a block of 16 channels further on is one plane further
-            auto place = [&](int tile_) { return qtab[min(tile_, nq_tiles - 1) * 32 + l32]; };
 #pragma unroll
-            for (int j = 0; j < MQ; ++j) p0[j] = place(q0 + j).x;
+            for (int j = 0; j < MQ; ++j) p0[j] = int(qtab[min(q0 + j, nq_tiles - 1) * 32 + l32]) * 16;
             auto set_out = [&] {
                 const int q_valid = a.n_row_tiles > 1 ? min(a.TH, a.OH - oh0) * a.OW : min(a.NB, a.N - n0) * a.TH * a.OW;
+                const float inv_tile_img = fresh_rcp(a.TH * a.OW);
                 const unsigned y_tile = ((unsigned(n0) * unsigned(a.CBo) * unsigned(a.OH) + unsigned(oh0)) * unsigned(a.OW)) * 16u;
 #pragma unroll
                 for (int j = 0; j < SJ; ++j) {
                     const int qt = SPLIT ? wave : q0 + j;
-                    ok[j] = qt < q_end && qt * 32 + l32 < q_valid;
-                    ybase[j] = y_tile + unsigned(place(qt).y) + unsigned(lh) * 4u;
+                    int q = qt * 32 + l32;
+                    if (SPLIT) asm("" : "+v"(q));  // (the same for every tile: not to be kept in registers across them)
+                    ok[j] = qt < q_end && q < q_valid;
+                    const int unit = q + quick_div(q, inv_tile_img) * ((a.CBo * a.OH - a.TH) * a.OW);
+                    ybase[j] = y_tile + unsigned(unit) * 16u + unsigned(lh) * 4u;
                 }
             };
             // The residual's bytes of every (tile, group), as one batch of loads; where registers allow, ahead of the chunks.
@@ -538,14 +568,13 @@ __global__ void __launch_bounds__(256) qblock_tables_kernel(QBlockArgs a, char *
     }
     __syncthreads();
     if (tid == 0) {
-        QBlockActHead h = {0, 0, 0, 0, {0, 0, 0, 0}};  // (a constant table: its first entry)
-        if (win[0] < win[1]) { h.lo1 = win[0]; h.hi1 = win[1]; }
-        if (win[2] < win[3]) { h.lo2 = win[2]; h.hi2 = win[3]; }
+        QBlockActHead h = {0, 0, 0, 0};  // (a constant table: its first entry)
+        if (win[0] < win[1]) { h.lo1 = uint8_t(win[0]); h.hi1 = uint8_t(win[1]); }
+        if (win[2] < win[3]) { h.lo2 = uint8_t(win[2]); h.hi2 = uint8_t(win[3]); }
         *reinterpret_cast<QBlockActHead *>(act) = h;
     }
-    const float inv_patch_hw = 1.0f / float(a.PH * a.PW), inv_pw = 1.0f / float(a.PW);
-    for (int p = tid; p < a.Ppad; p += 256) ptab[p] = qb_patch_pos(a, p, inv_patch_hw, inv_pw);
-    for (int q = tid; q < ((a.Q + 31) & ~31); q += 256) qtab[q] = qb_out_pos(a, q);
+    for (int p = tid; p < a.Ppad; p += 256) ptab[p] = QBlockPos(qb_patch_pos(a, p));
+    for (int q = tid; q < ((a.Q + 31) & ~31); q += 256) qtab[q] = QBlockPos(qb_out_pos(a, q));
 }
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -649,7 +678,7 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         t.Q = bNB * bTH * int(OW);
         t.n_row_tiles = int((OH + bTH - 1) / bTH);
         const int64_t n_tiles = ((N + bNB - 1) / bNB) * t.n_row_tiles;
-        if (n_tiles > INT32_MAX || t.P >= (1 << 20) || t.Q >= (1 << 20)) continue;
+        if (n_tiles > INT32_MAX || t.P > QB_POS_PAD) continue;
         t.n_tiles = int(n_tiles);
         size_t o = 0;
         t.o_xl = int(o); o += size_t(t.CBin) * t.Ppad * 16;
@@ -687,6 +716,12 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
         out->lds_bytes = cap_used;
     }
     a.packed_units = (a.o_qtab - a.o_w1 + ((a.Q + 31) & ~31) * int(sizeof(QBlockPos))) / 16;
+    // Wide blocks whose weights leave LDS room for half a matrix tile of output positions or less: the three layers by themselves are faster
+    // once the tiles are more than the CUs, a workgroup each (96 -> 576 -> 96 on 7x7: 32 images 42 us against 49, 64 64 / 53, 256 164 / 67,
+    // 1024 577 / 102; 128 -> 384 -> 128 67 / 64 at 256, 106 / 70 at 512).  Not those a chain of images may hold.
+    if (force_nb <= 0 && cap_used > 76 * 1024 && a.Q <= 16 && a.n_tiles > ctx->num_cus &&
+        zant_qblock_image_bytes(a.Cin32, a.Ce32, CO32, p_img, OH * OW, a.o_act - a.o_w1) > 160 * 1024)
+        return 1;
     if (plan_only) {
         out->a = a;
         out->packed = nullptr;
@@ -749,7 +784,6 @@ int zant_qblock_prepare(zant_ctx *ctx, const int64_t xdim[4], const zant_qconv_d
                            reinterpret_cast<QBlockPos *>(base + o_ptabp), reinterpret_cast<QBlockPos *>(base + o_qtabp));
         ZANT_LAUNCH_CHECK(ctx);
     }
-
 
     out->a = a;
     out->packed = reinterpret_cast<const uint4 *>(base + o_w1p);

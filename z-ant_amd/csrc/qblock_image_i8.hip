@@ -84,9 +84,8 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
     const int *c3 = reinterpret_cast<const int *>(m3 + co32 * 32);
     const QBlockPos *ptab = reinterpret_cast<const QBlockPos *>(lds + a.o_ptab), *qtab = reinterpret_cast<const QBlockPos *>(lds + a.o_qtab);
     int *R = reinterpret_cast<int *>(lds + l.o_r);
-    const QBlockActHead *head = reinterpret_cast<const QBlockActHead *>(lds + a.o_act);
-    const RequantLut lut1 = qb_lut(lds + a.o_act, 0, __builtin_amdgcn_readfirstlane(head->lo1), __builtin_amdgcn_readfirstlane(head->hi1), a.zp1);
-    const RequantLut lut2 = qb_lut(lds + a.o_act, 1, __builtin_amdgcn_readfirstlane(head->lo2), __builtin_amdgcn_readfirstlane(head->hi2), a.zp2);
+    const unsigned head = qb_act_head(lds + a.o_act);
+    const RequantLut lut1 = qb_lut(lds + a.o_act, head, 0, a.zp1), lut2 = qb_lut(lds + a.o_act, head, 1, a.zp2);
     const unsigned xl_a = lds_address(lds + a.o_xl), e_a = lds_address(lds + a.o_e);  // expanded patch: [Ce32*2][Ppad] units
     const int n_ptiles = a.Ppad >> 5, nq_tiles = (a.Q + 31) >> 5;
 
@@ -107,7 +106,7 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
         i32x4 xb;
         qb_read128(xb, xl_a + unsigned(lh * a.Ppad + ptile * 32 + l32) * 16u, 0);
         const i32x4 wa0 = as_i32x4(W1[kb * 64 + lh * 32 + l32]);
-        const int e = ptab[ptile * 32 + l32].x;
+        const bool padp = ptab[ptile * 32 + l32] & QB_POS_PAD;  // the depthwise convolution's padding: its zero point instead of an expansion
         i32x16 acc[1];
         float mv[16];
 #pragma unroll
@@ -115,8 +114,6 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
             acc[0][v] = c1[kch + (v >> 2) * 8 + (v & 3)];
             mv[v] = m1[kch + (v >> 2) * 8 + (v & 3)];
         }
-        // the depthwise convolution's padding: its zero point instead of an expansion
-        const bool padp = e < 0 || unsigned((e & 0xffff) - 1) >= unsigned(a.H);
         qb_ready(xb, 0);
         acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wa0, xb, acc[0], 0, 0, 0);
         for (int chunk = 1; chunk < a.Cin32; ++chunk)
@@ -156,7 +153,7 @@ __device__ __forceinline__ void image_block(const ImageLink &l, const ImageLink 
         for (int u = wave; u < d_units; u += kWaves) {
             const int j = small_div(u, a.Ce32, inv_ce), ch = u - j * a.Ce32, kch = ch * 32 + lh * 4;
             const bool half = a.half_last && ch == a.Ce32 - 1;
-            const unsigned r0 = e_a + unsigned((2 * ch + lh) * a.Ppad) * 16u + unsigned(qtab[j * 32 + l32].x),  // top-left tap
+            const unsigned r0 = e_a + unsigned((2 * ch + lh) * a.Ppad) * 16u + unsigned(qtab[j * 32 + l32]) * 16u,  // top-left tap
                            r1 = r0 + row_b, r2 = r1 + row_b;
             const uint32_t *wk = WDW + ((ch * 32 + l32) >> 2) * 36 + (l32 & 3);
             uint32_t wd[9];
@@ -310,7 +307,7 @@ size_t plan_lds(ImageChain &c) {
         const QBlockArgs &a = l.a;
         Need n;
         n.xl = align256(size_t(a.Cin32) * 2 * a.Ppad * 16);
-        n.w = align256(size_t(a.packed_units) * 16);
+        n.w = size_t(a.packed_units) * 16;
         n.e = align256(size_t(a.Ce32) * 2 * a.Ppad * 16);
         n.r = size_t((a.Q + 31) / 32) * l.co32 * 4096;
         return n;
