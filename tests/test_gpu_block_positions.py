@@ -33,3 +33,23 @@ def test_blocks_match_the_oracle(hw, c0, blocks, batch):
     assert m.num_launches == 3
     np.testing.assert_array_equal(m.predict_host(x)[sample], int8_ref.forward(arch, params, quant, x[sample]))
     m.close()
+
+
+@pytest.mark.parametrize("hw,c0,blocks,batch,kernel", [
+    ((4, 4), 40, [(240, 64, 2, "relu6", "relu6", 1)], 256, "qblock_kernel<2,1,true,true>"),   # eight chunks on one position tile: shared
+    ((6, 6), 24, [(72, 32, 1, "relu6", "relu6", 1)], 1, "qblock_kernel<1,1,true,true>"),      # three
+    ((3, 3), 24, [(72, 40, 2, "relu6", "relu6", 1)], 32, "qblock_kernel<2,1,true,false>"),    # three, two blocks of output channels: not shared
+])
+def test_few_positions_are_shared_by_chunks(hw, c0, blocks, batch, kernel):
+    import gpu_util as G
+    from zant_amd import networks as nets
+    arch = _arch(hw, c0, blocks)
+    params = nets.int8_params(arch, seed=9)
+    rng = np.random.default_rng(batch)
+    quant = int8_ref.calibrate(arch, params, rng.integers(0, 256, (2,) + arch["input"], dtype=np.uint8))
+    x = rng.integers(0, 256, (batch,) + arch["input"], dtype=np.uint8)
+    m = nets.build_int8_model(G.tm.context(), arch, params, quant, batch)
+    m.profile()
+    assert m.launch_kernels()[1] == kernel, m.launch_kernels()
+    np.testing.assert_array_equal(m.predict_host(x), int8_ref.forward(arch, params, quant, x))
+    m.close()
