@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "qblock_i8.h"
+#include "patch_deal.h"
 
 namespace {
 
@@ -34,10 +35,6 @@ __device__ __forceinline__ i32x4 as_i32x4(const uint4 &v) {
     r[0] = int(v.x); r[1] = int(v.y); r[2] = int(v.z); r[3] = int(v.w);
     return r;
 }
-
-// p / d for 0 <= p < 2^15 with inv = 1.0f / d to within a few units in the last place: (p + 1/2) / d is at least 1 / 2d away from a whole
-// number, further than reciprocal and fma err.
-__device__ __forceinline__ int quick_div(int p, float inv) { return int(__builtin_fmaf(float(p), inv, 0.5f * inv)); }
 
 // 1 / d, taken anew where it is used: two instructions, but registers are scarce from one tile to the next
 __device__ __forceinline__ float fresh_rcp(int d) {
@@ -57,7 +54,7 @@ __device__ __forceinline__ int qb_out_pos(const QBlockArgs &a, int q) {
 }
 
 // One block for the tiles of this workgroup; `lds` is the workgroup's dynamic LDS.
-template <int CO32, int MQ, bool PF, bool SPLIT>
+template <int CO32, int MQ, bool PF, bool SPLIT, bool FLAT = false>
 __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t *__restrict__ y, const uint4 *__restrict__ packed,
                                             const QBlockArgs &a, char *lds) {
     // A chunk of 32 channels is two blocks of 16; where the last chunk has one block only, the lanes of its second half read the first
@@ -98,18 +95,18 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     // first tile's patch is copied before the loop; every later one is loaded into registers before stage B of the tile
     // in front of it and written to LDS after that stage (the input patch is dead once B is done), so its global
     // latency passes under B.  Patches of more than QB_PF units per thread are copied in place instead. ----
-    // A round is 256 positions of one channel block.  A position's row, which with the position itself gives its place in x, is divided out
+    // A position's row, which with the position itself gives its place in x, is divided out
     // for the first tile, while the tables are on their way; every later tile's comes from the table (60 vector instructions a unit, six of
     // them quarter rate, when positions were taken apart for each).
-    constexpr int QB_PF = 4;
+    constexpr int QB_PF = PATCH_ROUNDS_AHEAD;
     const int patch_hw = a.PH * a.PW;
-    const int p_rounds = (a.Ppad + 255) >> 8, a_rounds = a.CBin * p_rounds;
-    const bool prefetch = PF && a_rounds <= QB_PF;  // PF is off for the instantiations without registers to spare
+    const int per_block = (a.P + 255) >> 8, rounds = patch_rounds(a.CBin, a.P, FLAT);
+    const bool prefetch = PF && rounds <= QB_PF;  // PF is off for the instantiations without registers to spare
     const int64_t in_plane = int64_t(a.H) * a.W * 16;
     // a row of the patch is in the map (tiles of whole images: as the table says)
     const int rows_in = a.n_row_tiles > 1 ? a.H : QB_POS_PAD;
     // valid: an offset that lies inside the tensor; img_gap: units from an image's rows to the next one's beyond those of the patch
-    struct Source { const char *base; int ih0, row0, positions, img_gap; unsigned valid; float inv_ph; };
+    struct Source { const char *base; int ih0, row0, positions, img_gap; unsigned valid; float inv_ph, inv_p; };
     auto source_of = [&](int tile_) {
         const int ig_ = tile_ / a.n_row_tiles, rt_ = tile_ - ig_ * a.n_row_tiles, n_ = ig_ * a.NB;
         Source s;
@@ -117,18 +114,35 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         s.row0 = a.n_row_tiles > 1 ? s.ih0 : 0;
         s.img_gap = (a.CBin * a.H - a.PH) * a.W;
         s.inv_ph = fresh_rcp(a.PH);
+        s.inv_p = fresh_rcp(a.P);
         s.positions = a.n_row_tiles > 1 ? a.P : min(a.NB, a.N - n_) * patch_hw;
         s.base = reinterpret_cast<const char *>(x) + (int64_t(n_) * a.CBin * a.H + s.ih0) * int64_t(a.W) * 16;
         s.valid = s.ih0 < 0 ? unsigned(a.W) * 16u : 0u;
         return s;
     };
+    // the rounds in order: of one channel block after the other, or all in a row
+    struct Turn { int cb, pr; };
+    auto next_turn = [&](Turn &t) {
+        if (++t.pr == per_block && !FLAT) { t.pr = 0; ++t.cb; }
+    };
     // every lane loads (from a place inside the tensor when it has nothing to fetch): no divergent branch around the load, so nothing
     // waits for it before the values are written to LDS
-    auto fetch = [&](const Source &s, int cb, int p, auto place, i32x4 &v) {
-        int unit;
-        const bool ok = place(s, p, unit) && p < s.positions;
-        v = *reinterpret_cast<const i32x4 *>(s.base + cb * in_plane + (ok ? unsigned(unit) * 16u : s.valid));
+    auto fetch = [&](const Source &s, const Turn &t, auto place, i32x4 &v) {
+        int p = t.pr * 256 + tid, unit, own = 0;
+        if (FLAT) p = patch_unit_flat(t.pr, tid, a.P, s.inv_p, &own);
+        bool ok = place(s, p, unit) && p < s.positions;
+        unsigned at = unsigned(unit) * 16u;
+        if (FLAT) {
+            ok = ok && own < a.CBin;
+            at += unsigned(own) * unsigned(in_plane);  // (tensors stay below 2^31 bytes)
+        }
+        v = *reinterpret_cast<const i32x4 *>(s.base + t.cb * in_plane + (ok ? at : s.valid));
         return ok;
+    };
+    auto put = [&](const Turn &t, float inv_p, const i32x4 &v) {
+        int p = t.pr * 256 + tid, own = t.cb;
+        if (FLAT) p = patch_unit_flat(t.pr, tid, a.P, inv_p, &own);
+        *reinterpret_cast<i32x4 *>(XL + own * a.Ppad + p) = v;
     };
     // whether patch position p lies in the map, and its unit from the patch's first row, column 0, on
     auto from_table = [&](const Source &s, int p, int &unit) {
@@ -139,24 +153,23 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
     };
     auto copy_patch = [&](int tile_, auto place) {  // four loads in flight per thread, then their four LDS writes
         const Source s = source_of(tile_);
-        int cb = 0, pr = 0;
-        for (int r0 = 0; r0 < a_rounds; r0 += 4) {
+        Turn from = {0, 0}, to = {0, 0};
+        for (int r0 = 0; r0 < rounds; r0 += 4) {
             i32x4 v[4];  // (a native vector type: arrays of it are kept in registers)
-            int dst[4];
             bool ok[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int p = pr * 256 + tid;
-                dst[r] = cb * a.Ppad + p;
                 ok[r] = false;
-                if (r0 + r < a_rounds) {
-                    ok[r] = fetch(s, cb, p, place, v[r]);
-                    if (++pr == p_rounds) { pr = 0; ++cb; }
+                if (r0 + r < rounds) {
+                    ok[r] = fetch(s, from, place, v[r]);
+                    next_turn(from);
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (ok[r]) *reinterpret_cast<i32x4 *>(XL + dst[r]) = v[r];
+            for (int r = 0; r < 4; ++r) {
+                if (ok[r]) put(to, s.inv_p, v[r]);
+                next_turn(to);
+            }
         }
     };
     if (int(blockIdx.x) < a.n_tiles) {
@@ -197,13 +210,12 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         unsigned nxt_ok = 0;
         if (PF && prefetch && has_next) {
             const Source s = source_of(next_tile);
-            int cb = 0, pr = 0;
+            Turn t = {0, 0};
 #pragma unroll
             for (int r = 0; r < QB_PF; ++r)
-                if (r < a_rounds) {
-                    const int p = pr * 256 + tid;
-                    nxt_ok |= fetch(s, cb, p, from_table, nxt[r]) ? 1u << r : 0u;
-                    if (++pr == p_rounds) { pr = 0; ++cb; }
+                if (r < rounds) {
+                    nxt_ok |= fetch(s, t, from_table, nxt[r]) ? 1u << r : 0u;
+                    next_turn(t);
                 }
         }
 
@@ -289,12 +301,13 @@ __device__ __forceinline__ void qblock_body(const uint4 *__restrict__ x, uint8_t
         // ---- the next tile's input patch goes to LDS (the current one is dead; stage D reads the expanded patch only) ----
         if (has_next) {
             if (PF && prefetch) {
-                int cb = 0, pr = 0;
+                const float inv_p = fresh_rcp(a.P);
+                Turn t = {0, 0};
 #pragma unroll
                 for (int r = 0; r < QB_PF; ++r)
-                    if (r < a_rounds) {
-                        if ((nxt_ok >> r) & 1u) *reinterpret_cast<i32x4 *>(XL + cb * a.Ppad + pr * 256 + tid) = nxt[r];
-                        if (++pr == p_rounds) { pr = 0; ++cb; }
+                    if (r < rounds) {
+                        if ((nxt_ok >> r) & 1u) put(t, inv_p, nxt[r]);
+                        next_turn(t);
                     }
             } else {
                 copy_patch(next_tile, from_table);
@@ -512,6 +525,13 @@ __global__ void __launch_bounds__(256, 2)  // 256 registers per lane for every i
 qblock_kernel(const uint4 *__restrict__ x, uint8_t *__restrict__ y, const uint4 *__restrict__ packed, QBlockArgs a) {
     extern __shared__ __attribute__((aligned(256))) char lds[];
     qblock_body<CO32, MQ, PF, SPLIT>(x, y, packed, a, lds);
+}
+// ... with patches of many channel blocks dealt in a row (patch_deal.h)
+template <int CO32, int MQ, bool PF, bool SPLIT>
+__global__ void __launch_bounds__(256, 2)
+qblock_flat_kernel(const uint4 *__restrict__ x, uint8_t *__restrict__ y, const uint4 *__restrict__ packed, QBlockArgs a) {
+    extern __shared__ __attribute__((aligned(256))) char lds[];
+    qblock_body<CO32, MQ, PF, SPLIT, true>(x, y, packed, a, lds);
 }
 
 // Several blocks in a row as ONE launch.  Every block of a chain works on tiles of the same NB whole images, one tile
@@ -811,27 +831,38 @@ int zant_qblock_blocked(zant_ctx *ctx, const uint8_t *x, const int64_t xdim[4], 
     const int per_cu = cap_used <= 76 * 1024 ? 2 : 1;
     const int grid = int(std::min<int64_t>(a.n_tiles, int64_t(ctx->num_cus) * per_cu));
     KernelTimer kt(ctx);
-#define ZANT_QBLOCK_LAUNCH(CO, M, P, S)                                                                                          \
-    do {                                                                                                                    \
-        if (!zant_raise_lds_limit(ctx, reinterpret_cast<const void *>(&qblock_kernel<CO, M, P, S>), 160 * 1024)) break;         \
-        ZANT_KERNEL_NAME(ctx, "qblock_kernel<%d,%d,%s,%s>", CO, M, P ? "true" : "false", S ? "true" : "false");                                          \
-        hipLaunchKernelGGL((qblock_kernel<CO, M, P, S>), dim3(grid), dim3(256), cap_used, ctx->stream,                           \
-                           reinterpret_cast<const uint4 *>(x), y, packed, a);       \
+#define ZANT_QBLOCK_LAUNCH(KERNEL, CO, M, P, S)                                                                                  \
+    do {                                                                                                                         \
+        if (!zant_raise_lds_limit(ctx, reinterpret_cast<const void *>(&KERNEL<CO, M, P, S>), 160 * 1024)) break;                 \
+        ZANT_KERNEL_NAME(ctx, #KERNEL "<%d,%d,%s,%s>", CO, M, P ? "true" : "false", S ? "true" : "false");                       \
+        hipLaunchKernelGGL((KERNEL<CO, M, P, S>), dim3(grid), dim3(256), cap_used, ctx->stream,                                  \
+                           reinterpret_cast<const uint4 *>(x), y, packed, a);                                                    \
     } while (0)
-    switch ((a.split ? 100 : 0) + CO32 * 10 + MQv) {
-    case 11: ZANT_QBLOCK_LAUNCH(1, 1, true, false); break;
-    case 12: ZANT_QBLOCK_LAUNCH(1, 2, true, false); break;
-    case 13: ZANT_QBLOCK_LAUNCH(1, 3, true, false); break;
-    case 14: ZANT_QBLOCK_LAUNCH(1, 4, false, false); break;
-    case 21: ZANT_QBLOCK_LAUNCH(2, 1, true, false); break;
-    case 22: ZANT_QBLOCK_LAUNCH(2, 2, false, false); break;
-    case 31: ZANT_QBLOCK_LAUNCH(3, 1, true, false); break;
-    case 111: ZANT_QBLOCK_LAUNCH(1, 1, true, true); break;
-    case 112: ZANT_QBLOCK_LAUNCH(1, 2, true, true); break;
-    case 113: ZANT_QBLOCK_LAUNCH(1, 3, false, true); break;
-    case 121: ZANT_QBLOCK_LAUNCH(2, 1, true, true); break;
-    case 122: ZANT_QBLOCK_LAUNCH(2, 2, false, true); break;
-    default: ZANT_QBLOCK_LAUNCH(4, 1, true, false); break;
+    const int key = (a.split ? 100 : 0) + CO32 * 10 + MQv;
+    if (patch_flat(a.CBin, a.P) && (key == 21 || key == 31 || key == 41 || key == 121)) {
+        switch (key) {
+        case 21: ZANT_QBLOCK_LAUNCH(qblock_flat_kernel, 2, 1, true, false); break;
+        case 31: ZANT_QBLOCK_LAUNCH(qblock_flat_kernel, 3, 1, true, false); break;
+        case 121: ZANT_QBLOCK_LAUNCH(qblock_flat_kernel, 2, 1, true, true); break;
+        default: ZANT_QBLOCK_LAUNCH(qblock_flat_kernel, 4, 1, true, false); break;
+        }
+        ZANT_LAUNCH_CHECK(ctx);
+        return ZANT_OK;
+    }
+    switch (key) {
+    case 11: ZANT_QBLOCK_LAUNCH(qblock_kernel, 1, 1, true, false); break;
+    case 12: ZANT_QBLOCK_LAUNCH(qblock_kernel, 1, 2, true, false); break;
+    case 13: ZANT_QBLOCK_LAUNCH(qblock_kernel, 1, 3, true, false); break;
+    case 14: ZANT_QBLOCK_LAUNCH(qblock_kernel, 1, 4, false, false); break;
+    case 21: ZANT_QBLOCK_LAUNCH(qblock_kernel, 2, 1, true, false); break;
+    case 22: ZANT_QBLOCK_LAUNCH(qblock_kernel, 2, 2, false, false); break;
+    case 31: ZANT_QBLOCK_LAUNCH(qblock_kernel, 3, 1, true, false); break;
+    case 111: ZANT_QBLOCK_LAUNCH(qblock_kernel, 1, 1, true, true); break;
+    case 112: ZANT_QBLOCK_LAUNCH(qblock_kernel, 1, 2, true, true); break;
+    case 113: ZANT_QBLOCK_LAUNCH(qblock_kernel, 1, 3, false, true); break;
+    case 121: ZANT_QBLOCK_LAUNCH(qblock_kernel, 2, 1, true, true); break;
+    case 122: ZANT_QBLOCK_LAUNCH(qblock_kernel, 2, 2, false, true); break;
+    default: ZANT_QBLOCK_LAUNCH(qblock_kernel, 4, 1, true, false); break;
     }
 #undef ZANT_QBLOCK_LAUNCH
     ZANT_LAUNCH_CHECK(ctx);
