@@ -1617,8 +1617,10 @@ size_t qdw_table_bytes(int C) {
 // The matrix-core kernel deals 64 channels to a workgroup, which reads their weights on its own: 1280 -> 1000 of one image on 16 of 256
 // CUs (9.9 us of MobileNetV2's pass; here the pass of one image takes 121.4 -> 114.6 us, a call by itself 17.7 -> 12.2, 4096 -> 4096 94 -> 12
 // and, with 64 images, 2076 -> 47).  C is a multiple of 16: a blocked tensor is then its channels in a row, like an NCHW one (flip: 0x80 in every byte for that).
+// U > 2: at most four waves a SIMD, or the compiler keeps registers for eight of them by waiting for one load after the other (64 images, 4096 ->
+// 1000: 45.4 us so, 17.2 here).
 template <int U>
-__global__ void __launch_bounds__(256) qfc_kernel(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const float *__restrict__ w_scale,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, U > 2 ? 4 : 8))) qfc_kernel(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const float *__restrict__ w_scale,
                                                   const int32_t *__restrict__ bias, uint8_t *__restrict__ y, int N, int units, int K, int y_pitch,
                                                   QConvArgs q, uint32_t flip, int y_flip) {
     const int lane = threadIdx.x & 63, k = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
@@ -1645,18 +1647,21 @@ __global__ void __launch_bounds__(256) qfc_kernel(const uint4 *__restrict__ x, c
     int mine = 0;  // lane n: image n's sum
     constexpr int G = 4;
     for (int n0 = 0; n0 < N; n0 += G) {
+        uint4 v[G][U];
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[i][u] = x[int64_t(min(n0 + i, N - 1)) * units + min(u * 64 + lane, units - 1)];  // (past the row: against zero weights)
         int acc[G];
 #pragma unroll
         for (int i = 0; i < G; ++i) {
-            const uint4 *xn = x + int64_t(min(n0 + i, N - 1)) * units;
             acc[i] = own;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const uint4 v = xn[min(u * 64 + lane, units - 1)];  // (past the row: against zero weights)
-                acc[i] = __builtin_amdgcn_sdot4(int(v.x ^ flip), int(wv[u].x), acc[i], false);
-                acc[i] = __builtin_amdgcn_sdot4(int(v.y ^ flip), int(wv[u].y), acc[i], false);
-                acc[i] = __builtin_amdgcn_sdot4(int(v.z ^ flip), int(wv[u].z), acc[i], false);
-                acc[i] = __builtin_amdgcn_sdot4(int(v.w ^ flip), int(wv[u].w), acc[i], false);
+                acc[i] = __builtin_amdgcn_sdot4(int(v[i][u].x ^ flip), int(wv[u].x), acc[i], false);
+                acc[i] = __builtin_amdgcn_sdot4(int(v[i][u].y ^ flip), int(wv[u].y), acc[i], false);
+                acc[i] = __builtin_amdgcn_sdot4(int(v[i][u].z ^ flip), int(wv[u].z), acc[i], false);
+                acc[i] = __builtin_amdgcn_sdot4(int(v[i][u].w ^ flip), int(wv[u].w), acc[i], false);
             }
         }
 #pragma unroll
