@@ -147,7 +147,9 @@ def test_global_avgpool_vector_path_and_its_neighbours(G, shape):
 # ---- dense int8 layers of a few output positions: less than one tile of the matrix-core kernel ---------------------
 FEW = [
     # N, C, H, W, K, k, stride, pad
-    (1, 1280, 1, 1, 1000, 1, 1, 0),  # a classifier head on one image: a single position, read as a 1 x 8 filter
+    (1, 1280, 1, 1, 1000, 1, 1, 0),  # a classifier head on one image: a wave an output channel
+    (1, 1272, 1, 1, 1000, 1, 1, 0),  # ... of channels that are no whole 16
+    (1, 4224, 1, 1, 300, 1, 1, 0),   # ... of more channels than that takes: a single position, read as a 1 x 8 filter
     (1, 112, 3, 3, 200, 1, 1, 0),    # nine positions
     (3, 40, 1, 1, 33, 1, 1, 0),      # three positions, channels that are no whole 32
     (1, 24, 5, 4, 20, 3, 2, 1),      # six positions, 3x3 stride 2
@@ -167,7 +169,8 @@ def test_dense_int8_layers_of_few_positions(G, case, act):
     kw = dict(act=act, act_alpha=0.0, act_scale=0.04, act_zp=30) if act else {}
     ref = zo.qlinearconv(x, 0.02, 117, w, ws, None, 0.05, 120, b, [s, s], [p] * 4, [1, 1], 1, **kw)
     y = G.tm.qlinearconv(G.dev(x), 0.02, 117, G.dev(w), G.dev(ws), None, 0.05, 120, G.dev(b), [s, s], [p] * 4, [1, 1], 1, **kw)
-    assert G.tm.context().kernel_name().startswith("qconv_mfma_kernel<"), G.tm.context().kernel_name()
+    head = H == W == 1 and C % 16 == 0 and C <= 4096
+    assert G.tm.context().kernel_name().startswith("qfc_kernel<" if head else "qconv_mfma_kernel<"), G.tm.context().kernel_name()
     np.testing.assert_array_equal(G.host(y), ref)
 
 

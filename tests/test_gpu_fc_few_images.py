@@ -1,5 +1,6 @@
-"""Fully connected int8 layers of few images (a wave an output channel): numbers of images around the groups of four and the limit of 64,
-channels around a wave's 1024, output channels that leave waves or a blocked tensor's last block empty, both layouts, activations.
+"""Fully connected int8 layers of few images (a wave an output channel) and where other kernels are faster: numbers of images around the
+groups of four and the limit of 64, channels around a wave's 1024, output channels that leave waves or a blocked tensor's last block empty,
+both layouts, activations.
 Bit for bit against the oracle; what the kernel does not take gives the same."""
 import numpy as np
 import pytest
@@ -23,12 +24,14 @@ def _layer(N, C, K, seed):
 
 @pytest.mark.parametrize("act", ["none", "leaky", "relu6"])
 @pytest.mark.parametrize("N,C,K", [(1, 16, 1), (1, 1280, 1000), (1, 2048, 1024), (3, 48, 5), (4, 1008, 4), (5, 1024, 3), (7, 1040, 33), (33, 2064, 17), (63, 4096, 9),
-                                   (64, 3072, 30), (65, 1280, 12), (2, 4112, 7), (9, 40, 21)])
+                                   (64, 3072, 30), (65, 1280, 12), (2, 4112, 7), (9, 40, 21),
+                                   # many filters: on the matrix cores, past what these have room for here again, of few terms the direct kernel
+                                   (64, 64, 4096), (40, 256, 4096), (40, 16, 8192)])
 def test_layers_match_the_oracle(G, N, C, K, act):
     x, w, ws, b = _layer(N, C, K, N + C + K)
     y = G.dev(np.full((N, K, 1, 1), 77, np.uint8))
     G.tm.qlinearconv_lean(G.dev(x), 0.02, 117, G.dev(w), G.dev(ws), None, 0.05, 128, G.dev(b), y, [1, 1], [0] * 4, [1, 1], 1, act, 0.1, 0.04, 30)
-    here = N <= 64 and C % 16 == 0 and C <= 4096 and (N > 1 or C * K >= 1 << 21)
+    here = N <= 64 and C % 16 == 0 and C <= 4096 and (N, C, K) not in ((64, 64, 4096), (40, 16, 8192))
     assert G.tm.context().kernel_name().startswith("qfc_kernel<") == here, G.tm.context().kernel_name()
     want = zo.qlinearconv(x, 0.02, 117, w, ws, None, 0.05, 128, b, [1, 1], [0] * 4, [1, 1], 1)
     if act != "none":
@@ -69,6 +72,7 @@ def test_chained_in_a_model(G, N):
         v, s, z = zo.qlinearconv(v, s, z, w, ws, None, 0.05, 120, b, [1, 1], [0] * 4, [1, 1], 1), 0.05, 120
     m.finalize()
     m.profile()
-    assert sum(k.startswith("qfc_kernel<") for k in m.launch_kernels()) == 2, m.launch_kernels()  # (48 channels in, and 96)
+    # 48 channels in, and 96; of 64 images, with the weights kept, the matrix-core kernel is the faster one
+    assert sum(k.startswith("qfc_kernel<") for k in m.launch_kernels()) == (2 if N < 64 else 0), m.launch_kernels()
     np.testing.assert_array_equal(m.predict_host(x), v)
     m.close()

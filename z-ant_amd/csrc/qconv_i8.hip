@@ -1616,7 +1616,7 @@ size_t qdw_table_bytes(int C) {
 // channel of all images: its row of weights, as it is stored, stays in registers (no packing), a lane holding 16 channels of every 1024.
 // The matrix-core kernel deals 64 channels to a workgroup, which reads their weights on its own: 1280 -> 1000 of one image on 16 of 256
 // CUs (9.9 us of MobileNetV2's pass; here the pass of one image takes 121.4 -> 114.6 us, a call by itself 17.7 -> 12.2, 4096 -> 4096 94 -> 12
-// and, with 64 images, 2076 -> 47).  C is a multiple of 16: a blocked tensor is then its channels in a row, like an NCHW one (flip: 0x80 in every byte for that).
+// and, with 64 images, 2076 -> 47).  Which of the two takes a layer: qfc_preferred.  C is a multiple of 16: a blocked tensor is then its channels in a row, like an NCHW one (flip: 0x80 in every byte for that).
 // U > 2: at most four waves a SIMD, or the compiler keeps registers for eight of them by waiting for one load after the other (64 images, 4096 ->
 // 1000: 45.4 us so, 17.2 here).
 template <int U>
@@ -1678,9 +1678,18 @@ bool qfc_eligible(const ConvGeom &g, const void *x, const void *w) {
     return g.groups == 1 && g.H == 1 && g.W == 1 && g.KH == 1 && g.KW == 1 && g.OH == 1 && g.OW == 1 && g.pt == 0 && g.pl == 0 && g.C % 16 == 0 &&
            g.C <= 4096 && g.N <= QFC_MAX_N && g.K <= (1 << 24) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
 }
-// A call by itself on one image keeps the kernel that it is tested to take below 2 MB of weights (1280 -> 1000: 17.7 us there, 12.2 here);
-// model nodes, plans, several images and larger layers (4096 -> 4096: 94 us there) take this one.
-bool qfc_preferred(const ConvGeom &g, bool kept) { return kept || g.N > 1 || int64_t(g.C) * g.K >= (int64_t(1) << 21); }
+// Whether this kernel is faster than the one that would take the layer else; by the kernels' times, in microseconds, at 1 to 64 images, 16 to
+// 4096 channels, 10 to 8192 filters.  Here a wave takes its images four at a time, one group after the other, and past some 2000 filters
+// the waves fill the chip; in the matrix-core kernel a workgroup's steps of 32 channels count, whatever the images, and a call by itself packs the
+// weights first; the direct kernel, for sums of less than 40 terms, has as much to do as there are products, and converts blocked tensors.
+// Kept weights, 64 images, 64 -> 1000 12.6 here and 6.9 there, 2048 -> 1000 14.2 and 16.8, 16 images, 64 -> 4096 9.3 and 7.4, 48 images, 16 ->
+// 1000 10.3 and 9.2; one image by itself always here (1280 -> 1000 22 us and a wait, 35 there).
+bool qfc_preferred(const ConvGeom &g, bool kept, bool blocked) {
+    const double groups = (g.N + 3) / 4, U = (g.C / 16 + 63) / 64;
+    const double here = std::max(6.0, 4.6 + groups * std::max(0.36 + 0.07 * U, g.K * (0.21e-3 + 0.085e-3 * U)));
+    if (g.C < 40 && g.N < 64) return here <= 4.0 + 0.28 * g.C + 1.3e-5 * g.N * double(g.K) + (blocked ? 8.0 : 0.0);
+    return here <= 5.8 + 0.0046 * g.C + 0.0003 * std::min(g.K, 2000) + (kept ? 0.0 : 6.5 + 3.3e-6 * double(g.C) * g.K);
+}
 int run_qfc(zant_ctx *ctx, const uint8_t *x, const int8_t *w, const float *w_scale, const int32_t *bias, uint8_t *y, const ConvGeom &g,
             const QConvArgs &q, bool xb, bool yb) {
     const int pitch = yb ? (g.K + 15) / 16 * 16 : g.K, units = g.C / 16;
@@ -1876,11 +1885,13 @@ int zant_qlinearconv_layout_pool(zant_ctx *ctx, const uint8_t *x, const int64_t 
         if (rc) return rc;
         return yb ? ZANT_OK : zant_from_blocked(ctx, yout, g.N, g.K, int64_t(g.OH) * g.OW, y);
     }
-    if (w_zp == nullptr && qfc_eligible(g, x, w) && qfc_preferred(g, slot != nullptr)) return run_qfc(ctx, x, w, w_scale, bias, y, g, q, xb, yb);
+    const bool qfc = w_zp == nullptr && qfc_eligible(g, x, w);
+    if (qfc && qfc_preferred(g, slot != nullptr, xb || yb)) return run_qfc(ctx, x, w, w_scale, bias, y, g, q, xb, yb);
     if (w_zp == nullptr) {  // a non-zero weight zero point makes the correction position dependent: direct kernel
         const int rc = run_qconv_mfma(ctx, x, w, w_scale, bias, y, g, q, xb, yb, slot);
         if (rc <= 0) return rc;
     }
+    if (qfc && g.C > 16) return run_qfc(ctx, x, w, w_scale, bias, y, g, q, xb, yb);  // (no tiling: many filters, whose tables fill LDS)
     // direct kernel: NCHW only; blocked operands pass through conversions in the workspace
     const uint8_t *xin = x;
     uint8_t *yout = y;
