@@ -130,8 +130,9 @@ static inline unsigned zant_stream_grid(int64_t vectors) {
 // 18 us instead of 25 at 64 MB, 33 (47) at 128, 48 (70) at 192, 68 (91) at 256, and a first pass 26 (26), 49 (48), 70 (70), 92 (92).  (Plain
 // stores leave it there too, but cost a first pass 2 % and an addition 4.)  Beyond 256 MB nothing of use is left there, and an addition is 1 %
 // slower; below 24 MB a first pass is, 7.7 us instead of 7.0 at 16 MB.  The data of a store wider than 64 bits must not be overwritten by the
-// next two instructions: the compiler, which does not see a store here, is kept from it by the s_nop (no time: eight f32 operators on 1001x32x26x26 227.1 us, 227.3 without).
-__device__ __forceinline__ bool zant_out_kept(int64_t bytes) { return bytes >= (int64_t(24) << 20) && bytes <= (int64_t(256) << 20); }
+// next two instructions: the compiler, which does not see a store here, is kept from it by the s_nop (no time: eight f32 operators on
+// 1001x32x26x26 227.1 us, 227.3 without).
+__host__ __device__ __forceinline__ bool zant_out_kept(int64_t bytes) { return bytes >= (int64_t(24) << 20) && bytes <= (int64_t(256) << 20); }
 template <typename V, typename P>
 __device__ __forceinline__ void zant_store_out(V v, P *p, bool kept) {
     static_assert(sizeof(V) == sizeof(P), "one object");
