@@ -1286,18 +1286,18 @@ extern "C" int zant_model_predict_host(zant_model *m, const void *input_host, vo
     if (!m || !input_host || !output_host) return ZANT_NullPointer;
     if (!m->finalized) return ZANT_NotFinalized;
     zant_ctx *ctx = m->ctx;
-    // Not waited for here: the caller has the buffer back after the last copy's wait, or after this one on a failure.  The nodes are enqueued
-    // while the input travels: README CNN on one image 67.5 -> 57.5 us.
+    // Not waited for here: the caller has the buffer back after the download's wait, or after one more where anything fails.  The nodes are
+    // enqueued while the input travels: README CNN on one image 67.5 -> 57.5 us.
     ZANT_HIP_TRY(ctx, hipMemcpyAsync(tensor_ptr(m, m->input), input_host, m->t[m->input].bytes(), hipMemcpyHostToDevice, ctx->stream));
+    int rc = ZANT_OK;
     for (const MNode &nd : m->n) {
         if (nd.skip) continue;
-        const int rc = run_node(m, nd);
-        if (rc) {
-            (void)hipStreamSynchronize(ctx->stream);
-            return rc;
-        }
+        rc = run_node(m, nd);
+        if (rc) break;
     }
-    return zant_hip_download(ctx, output_host, tensor_ptr(m, m->output), m->t[m->output].bytes());
+    if (!rc) rc = zant_hip_download(ctx, output_host, tensor_ptr(m, m->output), m->t[m->output].bytes());
+    if (rc) (void)hipStreamSynchronize(ctx->stream);
+    return rc;
 }
 
 namespace {
