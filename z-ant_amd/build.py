@@ -20,6 +20,8 @@ FLAGS = [
     # never let the compiler form packed-f32 VALU ops; rounding of a*b+c stays two-step everywhere
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-ffp-contract=off",
+    # requantisation by table address (quant_common.h) computes with f32 denormals: they must never be flushed
+    "-fno-gpu-flush-denormals-to-zero",
     "-Wall", "-Wno-unused-function",
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
 ]

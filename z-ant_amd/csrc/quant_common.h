@@ -143,6 +143,7 @@ __device__ __forceinline__ void qb_requant_lookup(const zq_i32x16 &acc, const fl
 // The bits of a float below 2^-125 are its value in units of 2^-149, so an fma whose result lies there rounds to a whole number of units,
 // half to even, and leaves that number as an integer in a register:
 //     fma(x, 2^-149, T * 2^-149)  =  the bits  rint(x) + T     for even T (a tie then goes the way rint(x) takes it).
+// (The build flags keep denormals; with them flushed every entry would be the first.)
 // With T = (LDS address of the table's entry 0) + zero point, these bits are the address of the entry; the table is laid at an
 // address of the zero point's parity.  The clamp to [0, 255] is a med3 on the floats (a negative sum is a negative float, a NaN
 // takes the lower bound), and costs nothing more when it is narrowed to the entries between which the table changes: of a ReLU6 these are
