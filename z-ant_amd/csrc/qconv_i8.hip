@@ -201,7 +201,6 @@ __global__ void __launch_bounds__(256) qpack_blocked_kernel(QPackJob p, BlockedJ
     else blocked_tile(j, blockIdx.x - pack_blocks);
 }
 
-// Bytes of the weight region of a staging buffer: the slab rounded up to one 16-byte unit per thread and round.
 // 3x3 layers of up to 16 channels: a matrix instruction takes 32 of the sum, two neighbouring taps of a filter row -- the halves of a wave read
 // positions one (dilated) column apart instead of two channel blocks -- and a row is two such pairs, the fourth tap's weights zero: six
 // instructions and operand reads instead of nine half empty ones.  What a fourth tap reads past a row or the patch is in the copy's unused
@@ -209,6 +208,7 @@ __global__ void __launch_bounds__(256) qpack_blocked_kernel(QPackJob p, BlockedJ
 // 49.6, with stride 2 33.4 -> 32.2, 256 maps of 64x64 8 -> 64 67 -> 63.4; tiny-YOLO's pass 125 -> 122.
 constexpr int TAPS_PAIRED = 6;
 __device__ __host__ __forceinline__ bool taps_paired(const ConvGeom &g) { return g.C <= 16 && g.KH == 3 && g.KW == 3; }
+// Bytes of the weight region of a staging buffer: the slab rounded up to one 16-byte unit per thread and round.
 __device__ __host__ __forceinline__ int w_region_bytes(int w_chunk, int nt) { return ((w_chunk / 16 + nt - 1) / nt) * nt * 16; }
 
 // Where this thread's patch slots of one tile come from: byte offset of the first 16-channel half of chunk 0 from the
